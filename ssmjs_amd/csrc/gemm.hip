@@ -1,4 +1,4 @@
-// Prefill projections on the fp32 matrix cores: Y = beta * Y + X W^T (+ bias), X (M, K) and
+// Projections on the fp32 matrix cores: Y = beta * Y + X W^T (+ bias), X (M, K) and
 // W (N, K) row-major (the Linear layers of the model behind model.forward, the in_proj /
 // x_proj / dt_proj / out_proj of the Mamba blocks), all arithmetic in fp32 with
 // v_mfma_f32_16x16x4_f32.
@@ -28,17 +28,6 @@
 // tiles are numbered in groups of 8 row tiles (a group walks its columns), so the tiles in
 // flight on an XCD share X rows and W rows through that XCD's L2.
 //
-// Split K. When the tiles alone leave CUs idle (prompts of a few hundred tokens), K may be
-// cut into S slices of a multiple of 16 (at least 128 each) and every (tile, slice) pair is
-// a workgroup of its own (slice z of row tile tm is row tile tm + z mt of an S times taller
-// grid, so the ordering above is unchanged); each writes its raw partial tile to a
-// workspace (S, M, N), and a second kernel adds the S partials in slice order
-// (deterministic) and applies the epilogue (row scale, bias, beta, gate) in the same order
-// as the unsplit kernel. The tile width and S are chosen together by a cost model measured
-// on MI355X: a CU running one of these workgroups does 0.44 TFLOP/s, two or more 0.50 (of
-// 0.61 peak), the partials cost their bytes written and read at 5 TB/s, and the finishing
-// launch about 4 us.
-//
 // Measured (MI355X, fp32 TFLOP/s, this kernel / hipBLASLt): M 32768 N 2048 K 4096 150 / 151,
 // M 32768 N 8448 K 2016 148 / 149, M 8192 N 3072 K 768 119 / 118. At a clock of 2.4 GHz the
 // fp32 MFMA peak is 157 TFLOP/s; with the operand loads running the clock drops to about
@@ -67,13 +56,6 @@ struct GemmArgs {
     int M, N, K;
     float beta;
     int mt, nt;
-    // row scale (RS): Y[m, :] = s[m] (X W^T)[m, :] + ..., s[m] = 1 / sqrt(inv_div *
-    // sum_j ssq[m nssq + j] + eps) -- an RMSNorm of X's rows applied after the product
-    const float* ssq; int nssq; float inv_div, eps;
-    int gate_c0;   // columns >= gate_c0 (a multiple of 16) are stored as silu(value)
-    // split K: ks slices of kslice (the last may be shorter); part (ks, M, N) row-major
-    int ks, kslice;
-    float* part;
 };
 
 __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
@@ -96,31 +78,24 @@ __device__ __forceinline__ void end_step() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int NJ, bool BETA, bool RS, bool SPLIT = false>
+template <int NJ, bool BETA>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs a) {
     constexpr int BN = 32 * NJ;
-    static_assert(!SPLIT || (!BETA && !RS), "the split kernel stores raw partials");
-    __shared__ float rs[RS ? BM : 1];
     __shared__ __attribute__((aligned(16))) float s0[kStage];
     __shared__ __attribute__((aligned(16))) float s1[kStage];
     __shared__ __attribute__((aligned(16))) float s2[kStage];
     __shared__ __attribute__((aligned(16))) float s3[kStage];
 
-    // ---- tile of this workgroup: consecutive ids per XCD, groups of GM row tiles (with
-    // split K, over the S times taller grid of (slice, row tile) pairs)
-    const int mtv = SPLIT ? a.mt * a.ks : a.mt;
-    const int T = mtv * a.nt;
+    // ---- tile of this workgroup: consecutive ids per XCD, groups of GM row tiles
+    const int T = a.mt * a.nt;
     const int b = blockIdx.x;
     const int xcd = b & 7, per = T >> 3, rem = T & 7;
     const int id = xcd * per + min(xcd, rem) + (b >> 3);
     const int gsz = GM * a.nt;
     const int grp = id / gsz, gr = id - grp * gsz;
-    const int gm = min(GM, mtv - grp * GM);
-    const int tmv = grp * GM + gr % gm, tn = gr / gm;
-    const int kz = SPLIT ? tmv / a.mt : 0, tm = SPLIT ? tmv - kz * a.mt : tmv;
-    // this workgroup's k range [kbeg, kbeg + K)
-    const int kbeg = SPLIT ? kz * a.kslice : 0;
-    const int K = SPLIT ? min(a.kslice, a.K - kbeg) : a.K;
+    const int gm = min(GM, a.mt - grp * GM);
+    const int tm = grp * GM + gr % gm, tn = gr / gm;
+    const int K = a.K;
 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -129,9 +104,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs a) {
 
     const int m0 = tm * BM, n0 = tn * BN;
     const int rows = min(BM, a.M - m0), cols = min(BN, a.N - n0);
-    const auto rx = ssm::rsrc(a.X + (long)m0 * a.ldx + kbeg,
+    const auto rx = ssm::rsrc(a.X + (long)m0 * a.ldx,
                               (unsigned)(((long)(rows - 1) * a.ldx + K) * 4));
-    const auto rw = ssm::rsrc(a.W + (long)n0 * a.ldw + kbeg,
+    const auto rw = ssm::rsrc(a.W + (long)n0 * a.ldw,
                               (unsigned)(((long)(cols - 1) * a.ldw + K) * 4));
 
     // Loads of wave w in a step: X row blocks 2w, 2w + 1 and W row blocks 2w, 2w + 1 (W row
@@ -222,39 +197,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs a) {
     for (; s + 7 <= nfull; s += 4) block(s, load);
     for (; s < nk; s += 4) block(s, load_tail);
 
-    // ---- row scales of the tile's rows (partial sums added in order)
-    if constexpr (RS) {
-        if (threadIdx.x < BM) {
-            float v = 1.f;
-            if ((int)threadIdx.x < rows) {
-                const float* p = a.ssq + (long)(m0 + threadIdx.x) * a.nssq;
-                float sum = 0.f;
-                for (int j = 0; j < a.nssq; ++j) sum += p[j];
-                v = rsqrtf(sum * a.inv_div + a.eps);
-            }
-            rs[threadIdx.x] = v;
-        }
-        __syncthreads();
-    }
-
     // ---- epilogue: acc[i][j][r] is Y[m0 + 16 (4 wm + i) + 4 q + r][n0 + 16 (NJ wn + j) + i16]
-    if constexpr (SPLIT) {   // the raw partial tile of slice kz
-        const auto rp = ssm::rsrc(a.part + ((long)kz * a.M + m0) * a.N + n0,
-                                  (unsigned)(((long)(rows - 1) * a.N + cols) * 4));
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int c = 16 * (NJ * wn + j) + i16;
-            const unsigned oor = c < cols ? 0u : 0x80000000u;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = 16 * (4 * wm + i) + 4 * q + r;
-                    ssm::bstore4(acc[i][j][r], rp, ((unsigned)(row * a.N + c) * 4u) | oor);
-                }
-        }
-        return;
-    }
     const auto ry = ssm::rsrc(a.Y + (long)m0 * a.ldy + n0,
                               (unsigned)(((long)(rows - 1) * a.ldy + cols) * 4));
 #pragma unroll
@@ -262,8 +205,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs a) {
         const int c = 16 * (NJ * wn + j) + i16;
         const unsigned oor = c < cols ? 0u : 0x80000000u;
         const float bv = a.bias && c < cols ? a.bias[n0 + c] : 0.f;
-        // the 16 columns of block j lie on one side of gate_c0: the choice is wave-uniform
-        const bool gate = n0 + 16 * (NJ * wn + j) >= a.gate_c0;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -271,47 +212,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmArgs a) {
                 const int row = 16 * (4 * wm + i) + 4 * q + r;
                 const unsigned off = ((unsigned)(row * a.ldy + c) * 4u) | oor;
                 float v = acc[i][j][r];
-                if constexpr (RS) v *= rs[row];
                 v += bv;
                 if constexpr (BETA) v += a.beta * ssm::bload4(ry, off);
-                if (gate) v = ssm::silu_fast(v);
                 ssm::bstore4(v, ry, off);
             }
-    }
-}
-
-// Split-K finish: Y = epilogue(sum over slices z = 0 .. ks-1 of part[z]), added in slice
-// order; the epilogue in the unsplit kernel's order (row scale, bias, beta, gate). Thread
-// (row m = blockIdx.y, columns 4 c4 .. 4 c4 + 3); N % 4 == 0.
-__global__ __launch_bounds__(256) void gemm_finish_kernel(GemmArgs a) {
-    const int m = blockIdx.y;
-    const int c4 = blockIdx.x * 256 + threadIdx.x;
-    if (4 * c4 >= a.N) return;
-    const long MN = (long)a.M * a.N;
-    const float4* p = reinterpret_cast<const float4*>(a.part + (long)m * a.N) + c4;
-    float4 v = p[0];
-    for (int z = 1; z < a.ks; ++z) {
-        const float4 u = p[z * (MN / 4)];
-        v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
-    }
-    float s = 1.f;
-    if (a.ssq) {   // same order as the unsplit kernel's row scales
-        const float* q = a.ssq + (long)m * a.nssq;
-        float sum = 0.f;
-        for (int j = 0; j < a.nssq; ++j) sum += q[j];
-        s = rsqrtf(sum * a.inv_div + a.eps);
-    }
-    float* y = a.Y + (long)m * a.ldy + 4 * c4;
-    float o[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int n = 4 * c4 + e;
-        float t = o[e];
-        if (a.ssq) t *= s;
-        if (a.bias) t += a.bias[n];
-        if (a.beta != 0.f) t += a.beta * y[e];
-        if (n >= a.gate_c0) t = ssm::silu_fast(t);
-        y[e] = t;
     }
 }
 
@@ -332,21 +236,9 @@ int pick_nj(int M, int N) {
 template <int NJ>
 void launch_nj(const GemmArgs& a, bool beta, hipStream_t st) {
     const dim3 block(256);
-    if (a.ks > 1) {
-        gemm_f32_kernel<NJ, false, false, true><<<dim3((unsigned)(a.mt * a.ks * a.nt)), block,
-                                                  0, st>>>(a);
-        gemm_finish_kernel<<<dim3((unsigned)((a.N / 4 + 255) / 256), (unsigned)a.M), block, 0,
-                             st>>>(a);
-        return;
-    }
     const dim3 grid((unsigned)(a.mt * a.nt));
-    if (a.ssq) {
-        if (beta) gemm_f32_kernel<NJ, true, true><<<grid, block, 0, st>>>(a);
-        else gemm_f32_kernel<NJ, false, true><<<grid, block, 0, st>>>(a);
-    } else {
-        if (beta) gemm_f32_kernel<NJ, true, false><<<grid, block, 0, st>>>(a);
-        else gemm_f32_kernel<NJ, false, false><<<grid, block, 0, st>>>(a);
-    }
+    if (beta) gemm_f32_kernel<NJ, true><<<grid, block, 0, st>>>(a);
+    else gemm_f32_kernel<NJ, false><<<grid, block, 0, st>>>(a);
 }
 
 // ---------------------------------------------------------------- x_proj -> dt_proj
@@ -583,61 +475,16 @@ bool gemm_ok(int M, int N, int K, long ldx, long ldw, long ldy) {
            (long)BM * ldy * 4 < lim;
 }
 
-// Tile width and split of K for a grid under two rounds of resident workgroups (pick_nj's
-// grid has fewer than 512 tiles): the (NJ, slice count) pair with the least modelled time
-// (above), slices at least 128 deep and a multiple of 16, within the workspace
-// (part_floats floats). Larger grids keep pick_nj's width, unsplit.
-struct Plan { int nj, ks, kslice; };
-Plan pick_plan(int M, int N, int K, size_t part_floats) {
-    const long mt = (M + BM - 1) / BM;
-    Plan p{pick_nj(M, N), 1, K};
-    if (mt * ((N + 32 * p.nj - 1) / (32 * p.nj)) >= 512) return p;
-    auto busy = [&](long wgs, int bn, int depth) {   // the most loaded CU's time (s)
-        const long n = (wgs + 255) / 256;
-        return (double)n * 2.0 * BM * bn * depth / (n == 1 ? 0.44e12 : 0.50e12);
-    };
-    double best = 1e300;
-    for (int nj : {2, 3, 4}) {
-        const int bn = 32 * nj;
-        const long tiles = mt * ((N + bn - 1) / bn);
-        const double t1 = busy(tiles, bn, K);
-        if (t1 < best) best = t1, p = Plan{nj, 1, K};
-        if (tiles >= 256 || N % 4 || K < 256) continue;
-        for (int ks = 2; ks <= K / 128; ++ks) {
-            if ((size_t)ks * M * N > part_floats) break;
-            const int sl = ((K + ks - 1) / ks + 15) / 16 * 16;
-            if ((K + sl - 1) / sl != ks) continue;
-            const double t = busy(tiles * ks, bn, sl) + 8.0 * ks * M * N / 5e12 + 4e-6;
-            if (t < best) best = t, p = Plan{nj, ks, sl};
-        }
-    }
-    return p;
-}
-
-size_t gemm_split_floats(int M, int N, int K) {
-    const Plan p = pick_plan(M, N, K, (size_t)-1);
-    return p.ks > 1 ? (size_t)p.ks * M * N : 0;
-}
-
 ssm_status launch_gemm(const float* X, long ldx, const float* W, long ldw, const float* bias,
-                       float* Y, long ldy, int M, int N, int K, float beta, hipStream_t st,
-                       const float* ssq, int nssq, float inv_div, float eps, int gate_c0,
-                       float* part, size_t part_floats) {
+                       float* Y, long ldy, int M, int N, int K, float beta, hipStream_t st) {
     if (!gemm_ok(M, N, K, ldx, ldw, ldy))
         return fail(SSM_ERR_INVALID_ARG, "gemm: unsupported shape M %d N %d K %d ld %ld/%ld/%ld",
                     M, N, K, ldx, ldw, ldy);
     if (((uintptr_t)X | (uintptr_t)W) & 15)
         return fail(SSM_ERR_INVALID_ARG, "gemm: X and W must be 16-byte aligned");
-    // with a workspace, the width and split of pick_plan; without, pick_nj's width unsplit
-    const bool ws = part && ((uintptr_t)part & 15) == 0;
-    const Plan p = ws ? pick_plan(M, N, K, part_floats) : Plan{pick_nj(M, N), 1, K};
-    const int nj = p.nj;
+    const int nj = pick_nj(M, N);
     GemmArgs a{X, ldx, W, ldw, Y, ldy, bias, M, N, K, beta, (M + BM - 1) / BM,
-               (N + 32 * nj - 1) / (32 * nj), ssq, nssq, inv_div, eps, gate_c0, p.ks, p.kslice,
-               p.ks > 1 ? part : nullptr};
-    if (gate_c0 < N && gate_c0 % 16)
-        return fail(SSM_ERR_INVALID_ARG, "gemm: gate column %d not a multiple of 16", gate_c0);
-    if (ssq && nssq <= 0) return fail(SSM_ERR_INVALID_ARG, "gemm: row scale needs nssq > 0");
+               (N + 32 * nj - 1) / (32 * nj)};
     if ((long)a.mt * a.nt > (1L << 30)) return fail(SSM_ERR_INVALID_ARG, "gemm: too many tiles");
     const bool bt = beta != 0.f;
     if (nj == 4) launch_nj<4>(a, bt, st);

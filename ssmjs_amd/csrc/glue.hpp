@@ -132,21 +132,29 @@ ssm_status launch_xg_ssq(const float* x, long ldx, const float* g, float* xg, fl
 // hid = E[ids] (M, d), then as launch_xg_ssq on hid with g; ids >= V flag *bad.
 ssm_status launch_embed_xg(const uint32_t* ids, const float* emb, float* hid, const float* g,
                            float* xg, float* ssq, int M, int d, int V, int* bad, hipStream_t st);
-// Prefill projection (gemm.hip): Y = beta * Y + s[m] X W^T (+ bias) on the fp32 matrix
-// cores; with ssq, s[m] = 1 / sqrt(inv_div * sum_j ssq[m nssq + j] + eps) (a row RMSNorm of
-// X applied after the product), else 1.
+// Projection (gemm.hip): Y = beta * Y + X W^T (+ bias) on the fp32 matrix cores, from operands
+// as they are.
 bool gemm_ok(int M, int N, int K, long ldx, long ldw, long ldy);
-// gate_c0 (a multiple of 16): columns n >= gate_c0 are stored as silu(value) (the Mamba-1
-// block's z half of in_proj, the scan's gate).
-// part (part_floats floats, 16-byte aligned): workspace of the split-K mode, used when the
-// tiles alone leave most CUs idle and part holds gemm_split_floats(M, N, K) floats; null
-// runs unsplit.
 ssm_status launch_gemm(const float* X, long ldx, const float* W, long ldw, const float* bias,
-                       float* Y, long ldy, int M, int N, int K, float beta, hipStream_t st,
-                       const float* ssq = nullptr, int nssq = 0, float inv_div = 0.f,
-                       float eps = 0.f, int gate_c0 = 0x7fffffff, float* part = nullptr,
-                       size_t part_floats = 0);
-size_t gemm_split_floats(int M, int N, int K);
+                       float* Y, long ldy, int M, int N, int K, float beta, hipStream_t st);
+// Prefill projection (gemm_h3.hip): Y = beta * Y + s[m] X W^T at fp32 precision on the fp16
+// matrix cores, from operands packed by launch_pack_h3 (h3_bytes(rows, K) bytes each, 16-byte
+// aligned); X and W are the same operands in fp32 (read for outputs that are not finite). With
+// ssq, s[m] = 1 / sqrt(inv_div * sum_j ssq[m nssq + j] + eps) (a row RMSNorm of X applied after
+// the product), else 1. Columns n >= gate_c0 (a multiple of 16) are stored as silu(value) (the
+// Mamba-1 block's z half of in_proj, the scan's gate). part (part_floats floats, 16-byte
+// aligned): workspace of the split-K mode, used where the tiles alone leave most CUs idle and
+// part holds h3_split_floats(M, N, K) floats; null runs unsplit.
+size_t h3_bytes(int rows, int K);
+bool h3_ok(int M, int N, int K, long ldx, long ldw, long ldy);
+size_t h3_split_floats(int M, int N, int K);
+ssm_status launch_pack_h3(const float* X, long ldx, int rows, int K, void* packed,
+                          hipStream_t st);
+ssm_status launch_gemm_h3(const void* Xp, const float* X, long ldx, const void* Wp,
+                          const float* W, long ldw, float* Y, long ldy, int M, int N, int K,
+                          float beta, hipStream_t st, const float* ssq = nullptr, int nssq = 0,
+                          float inv_div = 0.f, float eps = 0.f, int gate_c0 = 0x7fffffff,
+                          float* part = nullptr, size_t part_floats = 0);
 // The Mamba-1 block's x_proj and dt_proj in one pass (gemm.hip): dbl = x Wx^T (T, R + 2N),
 // dt = dbl[:, :R] Wdt^T (T, D); given dt_bias, dt = softplus(dbl[:, :R] Wdt^T + dt_bias) (the
 // scan's dt').

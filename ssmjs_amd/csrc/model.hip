@@ -10,8 +10,8 @@
 //                 dt = dt_proj(dt); y = scan(x, dt, A, B, C, D, z, softplus(dt + bias)); out_proj
 //   mamba2 mixer: in_proj -> (z, xBC, dt); xBC = SiLU(conv(xBC)); y = SSD(x, dt, A, B, C, D);
 //                 y = RMSNorm_grouped(y * SiLU(z)); out_proj
-// Projections are rocBLAS SGEMMs on the context stream; the residual add is folded into the
-// out_proj GEMM (beta = 1).
+// Projections run on the context stream (own kernels, hipBLASLt / rocBLAS for the shapes those
+// do not take); the residual add is folded into out_proj (beta = 1).
 #include <hipblaslt/hipblaslt.h>
 #include <rocblas/rocblas.h>
 
@@ -253,11 +253,12 @@ ssm_ctx::LtPlan& lt_plan(ssm_ctx* c, int M, int Nout, int K, long ldx, long ldy,
 }
 
 // Y (M, Nout) [ld ldy] = X (M, K) [ld ldx] * W^T, W (Nout, K) row-major; Y = beta*Y + ...
-// Products of M >= kOwnGemmRows rows run the fp32 matrix-core kernel of gemm.hip (split over
-// K when its tiles leave CUs idle and a workspace is given); the prefill of up to
-// kFewRows tokens runs the row kernel of rowgemm.hip (proj_rows); the rest (prompts of 65 to
-// 255 tokens, the one-token fallbacks) go to hipBLASLt for K >= 128 (below that rocBLAS
-// measured faster) and rocBLAS for the rest and any shape hipBLASLt has no algorithm for.
+// The prefill's products run elsewhere: up to kFewRows tokens on the row kernel of rowgemm.hip
+// (proj_rows), more on the split fp16 kernel of gemm_h3.hip (proj_h3). What is left here (the
+// narrow dt_proj, the one-token fallbacks, shapes those kernels do not take) goes to the fp32
+// matrix-core kernel of gemm.hip from kOwnGemmRows rows on, to hipBLASLt for K >= 128 (below
+// that rocBLAS measured faster) and to rocBLAS for the rest and any shape hipBLASLt has no
+// algorithm for.
 // SSM_GEMM=lib sends every product to the libraries, SSM_GEMM=rocblas everything to rocBLAS.
 constexpr int kOwnGemmRows = 256;
 constexpr int kFewRows = 64;
@@ -270,9 +271,9 @@ bool lib_only() {
 }
 bool own_kernels(int M) { return !lib_only() && M >= kOwnGemmRows; }
 bool few_rows(int M) { return !lib_only() && M >= 1 && M <= kFewRows; }
-// part / part_n: the own kernel's split-K workspace (gemm.hip; null runs unsplit).
+bool h3_rows(long M) { return !lib_only() && M > kFewRows; }
 ssm_status gemm(ssm_ctx* c, int M, int Nout, int K, const float* X, long ldx, const float* W,
-                float* Y, long ldy, float beta, float* part = nullptr, size_t part_n = 0) {
+                float* Y, long ldy, float beta) {
     if (M == 0 || Nout == 0) return SSM_OK;
     const float one = 1.f;
     static const bool rb_only = [] {
@@ -281,8 +282,7 @@ ssm_status gemm(ssm_ctx* c, int M, int Nout, int K, const float* X, long ldx, co
     }();
     if (own_kernels(M) && ssm::gemm_ok(M, Nout, K, ldx, K, ldy) &&
         (((uintptr_t)X | (uintptr_t)W) & 15) == 0)
-        return ssm::launch_gemm(X, ldx, W, K, nullptr, Y, ldy, M, Nout, K, beta, c->stream,
-                                nullptr, 0, 0.f, 0.f, 0x7fffffff, part, part_n);
+        return ssm::launch_gemm(X, ldx, W, K, nullptr, Y, ldy, M, Nout, K, beta, c->stream);
     if (c->lt && K >= 128 && !rb_only) {
         auto& p = lt_plan(c, M, Nout, K, ldx, ldy);
         if (p.ok) {
@@ -534,6 +534,12 @@ struct ssm_model {
     // at its first call and rebuilt whenever the weights change
     __bf16* wb = nullptr;
     std::vector<long> wb_in, wb_out;   // element offsets into wb per layer (-1: none)
+    // the projections' weights packed for gemm_h3.hip, built at the first prefill of more than
+    // kFewRows tokens (the tied embedding: at the first such product with it) and rebuilt
+    // whenever the weights change; byte offsets into wh per layer (-1: none)
+    char* wh = nullptr;
+    std::vector<long> wh_in, wh_out, wh_x;
+    char* wh_emb = nullptr;
     int* d_flag = nullptr;   // out-of-range token id flag
     uint32_t* d_ids = nullptr;
     size_t ids_cap = 0;
@@ -631,6 +637,52 @@ void build_layout(ssm_model* m) {
 
 ssm_status pack_weights(ssm_model* m);
 
+// Packed copies (gemm_h3.hip) of the layers' in_proj and out_proj, and of the Mamba-1 layers'
+// x_proj. Weights that kernel does not take (rows not 16-byte aligned) have none.
+ssm_status build_wh(ssm_model* m) {
+    const Dims& d = m->dm;
+    hipStream_t st = m->ctx->stream;
+    const int RN = d.R + 2 * d.N;
+    auto ok = [&](long off, int K) { return K % 4 == 0 && ((uintptr_t)(m->w + off) & 15) == 0; };
+    if (!m->wh) {
+        m->wh_in.assign(d.nl, -1);
+        m->wh_out.assign(d.nl, -1);
+        m->wh_x.assign(d.nl, -1);
+        long off = 0;
+        auto take = [&](long& at, long w, int rows, int K) {
+            if (!ok(w, K)) return;
+            at = off;
+            off += (long)ssm::h3_bytes(rows, K);
+        };
+        for (int l = 0; l < d.nl; ++l) {
+            const LayerW& Ly = m->layers[l];
+            const bool m1 = Ly.type == SSM_LAYER_MAMBA1;
+            take(m->wh_in[l], Ly.in_proj, m1 ? 2 * d.D : d.nin, d.d);
+            take(m->wh_out[l], Ly.out_proj, d.d, d.D);
+            if (m1) take(m->wh_x[l], Ly.x_proj, RN, d.D);
+        }
+        SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh, off ? (size_t)off : 1));
+    }
+    for (int l = 0; l < d.nl; ++l) {
+        const LayerW& Ly = m->layers[l];
+        const bool m1 = Ly.type == SSM_LAYER_MAMBA1;
+        if (m->wh_in[l] >= 0)
+            SSM_TRY(ssm::launch_pack_h3(m->w + Ly.in_proj, d.d, m1 ? 2 * d.D : d.nin, d.d,
+                                        m->wh + m->wh_in[l], st));
+        if (m->wh_out[l] >= 0)
+            SSM_TRY(ssm::launch_pack_h3(m->w + Ly.out_proj, d.D, d.d, d.D, m->wh + m->wh_out[l],
+                                        st));
+        if (m->wh_x[l] >= 0)
+            SSM_TRY(ssm::launch_pack_h3(m->w + Ly.x_proj, d.D, RN, d.D, m->wh + m->wh_x[l], st));
+    }
+    return SSM_OK;
+}
+ssm_status build_wh_emb(ssm_model* m) {
+    const Dims& d = m->dm;
+    if (!m->wh_emb) SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh_emb, ssm::h3_bytes(d.V, d.d)));
+    return ssm::launch_pack_h3(m->w + m->emb, d.d, d.V, d.d, m->wh_emb, m->ctx->stream);
+}
+
 // bf16 (round to nearest even) copies of the Mamba-2 layers' in_proj and out_proj.
 ssm_status build_wb(ssm_model* m) {
     const Dims& d = m->dm;
@@ -666,6 +718,8 @@ ssm_status refresh_A(ssm_model* m) {
         SSM_TRY(ssm::launch_neg_exp(m->w + L.A_log, m->Ab + L.A, n, st));
     }
     if (m->wb) SSM_TRY(build_wb(m));
+    if (m->wh) SSM_TRY(build_wh(m));
+    if (m->wh_emb) SSM_TRY(build_wh_emb(m));
     return m->wp ? pack_weights(m) : SSM_OK;
 }
 
@@ -720,8 +774,11 @@ struct Ws {
     // T <= kStepProjMaxRows (one-token steps, short forwards), else a prefill's B last
     // positions when B <= kStepProjMaxRows; null otherwise
     float* hpart;
-    // split-K partials of the own prefill GEMM (gemm.hip) for the largest split product of
-    // the mixers at T tokens (gpart_n floats); null when none splits
+    // the packed left operand of a product of more than kFewRows rows (gemm_h3.hip), and the
+    // split-K partials of the largest split product at T tokens (gpart_n floats; null when
+    // none splits)
+    void* xh;
+    size_t xh_bytes;
     float* gpart;
     size_t gpart_n;
     void* scan;
@@ -776,17 +833,25 @@ size_t plan_ws(ssm_model* m, int B, int L, bool full_logits, Ws* out) {
     size_t o_xp = off; off += al(4 * nxp);
     const size_t nhp = nhead * (size_t)ssm::head_parts(d.V) * 2;
     size_t o_hp = off; off += al(4 * nhp);
-    size_t ngp = 0;
-    if (T >= (size_t)kOwnGemmRows && T <= (size_t)INT32_MAX) {
+    size_t ngp = 0, nxh = 0;
+    if (h3_rows((long)T) && T <= (size_t)INT32_MAX) {
         const int t = (int)T;
-        if (has1)
-            for (auto nk : {std::pair<int, int>{2 * d.D, d.d}, {d.d, d.D}, {d.R + 2 * d.N, d.D},
-                            {d.D, d.R}})
-                ngp = std::max(ngp, ssm::gemm_split_floats(t, nk.first, nk.second));
-        if (has2)
-            for (auto nk : {std::pair<int, int>{d.nin, d.d}, {d.d, d.D}})
-                ngp = std::max(ngp, ssm::gemm_split_floats(t, nk.first, nk.second));
+        auto product = [&](int rows, int n, int k) {
+            ngp = std::max(ngp, ssm::h3_split_floats(rows, n, k));
+            nxh = std::max(nxh, ssm::h3_bytes(rows, k));
+        };
+        if (has1) {
+            product(t, 2 * d.D, d.d);
+            product(t, d.d, d.D);
+            product(t, d.R + 2 * d.N, d.D);
+        }
+        if (has2) {
+            product(t, d.nin, d.d);
+            product(t, d.d, d.D);
+        }
+        if (nhead == 0) product(full_logits ? t : B, d.V, d.d);
     }
+    size_t o_xh = off; off += al(nxh);
     size_t o_gp = off; off += al(4 * ngp);
     if (out) {
         char* base = m->ws;
@@ -802,6 +867,8 @@ size_t plan_ws(ssm_model* m, int B, int L, bool full_logits, Ws* out) {
         out->ssq_y = nstep ? (float*)(base + o_sqy) : nullptr;
         out->xpart = nxp ? (float*)(base + o_xp) : nullptr;
         out->hpart = nhp ? (float*)(base + o_hp) : nullptr;
+        out->xh = nxh ? base + o_xh : nullptr;
+        out->xh_bytes = nxh;
         out->gpart = ngp ? (float*)(base + o_gp) : nullptr;
         out->gpart_n = ngp;
     }
@@ -840,10 +907,28 @@ ssm_status proj_rows(ssm_model* m, int mode, const float* x, long ldx, const flo
                      float beta, float* tmp, const float* g2 = nullptr, float* nout = nullptr,
                      bool* normed = nullptr, bool rows = false);
 
+// Y (M, N) [ld ldy] = beta Y + s[m] X W^T on the split fp16 kernel (gemm_h3.hip): X packed into
+// the workspace, then the product with W's packed copy Wp. ssq / nssq / inv_div: the row scale;
+// gate_c0: silu from that column on.
+bool h3_product_ok(const Ws& w, const void* Wp, int M, int N, int K, const float* X, long ldx,
+                   const float* W, long ldy) {
+    return h3_rows(M) && w.xh && Wp && ssm::h3_ok(M, N, K, ldx, K, ldy) && al16(X) && al16(W) &&
+           ssm::h3_bytes(M, K) <= w.xh_bytes;
+}
+ssm_status proj_h3(ssm_model* m, const Ws& w, int M, int N, int K, const float* X, long ldx,
+                   const float* W, const void* Wp, float* Y, long ldy, float beta,
+                   const float* ssq = nullptr, int nssq = 0, float inv_div = 0.f,
+                   int gate_c0 = 0x7fffffff) {
+    hipStream_t st = m->ctx->stream;
+    SSM_TRY(ssm::launch_pack_h3(X, ldx, M, K, w.xh, st));
+    return ssm::launch_gemm_h3(w.xh, X, ldx, Wp, W, K, Y, ldy, M, N, K, beta, st, ssq, nssq,
+                               inv_div, m->dm.eps, gate_c0, w.gpart, w.gpart_n);
+}
+
 // One mixer over (B, L) tokens: reads x (T, d) [normalised], adds its output into out (T, d)
 // with beta (0: overwrite, 1: residual add). ssm/conv state may be null (zero initial state).
-// Its products: up to kFewRows tokens on the row kernel (proj_rows), else gemm() (the own
-// kernel from kOwnGemmRows rows, with the split-K workspace).
+// Its products: up to kFewRows tokens on the row kernel (proj_rows), more on the split fp16
+// kernel (proj_h3), and gemm() for what neither takes.
 ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, float beta, int B,
                  int L, float* ssm_st, float* conv_st, const Ws& w) {
     const Dims& d = m->dm;
@@ -853,12 +938,20 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
     const float* W = m->w;
     const float* A = m->Ab + Ly.A;
     const bool few = few_rows(T);
-    auto proj = [&](int N, int K, const float* X, long ldx, const float* Wt, float* Y, long ldy,
-                    float b) -> ssm_status {
+    if (h3_rows(T) && !m->wh) SSM_TRY(build_wh(m));
+    const long l = &Ly - m->layers.data();
+    auto packed = [&](const std::vector<long>& at) -> const void* {
+        return m->wh && at[l] >= 0 ? m->wh + at[l] : nullptr;
+    };
+    const void *Wp_in = packed(m->wh_in), *Wp_out = packed(m->wh_out), *Wp_x = packed(m->wh_x);
+    auto proj = [&](int N, int K, const float* X, long ldx, const float* Wt, const void* Wp,
+                    float* Y, long ldy, float b) -> ssm_status {
         if (few)
             return proj_rows(m, 0, X, ldx, nullptr, 0, nullptr, Wt, Y, ldy, T, N, K, b, nullptr,
                              nullptr, nullptr, nullptr, true);
-        return gemm(c, T, N, K, X, ldx, Wt, Y, ldy, b, w.gpart, w.gpart_n);
+        if (h3_product_ok(w, Wp, T, N, K, X, ldx, Wt, ldy))
+            return proj_h3(m, w, T, N, K, X, ldx, Wt, Wp, Y, ldy, b);
+        return gemm(c, T, N, K, X, ldx, Wt, Y, ldy, b);
     };
     if (Ly.type == SSM_LAYER_MAMBA1) {
         float *xz = w.a, *xc = w.b, *dbl = w.c, *dtv = w.d, *y = w.e;
@@ -871,13 +964,12 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
         const bool fused_xd = own_kernels(T) && (T + 31) / 32 >= 256 &&
                               ssm::xproj_dt_ok(T, d.D, d.R, d.N, d.D, RN, d.D) &&
                               al16(W + Ly.x_proj) && al16(W + Ly.dt_w);
-        const bool pre = fused_xd && ssm::gemm_ok(T, 2 * d.D, d.d, d.d, d.d, 2 * d.D) &&
-                         al16(x) && al16(W + Ly.in_proj) && d.D % 16 == 0;
+        const bool pre = fused_xd && d.D % 16 == 0 &&
+                         h3_product_ok(w, Wp_in, T, 2 * d.D, d.d, x, d.d, W + Ly.in_proj, 2 * d.D);
         { Stage g(c, "m1.in_proj");
-          if (pre) SSM_TRY(ssm::launch_gemm(x, d.d, W + Ly.in_proj, d.d, nullptr, xz, 2 * d.D, T,
-                                            2 * d.D, d.d, 0.f, st, nullptr, 0, 0.f, 0.f, d.D,
-                                            w.gpart, w.gpart_n));
-          else SSM_TRY(proj(2 * d.D, d.d, x, d.d, W + Ly.in_proj, xz, 2 * d.D, 0.f)); }
+          if (pre) SSM_TRY(proj_h3(m, w, T, 2 * d.D, d.d, x, d.d, W + Ly.in_proj, Wp_in, xz,
+                                   2 * d.D, 0.f, nullptr, 0, 0.f, d.D));
+          else SSM_TRY(proj(2 * d.D, d.d, x, d.d, W + Ly.in_proj, Wp_in, xz, 2 * d.D, 0.f)); }
         { Stage g(c, "m1.conv");
           SSM_TRY(ssm_causal_conv1d(xz, 2 * d.D, W + Ly.conv_w, W + Ly.conv_b, xc, d.D, B, L, d.D,
                                     d.K, 1, conv_st, conv_st, st)); }
@@ -887,26 +979,25 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
             SSM_TRY(ssm::launch_xproj_dt(xc, d.D, W + Ly.x_proj, W + Ly.dt_w, dbl, RN, dtv, d.D,
                                          T, d.D, d.R, d.N, st, pre ? W + Ly.dt_b : nullptr));
         } else {
-            { Stage g(c, "m1.x_proj"); SSM_TRY(proj(RN, d.D, xc, d.D, W + Ly.x_proj, dbl, RN, 0.f)); }
-            { Stage g(c, "m1.dt_proj"); SSM_TRY(proj(d.D, d.R, dbl, RN, W + Ly.dt_w, dtv, d.D, 0.f)); }
+            { Stage g(c, "m1.x_proj"); SSM_TRY(proj(RN, d.D, xc, d.D, W + Ly.x_proj, Wp_x, dbl, RN, 0.f)); }
+            { Stage g(c, "m1.dt_proj"); SSM_TRY(proj(d.D, d.R, dbl, RN, W + Ly.dt_w, nullptr, dtv, d.D, 0.f)); }
         }
         { Stage g(c, "m1.scan");
           SSM_TRY(ssm::selective_scan(xc, d.D, dtv, d.D, pre ? nullptr : W + Ly.dt_b, pre ? 0 : 1,
                                       A, dbl + d.R, RN, dbl + d.R + d.N, RN, W + Ly.Dsk, xz + d.D,
                                       2 * d.D, pre ? 1 : 0, y, d.D, B, L, d.D, d.N, ssm_st, ssm_st,
                                       w.scan, w.scan_bytes, st)); }
-        { Stage g(c, "m1.out_proj"); SSM_TRY(proj(d.d, d.D, y, d.D, W + Ly.out_proj, out, d.d, beta)); }
+        { Stage g(c, "m1.out_proj"); SSM_TRY(proj(d.d, d.D, y, d.D, W + Ly.out_proj, Wp_out, out, d.d, beta)); }
     } else {
         float *zx = w.a, *xbc = w.b, *y = w.c, *yn = w.d;
         const int GN = d.G * d.N;
-        { Stage g(c, "m2.in_proj"); SSM_TRY(proj(d.nin, d.d, x, d.d, W + Ly.in_proj, zx, d.nin, 0.f)); }
+        { Stage g(c, "m2.in_proj"); SSM_TRY(proj(d.nin, d.d, x, d.d, W + Ly.in_proj, Wp_in, zx, d.nin, 0.f)); }
         { Stage g(c, "m2.conv");
           SSM_TRY(ssm_causal_conv1d(zx + d.D, d.nin, W + Ly.conv_w, W + Ly.conv_b, xbc, d.cd, B, L,
                                     d.cd, d.K, 1, conv_st, conv_st, st)); }
         const float* dtp = zx + d.D + d.cd;
         const bool fuse_gate =
-            own_kernels(T) && ssm::gemm_ok(T, d.d, d.D, d.D, d.D, d.d) &&
-            al16(W + Ly.out_proj) &&
+            h3_product_ok(w, Wp_out, T, d.d, d.D, y, d.D, W + Ly.out_proj, d.d) &&
             ssm::ssd_gated_ok(d.P, d.G, d.N, d.cd, d.nin, d.cd, d.cd, d.D, d.nin, xbc, xbc + d.D,
                               xbc + d.D + GN, y, zx, W + Ly.gnorm);
         if (fuse_gate) {
@@ -919,9 +1010,8 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
                                    d.H, d.G, d.N, ssm_st, ssm_st, w.scan, w.scan_bytes, st, zx,
                                    d.nin, W + Ly.gnorm, yn)); }
             { Stage g(c, "m2.out_proj");
-              SSM_TRY(ssm::launch_gemm(y, d.D, W + Ly.out_proj, d.D, nullptr, out, d.d, T, d.d,
-                                       d.D, beta, st, yn, d.H, 1.f / (float)d.D, d.eps,
-                                       0x7fffffff, w.gpart, w.gpart_n)); }
+              SSM_TRY(proj_h3(m, w, T, d.d, d.D, y, d.D, W + Ly.out_proj, Wp_out, out, d.d, beta,
+                              yn, d.H, 1.f / (float)d.D)); }
         } else {
             { Stage g(c, "m2.ssd");
               SSM_TRY(ssm_ssd_chunk_scan(SSM_F32, xbc, d.cd, dtp, d.nin, W + Ly.dt_b, 1,
@@ -937,8 +1027,7 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
                   SSM_TRY(ssm_gated_rmsnorm(y, d.D, zx, d.nin, W + Ly.gnorm, yn, d.D, T, d.D, d.G,
                                             d.eps, st)); }
                 { Stage g(c, "m2.out_proj");
-                  SSM_TRY(gemm(c, T, d.d, d.D, yn, d.D, W + Ly.out_proj, out, d.d, beta, w.gpart,
-                               w.gpart_n)); }
+                  SSM_TRY(proj(d.d, d.D, yn, d.D, W + Ly.out_proj, Wp_out, out, d.d, beta)); }
             }
         }
     }
@@ -1382,6 +1471,16 @@ ssm_status head_rows(ssm_model* m, const Ws& w, const float* x, long ldx, int ro
                             m->wp + m->wp_emb, lg, d.V, rows, d.V, d.d, w.hpart, d_argmax, st);
 }
 
+// The LM head over more rows than the own head takes: x already normalised.
+ssm_status head_many(ssm_model* m, const Ws& w, const float* x, int rows, float* lg) {
+    const Dims& d = m->dm;
+    const float* E = m->w + m->emb;
+    if (h3_rows(rows) && w.xh && d.d % 4 == 0 && !m->wh_emb) SSM_TRY(build_wh_emb(m));
+    if (h3_product_ok(w, m->wh_emb, rows, d.V, d.d, x, d.d, E, d.V))
+        return proj_h3(m, w, rows, d.V, d.d, x, d.d, E, m->wh_emb, lg, d.V, 0.f);
+    return gemm(m->ctx, rows, d.V, d.d, x, d.d, E, lg, d.V, 0.f);
+}
+
 ssm_status check_flag(ssm_model* m) {
     int bad = 0;
     SSM_HIP_TRY(hipMemcpyAsync(&bad, m->d_flag, sizeof(int), hipMemcpyDeviceToHost,
@@ -1479,7 +1578,7 @@ extern "C" ssm_status ssm_model_destroy(ssm_model* m) {
         hipSetDevice(m->ctx->device);
         hipStreamSynchronize(m->ctx->stream);
         hipFree(m->w); hipFree(m->Ab); hipFree(m->ws); hipFree(m->d_flag); hipFree(m->d_ids);
-        hipFree(m->rg); hipFree(m->wp); hipFree(m->wb);
+        hipFree(m->rg); hipFree(m->wp); hipFree(m->wb); hipFree(m->wh); hipFree(m->wh_emb);
     }
     m->destroyed = true;
     return SSM_OK;
@@ -1576,8 +1675,7 @@ extern "C" ssm_status ssm_forward_device(ssm_model* m, const uint32_t* d_ids, in
     const bool own = own_head_ok(m, w, T);
     SSM_TRY(trunk(m, d_ids, B, L, nullptr, w, !own));
     if (own) return head_rows(m, w, w.hid, m->dm.d, (int)T, d_logits, nullptr);
-    return gemm(m->ctx, B * L, m->dm.V, m->dm.d, w.nrm, m->dm.d, m->w + m->emb, d_logits,
-                m->dm.V, 0.f);
+    return head_many(m, w, w.nrm, B * L, d_logits);
 }
 
 extern "C" ssm_status ssm_forward(ssm_model* m, const uint32_t* ids, int B, int L,
@@ -1594,8 +1692,7 @@ extern "C" ssm_status ssm_forward(ssm_model* m, const uint32_t* ids, int B, int 
     const bool own = own_head_ok(m, w, (long)T);
     SSM_TRY(trunk(m, m->d_ids, B, L, nullptr, w, !own));
     if (own) SSM_TRY(head_rows(m, w, w.hid, m->dm.d, (int)T, w.logits, nullptr));
-    else SSM_TRY(gemm(m->ctx, (int)T, m->dm.V, m->dm.d, w.nrm, m->dm.d, m->w + m->emb, w.logits,
-                      m->dm.V, 0.f));
+    else SSM_TRY(head_many(m, w, w.nrm, (int)T, w.logits));
     SSM_HIP_TRY(hipMemcpyAsync(logits, w.logits, T * m->dm.V * 4, hipMemcpyDeviceToHost,
                                m->ctx->stream));
     return check_flag(m);
@@ -1759,7 +1856,7 @@ ssm_status prefill_device(ssm_model* m, ssm_state* s, const uint32_t* d_ids, int
         return head_rows(m, w, w.hid + (long)(L - 1) * d.d, (long)L * d.d, s->B, s->d_logits,
                          d_argmax);
     SSM_TRY(ssm::launch_gather_rows(w.nrm, L, L - 1, w.last, s->B, d.d, m->ctx->stream));
-    SSM_TRY(gemm(m->ctx, s->B, d.V, d.d, w.last, d.d, m->w + m->emb, s->d_logits, d.V, 0.f));
+    SSM_TRY(head_many(m, w, w.last, s->B, s->d_logits));
     if (d_argmax) SSM_TRY(ssm::launch_argmax(s->d_logits, d.V, s->B, d.V, d_argmax, m->ctx->stream));
     return SSM_OK;
 }
