@@ -1002,16 +1002,16 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
                               xbc + d.D + GN, y, zx, W + Ly.gnorm);
         if (fuse_gate) {
             // The gated RMSNorm split over its neighbours: the SSD stores u * g (u = y silu(z))
-            // and per-head sums of u^2 (in yn's space), and out_proj scales each row by
+            // and sums of u^2 per 64 channels (in yn's space), and out_proj scales each row by
             // 1 / rms(u) after the product.
             { Stage g(c, "m2.ssd_gate");
               SSM_TRY(ssm::ssd_f32(xbc, d.cd, dtp, d.nin, W + Ly.dt_b, 1, 0.f, INFINITY, A,
                                    xbc + d.D, d.cd, xbc + d.D + GN, d.cd, W + Ly.Dsk, y, d.D, B, L,
-                                   d.H, d.G, d.N, ssm_st, ssm_st, w.scan, w.scan_bytes, st, zx,
-                                   d.nin, W + Ly.gnorm, yn)); }
+                                   d.H, d.P, d.G, d.N, ssm_st, ssm_st, w.scan, w.scan_bytes, st,
+                                   zx, d.nin, W + Ly.gnorm, yn)); }
             { Stage g(c, "m2.out_proj");
               SSM_TRY(proj_h3(m, w, T, d.d, d.D, y, d.D, W + Ly.out_proj, Wp_out, out, d.d, beta,
-                              yn, d.H, 1.f / (float)d.D)); }
+                              yn, d.D / 64, 1.f / (float)d.D)); }
         } else {
             { Stage g(c, "m2.ssd");
               SSM_TRY(ssm_ssd_chunk_scan(SSM_F32, xbc, d.cd, dtp, d.nin, W + Ly.dt_b, 1,

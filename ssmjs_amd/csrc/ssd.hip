@@ -1087,14 +1087,17 @@ bool chunked_fallback_shape(int Pd, int G, int N) {
 
 extern "C" size_t ssm_ssd_workspace(int B, int L, int H, int Pd, int G, int N) {
     if (B <= 0 || L <= 0 || H <= 0 || Pd <= 0 || N <= 0) return 0;
-    if (chunked_fallback_shape(Pd, G, N)) return chunked_fallback_bytes(B, L, H, Pd, N);
-    if (Pd != P || (N != 64 && N != 128)) return 0;
+    // (operands the matrix-core kernel does not take, by alignment, may need the fallback's)
+    const size_t f32 = ssm::ssd_f32_workspace(B, L, H, G, Pd, N);
+    if (chunked_fallback_shape(Pd, G, N))
+        return std::max(f32, chunked_fallback_bytes(B, L, H, Pd, N));
+    if (Pd != P || (N != 64 && N != 128)) return f32;
     // the larger of the bf16 kernel's and the fp32 kernel's segment states (the size does
     // not depend on the element type the caller will pass)
     int nchunks, nseg, per;
     plan(B, L, H, nchunks, nseg, per);
     const size_t bf = nseg <= 1 ? 0 : sizeof(float) * (size_t)B * H * nseg * ((size_t)Pd * N + 1);
-    return std::max(bf, ssm::ssd_f32_workspace(B, L, H, G, Pd, N));
+    return std::max(bf, f32);
 }
 
 namespace ssm {
@@ -1158,6 +1161,23 @@ extern "C" ssm_status ssm_ssd_chunk_scan(int in_dtype, const void* x, long ldx, 
     a.ldc = ldc; a.Dsk = Dsk; a.y = y; a.ldy = ldy; a.B = B; a.L = L; a.H = H; a.G = G; a.N = N;
     a.h0 = h0; a.hT = hT;
     hipStream_t st = (hipStream_t)stream;
+    // Head dims of 128, 192, ... and d_state 16 and 32 (the session presets' Mamba-2 heads) on
+    // the fp32 matrix-core kernel too, which takes 64 state rows per workgroup head: 12 heads of
+    // 128 x 16 over 2000 steps 61 -> 23 us against the scan over H*P channels below, which reads
+    // dt and the states once per channel. It wants 16-byte rows and, for a sequence cut into
+    // segments, their workspace; calls without either keep the routes below.
+    const bool f32_rows = ldx % 4 == 0 && ldy % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 &&
+                          (((uintptr_t)x | (uintptr_t)y | (uintptr_t)Bm | (uintptr_t)Cm |
+                            (uintptr_t)h0 | (uintptr_t)hT) & 15) == 0;
+    if (!mfma_path && in_dtype == SSM_F32 && ssm::ssd_f32_shape(Pd, N) && offsets_fit &&
+        f32_rows) {
+        const size_t least = ssm::ssd_f32_least_workspace(B, L, H, Pd, N);
+        if (least == 0 || (workspace && workspace_bytes >= least &&
+                           ((uintptr_t)workspace & 15) == 0))
+            return ssm::ssd_f32((const float*)x, ldx, dt, lddt, dt_bias, softplus, dt_min, dt_max,
+                                A, (const float*)Bm, ldb, (const float*)Cm, ldc, Dsk, y, ldy, B, L,
+                                H, Pd, G, N, h0, hT, workspace, workspace_bytes, st);
+    }
     // the Mamba-1 scan has no dt clamp: it stands in when the clamp cannot bind
     const bool no_clamp = (softplus && dt_min <= 0.f && dt_max == INFINITY) ||
                           (dt_min == -INFINITY && dt_max == INFINITY);
@@ -1187,8 +1207,8 @@ extern "C" ssm_status ssm_ssd_chunk_scan(int in_dtype, const void* x, long ldx, 
                                    : launch_ssd_seq<__bf16>(a, Pd, st);
     if (in_dtype == SSM_F32)
         return ssm::ssd_f32((const float*)x, ldx, dt, lddt, dt_bias, softplus, dt_min, dt_max, A,
-                            (const float*)Bm, ldb, (const float*)Cm, ldc, Dsk, y, ldy, B, L, H, G,
-                            N, h0, hT, workspace, workspace_bytes, st);
+                            (const float*)Bm, ldb, (const float*)Cm, ldc, Dsk, y, ldy, B, L, H,
+                            Pd, G, N, h0, hT, workspace, workspace_bytes, st);
     plan(B, L, H, a.nchunks, a.nseg, a.chunks_per_seg);
     if (a.nseg > 1) {
         // the bf16 kernel's own part: the segment states and decays

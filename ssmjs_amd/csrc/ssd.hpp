@@ -6,18 +6,20 @@
 
 namespace ssm {
 
-// Head dim 64 with d_state 64 or 128: the shapes the fp32 kernel takes.
+// Head dims in multiples of 64 with d_state 16, 32, 64 or 128: the shapes the fp32 kernel takes.
 bool ssd_f32_shape(int Pd, int N);
-// Workspace bytes of ssd_f32 (segment states when long sequences are cut into segments).
+// Workspace bytes of ssd_f32 (segment states when long sequences are cut into segments, the
+// C B^T tiles), and the part of it that it cannot do without.
 size_t ssd_f32_workspace(int B, int L, int H, int G, int Pd, int N);
+size_t ssd_f32_least_workspace(int B, int L, int H, int Pd, int N);
 // The SSD of ssm_ssd_chunk_scan for float32 inputs (arguments as there; shapes checked by the
 // caller). With ssq, the output carries the gated RMSNorm's element-wise part instead of y:
 // y <- u * gn with u = y * silu(z) (z (B*L, H*P), row stride ldz; gn (H*P)), and
-// ssq[(b L + t) H + h] = sum over head h's P channels of u^2.
+// ssq[(b L + t) (H P / 64) + k] = sum of u^2 over the 64 channels from 64 k on.
 ssm_status ssd_f32(const float* x, long ldx, const float* dt, long lddt, const float* dt_bias,
                    int softplus, float dt_min, float dt_max, const float* A, const float* Bm,
                    long ldb, const float* Cm, long ldc, const float* Dsk, float* y, long ldy,
-                   int B, int L, int H, int G, int N, const float* h0, float* hT,
+                   int B, int L, int H, int Pd, int G, int N, const float* h0, float* hT,
                    void* workspace, size_t workspace_bytes, hipStream_t st,
                    const float* z = nullptr, long ldz = 0, const float* gn = nullptr,
                    float* ssq = nullptr);

@@ -50,7 +50,7 @@
 namespace {
 
 constexpr int QF = 32;       // time steps per chunk
-constexpr int PF = 64;       // head dim
+constexpr int PF = 64;       // rows of a head's state per workgroup head (below: "head")
 constexpr int kTargetWG = 512;
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -68,11 +68,12 @@ struct F32Args {
     const float* Cm; long ldc;
     const float* Dsk;
     float* y; long ldy;
-    int B, L, H, G;
+    int B, L, H, G;     // H counts 64-row heads: P / 64 of them per head of the call
+    int hs;             // P / 64: head h reads dt, A, dt_bias and D of h / hs
     int nchunks, nseg, chunks_per_seg;
     const float* h0;
     float* hT;
-    float* seg_state;   // (B,H,nseg,P,N)
+    float* seg_state;   // (B,H,nseg,64,N)
     float* seg_decay;   // (B,H,nseg)
     // given: the raw C B^T tiles of every (batch, group, chunk) from ssd_f32_cb_kernel,
     // (B, G, nchunks, 3 tiles, 64 lanes, 4) in accumulator order; else the full pass forms them
@@ -135,7 +136,8 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     static_assert(NCB == 3, "three tiles over four waves: one wave per chunk has no tile");
     constexpr int RL = NN / 4;           // lanes per staged B / C row (one float4 each)
     constexpr int RPP = 256 * HPW / RL;  // rows per staging pass
-    constexpr int SP = QF / RPP;         // staging passes
+    constexpr int SP = RPP < QF ? QF / RPP : 1;   // staging passes
+    constexpr bool PART = RPP > QF;      // the threads past row QF stage nothing
 
     int wg = blockIdx.x;
     if (a.remap) {
@@ -158,15 +160,17 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     const int h = h0w + hw;
     const int bh = b * a.H + h;
     const int g = h / (a.H / a.G);
+    const int hp = h / a.hs;             // head of the call
     const int l16 = lane & 15, q4 = lane >> 4;
     const int p0 = 16 * wl;
     const int sr = tid / RL, sc4 = 4 * (tid % RL);   // staging row / column
+    const unsigned s_oor = PART && sr >= QF ? 0x80000000u : 0u;
 
-    const float Ah = a.A[h] * ssm::kLog2e;
-    const float dtb = a.dt_bias ? a.dt_bias[h] : 0.f;
+    const float Ah = a.A[hp] * ssm::kLog2e;
+    const float dtb = a.dt_bias ? a.dt_bias[hp] : 0.f;
     float Dh[HPW];   // D of the workgroup's heads (the C B^T tiles serve them all)
 #pragma unroll
-    for (int k = 0; k < HPW; ++k) Dh[k] = a.Dsk ? a.Dsk[h0w + k] : 0.f;
+    for (int k = 0; k < HPW; ++k) Dh[k] = a.Dsk ? a.Dsk[(h0w + k) / a.hs] : 0.f;
     // gated output: this lane's four norm weights (columns p0 + 4 q4 .. + 3 of the head)
     float4 gw = make_float4(0.f, 0.f, 0.f, 0.f);
     if constexpr (GATED) gw = *reinterpret_cast<const float4*>(a.gn + (long)h * PF + p0 + 4 * q4);
@@ -178,7 +182,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     const float* x0 = a.x + brow * a.ldx + (long)h * PF + p0;   // wave-uniform base
     const float* b0 = a.Bm + brow * a.ldb + (long)g * NN;
     const float* cm0 = a.Cm + brow * a.ldc + (long)g * NN;
-    const float* d0 = a.dt + brow * a.lddt + h;
+    const float* d0 = a.dt + brow * a.lddt + hp;
     auto rows_of = [&](int c) { return c < c_end ? min(QF, a.L - c * QF) : 0; };
     // ssq[(b L + t) H + h] for row t of chunk c and head h0w + tid / QF from the head's four
     // waves' partial sums (threads tid < HPW QF)
@@ -240,12 +244,12 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
                 raw.x[jb][s] = bload4(rx, (unsigned)((16 * jb + 4 * q4 + s) * a.ldx + l16) * 4u);
 #pragma unroll
         for (int k = 0; k < SP; ++k)
-            raw.b[k] = bload16<float4>(rb, (unsigned)((sr + RPP * k) * a.ldb + sc4) * 4u);
+            raw.b[k] = bload16<float4>(rb, (unsigned)((sr + RPP * k) * a.ldb + sc4) * 4u | s_oor);
         if constexpr (FULL) {
             const auto rc = rsrc(cm0 + r0 * a.ldc, span(qv, a.ldc, NN));
 #pragma unroll
             for (int k = 0; k < SP; ++k)
-                raw.c[k] = bload16<float4>(rc, (unsigned)((sr + RPP * k) * a.ldc + sc4) * 4u);
+                raw.c[k] = bload16<float4>(rc, (unsigned)((sr + RPP * k) * a.ldc + sc4) * 4u | s_oor);
         }
         if constexpr (GATED) {
             // issued last: the chunk's first wait (for B and C) does not wait for them
@@ -256,23 +260,54 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
         }
     };
 
-    // entering state: S^T tile nb holds S[p0 + l16][16 nb + 4 q4 + r] in register r
+    // entering state: S^T tile nb holds S[p0 + l16][16 nb + 4 q4 + r] in register r. With
+    // NN <= 32 a segment's entering state is formed here from the local states and decays of
+    // the segments before it (a few float4 per lane from L2, loaded ahead of the chain);
+    // larger states come combined from ssd_f32_seg_prefix.
+    constexpr bool CHAIN = FULL && NN <= 32;
     const float* init = nullptr;
     if (FULL) {
-        if (a.nseg > 1) init = a.seg_state + ((long)bh * a.nseg + seg) * PF * NN;
+        if (a.nseg > 1 && !CHAIN) init = a.seg_state + ((long)bh * a.nseg + seg) * PF * NN;
         else if (a.h0) init = a.h0 + (long)bh * PF * NN;
     }
+    const long lane_off = (long)(p0 + l16) * NN + 4 * q4;
     floatx4 S[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         if (init) {
-            const float4 v = *reinterpret_cast<const float4*>(init + (long)(p0 + l16) * NN + 16 * nb + 4 * q4);
+            const float4 v = *reinterpret_cast<const float4*>(init + lane_off + 16 * nb);
             S[nb] = floatx4{v.x, v.y, v.z, v.w};
         } else {
             S[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    bool state_live = init != nullptr;
+    if constexpr (CHAIN) {
+        constexpr int GS = 8;
+        const float* ls = a.seg_state + (long)bh * a.nseg * PF * NN + lane_off;
+        const float* dc = a.seg_decay + (long)bh * a.nseg;
+        for (int s0 = 0; s0 < seg; s0 += GS) {
+            floatx4 loc[GS][NB];
+            float dec[GS];
+#pragma unroll
+            for (int j = 0; j < GS; ++j) {
+                const int sj = min(s0 + j, seg - 1);   // past seg: in range, not used
+                dec[j] = dc[sj];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    loc[j][nb] = *reinterpret_cast<const floatx4*>(ls + (long)sj * PF * NN + 16 * nb);
+            }
+#pragma unroll
+            for (int j = 0; j < GS; ++j) {
+                if (s0 + j >= seg) break;
+                const float e = ssm::ex2(dec[j]);
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) S[nb][r] = fmaf(e, S[nb][r], loc[j][nb][r]);
+            }
+        }
+    }
+    bool state_live = init != nullptr || (CHAIN && seg > 0);
     float decay_sum = 0.f;
     // dt' of chunk cc (0 past the segment), its running sum times A_h and the weights w_t into
     // LDS buffer bf (lane = time step)
@@ -336,6 +371,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
         // ---- stage B (and C) rows
 #pragma unroll
         for (int k = 0; k < SP; ++k) {
+            if (PART && sr >= QF) break;
             *reinterpret_cast<float4*>(&sm.b[buf][sr + RPP * k][sc4]) = raw.b[k];
             if constexpr (FULL) *reinterpret_cast<float4*>(&sm.c[buf][sr + RPP * k][sc4]) = raw.c[k];
         }
@@ -372,6 +408,14 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
                 const float* brw = &sm.b[buf][16 * jb + l16][4 * q4];
                 const float* crw = &sm.c[buf][16 * ib + l16][4 * q4];
                 float4 opv[2][4];
+                if constexpr (NB == 1) {
+                    const float4 o0 = *reinterpret_cast<const float4*>(brw);
+                    const float4 o1 = *reinterpret_cast<const float4*>(crw);
+                    acc0 = mfma4(o0.x, o1.x, acc0);
+                    acc1 = mfma4(o0.y, o1.y, acc1);
+                    acc0 = mfma4(o0.z, o1.z, acc0);
+                    acc1 = mfma4(o0.w, o1.w, acc1);
+                } else {
                 auto ld_pair = [&](int kk, float4* o) {
                     o[0] = *reinterpret_cast<const float4*>(brw + 16 * kk);
                     o[1] = *reinterpret_cast<const float4*>(crw + 16 * kk);
@@ -392,6 +436,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
                     acc1 = mfma4(o[2].z, o[3].z, acc1);
                     acc0 = mfma4(o[0].w, o[1].w, acc0);
                     acc1 = mfma4(o[2].w, o[3].w, acc1);
+                }
                 }
                 }
                 // acc0[r] + acc1[r] = (C B^T)[i = 16 ib + l16][j = 16 jb + 4 q4 + r] (from the
@@ -558,6 +603,7 @@ __global__ void ssd_f32_seg_prefix(F32Args a, int PN) {
 // workgroup forms causal tile t with the full pass's own MFMA sequence on the same operand
 // values (B and C rows of the chunk, zeros past L), so the tile holds the same bits, and
 // stores it in accumulator order, one float4 per lane.
+// (d_state 64 and 128; with less the tiles are a few MFMAs and the workgroups form their own.)
 template <int NN>
 __global__ __launch_bounds__(192) void ssd_f32_cb_kernel(F32Args a) {
     constexpr int NB = NN / 16;
@@ -596,13 +642,18 @@ __global__ __launch_bounds__(192) void ssd_f32_cb_kernel(F32Args a) {
     *reinterpret_cast<floatx4*>(const_cast<float*>(a.cbw) + (id * NCB + t) * 256 + 4 * lane) = sum;
 }
 
-void plan_f32(int B, int L, int H, int& nchunks, int& nseg, int& per) {
+// Chunks per segment: enough segments for kTargetWG workgroups. With d_state <= 32 a segment
+// also chains the states of all segments before it (about 0.09 us each against 1.7 us for a
+// chunk in both passes), so it gets at least sqrt(nchunks / 20) chunks.
+void plan_f32(int B, int L, int H, int N, int& nchunks, int& nseg, int& per) {
     nchunks = (int)ssm::cdiv(L, QF);
     const long bh = (long)B * H;
     long s = ssm::cdiv(kTargetWG, bh > 0 ? bh : 1);
     if (s > nchunks) s = nchunks;
     if (s < 1) s = 1;
     per = (int)ssm::cdiv(nchunks, s);
+    if (N <= 32)
+        while (20l * per * per < nchunks) ++per;
     nseg = (int)ssm::cdiv(nchunks, per);
 }
 
@@ -615,15 +666,19 @@ ssm_status launch(F32Args& a, hipStream_t st) {
         ssd_f32_kernel<NN, false><<<nwg1, 256, 0, st>>>(s1);
         ssm_status e = ssm::check_launch("ssd_f32_state_pass");
         if (e != SSM_OK) return e;
-        const long n = (long)a.B * a.H * PF * NN;
-        ssd_f32_seg_prefix<<<(unsigned)ssm::cdiv(n, 256), 256, 0, st>>>(a, PF * NN);
-        e = ssm::check_launch("ssd_f32_seg_prefix");
-        if (e != SSM_OK) return e;
+        if constexpr (NN > 32) {
+            const long n = (long)a.B * a.H * PF * NN;
+            ssd_f32_seg_prefix<<<(unsigned)ssm::cdiv(n, 256), 256, 0, st>>>(a, PF * NN);
+            e = ssm::check_launch("ssd_f32_seg_prefix");
+            if (e != SSM_OK) return e;
+        }
     }
-    if (a.cbw) {
-        ssd_f32_cb_kernel<NN><<<(unsigned)((long)a.B * a.G * a.nchunks), 192, 0, st>>>(a);
-        ssm_status e = ssm::check_launch("ssd_f32_cb");
-        if (e != SSM_OK) return e;
+    if constexpr (NN > 32) {
+        if (a.cbw) {
+            ssd_f32_cb_kernel<NN><<<(unsigned)((long)a.B * a.G * a.nchunks), 192, 0, st>>>(a);
+            ssm_status e = ssm::check_launch("ssd_f32_cb");
+            if (e != SSM_OK) return e;
+        }
     }
     // two heads per workgroup when heads 2k and 2k + 1 share a group
     const int hpw = ((a.H / a.G) % 2 == 0) ? 2 : 1;
@@ -643,13 +698,16 @@ ssm_status launch(F32Args& a, hipStream_t st) {
 
 namespace ssm {
 
-bool ssd_f32_shape(int Pd, int N) { return Pd == PF && (N == 64 || N == 128); }
+bool ssd_f32_shape(int Pd, int N) {
+    return Pd % PF == 0 && (N == 16 || N == 32 || N == 64 || N == 128);
+}
 
 // Workspace: the segment states and decays when the sequence is cut into segments, then
-// (at a 256-byte boundary) the C B^T tiles of the pre-pass, 3 KB per (batch, group, chunk).
-// A workspace without room for the tiles runs the full pass with its own tiles.
-static size_t f32_seg_bytes(int B, int H, int nseg, int Pd, int N) {
-    return nseg <= 1 ? 0 : sizeof(float) * (size_t)B * H * nseg * ((size_t)Pd * N + 1);
+// (at a 256-byte boundary, d_state 64 and 128) the C B^T tiles of the pre-pass, 3 KB per
+// (batch, group, chunk). A workspace without room for the tiles runs the full pass with its
+// own tiles. (H counts 64-row heads.)
+static size_t f32_seg_bytes(int B, int H, int nseg, int N) {
+    return nseg <= 1 ? 0 : sizeof(float) * (size_t)B * H * nseg * ((size_t)PF * N + 1);
 }
 static size_t f32_cb_off(size_t seg) { return (seg + 255) & ~(size_t)255; }
 static size_t f32_cb_bytes(int B, int G, int nchunks) {
@@ -659,17 +717,28 @@ static size_t f32_cb_bytes(int B, int G, int nchunks) {
 size_t ssd_f32_workspace(int B, int L, int H, int G, int Pd, int N) {
     if (!ssd_f32_shape(Pd, N) || B <= 0 || L <= 0 || H <= 0 || G <= 0) return 0;
     int nchunks, nseg, per;
-    plan_f32(B, L, H, nchunks, nseg, per);
-    return f32_cb_off(f32_seg_bytes(B, H, nseg, Pd, N)) + f32_cb_bytes(B, G, nchunks);
+    H *= Pd / PF;
+    plan_f32(B, L, H, N, nchunks, nseg, per);
+    const size_t seg = f32_seg_bytes(B, H, nseg, N);
+    return N > 32 ? f32_cb_off(seg) + f32_cb_bytes(B, G, nchunks) : seg;
+}
+
+size_t ssd_f32_least_workspace(int B, int L, int H, int Pd, int N) {
+    int nchunks, nseg, per;
+    H *= Pd / PF;
+    plan_f32(B, L, H, N, nchunks, nseg, per);
+    return f32_seg_bytes(B, H, nseg, N);
 }
 
 ssm_status ssd_f32(const float* x, long ldx, const float* dt, long lddt, const float* dt_bias,
                    int softplus, float dt_min, float dt_max, const float* A, const float* Bm,
                    long ldb, const float* Cm, long ldc, const float* Dsk, float* y, long ldy,
-                   int B, int L, int H, int G, int N, const float* h0, float* hT,
+                   int B, int L, int H, int Pd, int G, int N, const float* h0, float* hT,
                    void* workspace, size_t workspace_bytes, hipStream_t st, const float* z,
                    long ldz, const float* gn, float* ssq) {
     F32Args a{};
+    a.hs = Pd / PF;
+    H *= a.hs;
     a.z = z; a.ldz = ldz; a.gn = gn; a.ssq = ssq;
     if (ssq) {
         SSM_REQUIRE(z && gn && ldz >= (long)H * PF, "ssd_f32: the gated output needs z and gn");
@@ -681,20 +750,25 @@ ssm_status ssd_f32(const float* x, long ldx, const float* dt, long lddt, const f
     a.dt_min = dt_min; a.dt_max = dt_max; a.A = A; a.Bm = Bm; a.ldb = ldb; a.Cm = Cm;
     a.ldc = ldc; a.Dsk = Dsk; a.y = y; a.ldy = ldy; a.B = B; a.L = L; a.H = H; a.G = G;
     a.h0 = h0; a.hT = hT;
-    plan_f32(B, L, H, a.nchunks, a.nseg, a.chunks_per_seg);
-    const size_t seg = f32_seg_bytes(B, H, a.nseg, PF, N);
+    plan_f32(B, L, H, N, a.nchunks, a.nseg, a.chunks_per_seg);
+    const size_t seg = f32_seg_bytes(B, H, a.nseg, N);
     if (a.nseg > 1) {
         SSM_REQUIRE(workspace && workspace_bytes >= seg,
                     "ssm_ssd_chunk_scan: workspace of %zu bytes needed",
-                    ssd_f32_workspace(B, L, H, G, PF, N));
+                    ssd_f32_workspace(B, L, H / a.hs, G, Pd, N));
         a.seg_state = (float*)workspace;
         a.seg_decay = a.seg_state + (size_t)B * H * a.nseg * PF * N;
     }
     const size_t cbo = f32_cb_off(seg);
-    if (workspace && ((uintptr_t)workspace & 15) == 0 &&
+    if (N > 32 && workspace && ((uintptr_t)workspace & 15) == 0 &&
         workspace_bytes >= cbo + f32_cb_bytes(B, G, a.nchunks))
         a.cbw = (const float*)((char*)workspace + cbo);
-    return N == 128 ? launch<128>(a, st) : launch<64>(a, st);
+    switch (N) {
+        case 128: return launch<128>(a, st);
+        case 64: return launch<64>(a, st);
+        case 32: return launch<32>(a, st);
+        default: return launch<16>(a, st);
+    }
 }
 
 }  // namespace ssm
