@@ -1,5 +1,6 @@
 // K2: Mamba-1 selective scan (Gu & Dao 2023, Algorithm 2) for gfx950, and its one-token
-// decode update. Two designs, chosen by how many waves the channels alone give:
+// decode update. Three designs, chosen by how many waves the channels alone give and the length
+// (few channels and up to 1024 steps of 16 states: the time slices, scan_t16_kernel, below):
 //
 // Single pass (scan_single_kernel, when B * D * N / 64 waves give every SIMD one): lane
 // (c, n) holds state h[d, n] in a register and walks the whole sequence once; the inputs of
@@ -14,13 +15,13 @@
 // wave-uniform and the pointers are read-only restrict parameters, so they are fetched with
 // scalar loads into SGPRs. Time is cut into NC chunks so that B*D/64*NC waves fill the chip:
 //   pass A  scan_chunk_state : each chunk from a zero state -> chunk-end state + sum(dt')
-//   pass B  scan_chunk_prefix: per (b,n,d) sequential combine over chunks -> state entering
-//                               each chunk (h_in[c] = exp(A*sum_dt[c-1]) h_in[c-1] + hend[c-1]),
-//                               final state
+//   pass B  scan_chunk_prefix: per (b,n,d) combine over chunks -> state entering each chunk
+//                               (h_in[c] = exp(A*sum_dt[c-1]) h_in[c-1] + hend[c-1]), final state
 //   pass C  scan_chunk_output: re-run each chunk from its entering state, emit y with the D
 //                               skip and SiLU(z) gate.
 // exp(dt A) is exp2(dt * (A log2 e)) with A pre-scaled once per lane (one v_exp_f32 each).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "glue.hpp"
@@ -111,40 +112,64 @@ __global__ __launch_bounds__(kWave) void scan_chunk_state(
     sdt_out[((long)b * NC + c) * D + d] = sdt;
 }
 
-// One thread per (b, n, d); d fastest so the chunk-state rows are read coalesced.
-__global__ void scan_chunk_prefix(const float* __restrict__ A, int L, int D, int N, int NC,
-                                  long total, float* __restrict__ hc,
-                                  const float* __restrict__ sdt, const float* __restrict__ h0,
-                                  float* __restrict__ hT) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const int d = (int)(i % D);
-    const int n = (int)((i / D) % N);
-    const int b = (int)(i / ((long)D * N));
-    const float A2 = A[(long)d * N + n] * ssm::kLog2e;
-    float carry = h0 ? h0[((long)b * D + d) * N + n] : 0.f;
-    // the chunk-end states and dt sums of kPre chunks are loaded before the carry chain
-    // consumes them (the chain itself has no memory latency in it)
-    constexpr int kPre = 8;
+// Entering states of the chunks, in place of their end states. Workgroup (channels 64 x .. + 63,
+// state n, sequence b), lane = channel (chunk-state rows are read coalesced); wave w takes chunks
+// kPer w .. of a round of kPer kPreW chunks: all its loads at once, its chunks composed to one
+// (decay, state) pair, the pairs exchanged through LDS, then its chunks' entering states. (One
+// thread per (b, n, d) walking all chunks, 8 loads at a time, waited 16 memory latencies for 128
+// chunks: 16.5 us for 1536 channels x 16 states; the whole scan went 49.1 -> 40.2 us, and 46.5 ->
+// 23.7 for 256 channels x 4096 steps.) No branch leaves the unrolled loops, so the values stay
+// in registers.
+template <int kPreW, int kPer>
+__global__ __launch_bounds__(64 * kPreW) void scan_chunk_prefix(
+    const float* __restrict__ A, int D, int N, int NC, float* __restrict__ hc,
+    const float* __restrict__ sdt, const float* __restrict__ h0, float* __restrict__ hT) {
+    __shared__ float2 seg[2][kPreW][64];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int d = blockIdx.x * 64 + lane, n = blockIdx.y, b = blockIdx.z;
+    const bool ok = d < D;
+    const int dc = ok ? d : D - 1;
+    const float A2 = A[(long)dc * N + n] * ssm::kLog2e;
+    float carry = h0 ? h0[((long)b * D + dc) * N + n] : 0.f;
     const long cstride = (long)N * D;
-    float* p0 = hc + ((long)b * NC * N + n) * D + d;
-    const float* s0 = sdt + (long)b * NC * D + d;
-    for (int c0 = 0; c0 < NC; c0 += kPre) {
-        float he[kPre], sd[kPre];
+    float* p0 = hc + ((long)b * NC * N + n) * D + dc;
+    const float* s0 = sdt + (long)b * NC * D + dc;
+    int buf = 0;
+    for (int r0 = 0; r0 < NC; r0 += kPer * kPreW, buf ^= 1) {
+        const int c0 = r0 + w * kPer;
+        float he[kPer], av[kPer];
 #pragma unroll
-        for (int u = 0; u < kPre; ++u) {
-            const bool live = c0 + u < NC;
-            he[u] = live ? p0[(long)(c0 + u) * cstride] : 0.f;
-            sd[u] = live ? s0[(long)(c0 + u) * D] : 0.f;
+        for (int u = 0; u < kPer; ++u) {
+            const int cc = min(c0 + u, NC - 1);
+            he[u] = p0[(long)cc * cstride];
+            av[u] = s0[(long)cc * D];
+        }
+        float P = 1.f, H = 0.f;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const bool live = c0 + u < NC;       // (uniform; chunks past the last keep the state)
+            av[u] = live ? ssm::ex2(A2 * av[u]) : 1.f;
+            he[u] = live ? he[u] : 0.f;
+            H = fmaf(av[u], H, he[u]);
+            P *= av[u];
+        }
+        seg[buf][w][lane] = make_float2(P, H);
+        __syncthreads();   // (also: every wave's loads of the round are done before its stores)
+        float e = carry;
+#pragma unroll
+        for (int v = 0; v < kPreW; ++v) {
+            const float2 g = seg[buf][v][lane];
+            e = v == w ? carry : e;
+            carry = fmaf(g.x, carry, g.y);
         }
 #pragma unroll
-        for (int u = 0; u < kPre; ++u) {
-            if (c0 + u >= NC) break;
-            p0[(long)(c0 + u) * cstride] = carry;
-            carry = fmaf(ssm::ex2(A2 * sd[u]), carry, he[u]);
+        for (int u = 0; u < kPer; ++u) {
+            if (ok && c0 + u < NC) p0[(long)(c0 + u) * cstride] = e;
+            e = fmaf(av[u], e, he[u]);
         }
     }
-    if (hT) hT[((long)b * D + d) * N + n] = carry;
+    if (hT && ok && w == 0) hT[((long)b * D + d) * N + n] = carry;
 }
 
 template <int N, bool EXACT>
@@ -244,9 +269,16 @@ void launch_all(const ScanArgs& a, hipStream_t st) {
     scan_chunk_state<N, EXACT><<<grid, kWave, 0, st>>>(a.u, a.ldu, a.dt, a.lddt, a.dt_bias, a.softplus,
                                                 a.A, a.Bm, a.ldb, a.L, a.D, a.N, a.T, a.NC, a.hc,
                                                 a.sdt);
-    const long nthr = (long)a.B * a.N * a.D;
-    scan_chunk_prefix<<<(unsigned)ssm::cdiv(nthr, 256), 256, 0, st>>>(
-        a.A, a.L, a.D, a.N, a.NC, nthr, a.hc, a.sdt, a.h0, a.hT);
+    const dim3 pgrid((unsigned)ssm::cdiv(a.D, 64), (unsigned)a.N, (unsigned)a.B);
+    auto prefix = [&](auto waves, auto per) {   // the fewest waves that take all chunks at once
+        scan_chunk_prefix<waves, per><<<pgrid, 64 * waves, 0, st>>>(a.A, a.D, a.N, a.NC, a.hc,
+                                                                    a.sdt, a.h0, a.hT);
+    };
+    using std::integral_constant;
+    if (a.NC <= 16) prefix(integral_constant<int, 2>(), integral_constant<int, 8>());
+    else if (a.NC <= 32) prefix(integral_constant<int, 4>(), integral_constant<int, 8>());
+    else if (a.NC <= 64) prefix(integral_constant<int, 8>(), integral_constant<int, 8>());
+    else prefix(integral_constant<int, 8>(), integral_constant<int, 16>());
     scan_chunk_output<N, EXACT><<<grid, kWave, 0, st>>>(a.u, a.ldu, a.dt, a.lddt, a.dt_bias,
                                                  a.softplus, a.A, a.Bm, a.ldb, a.Cm, a.ldc,
                                                  a.Dsk, a.z, a.ldz, a.y, a.ldy, a.L, a.D, a.N,
@@ -706,6 +738,212 @@ void launch_w16(const ScanArgs& a, hipStream_t st) {
     scan_w16_kernel<W><<<(unsigned)nwg, 64 * W, 0, st>>>(a);
 }
 
+// ---------------------------------------------------------------- time slices, N = 16
+// The scan of a few channels: a workgroup owns 4 channels of one sequence and its W waves take
+// consecutive slices of 16 steps, so a block of 16 W steps is walked by all waves at once (the
+// single pass above has one wave walk every step: 22 workgroups and 17 us for 512 channels over
+// 256 steps). Lane (c, n) holds state n of channel c.
+//   inputs   lane (c, t) loads u, dt, z of step t of the wave's slice (one block ahead) and
+//            forms dt' and dt' u once; B and C of the slice go through the wave's own LDS tile;
+//   walk     from a zero state: a_t = exp2(dt'_t A log2 e), h_t = a_t h_{t-1} + dt'_t u_t B_t[n]
+//            with dt' and dt' u taken from lane t of the channel's row (row_newbcast inside the
+//            multiplies); the 16 a_t and h_t stay in registers;
+//   combine  the slice's end state and decay exp2(A log2 e sum dt') go to LDS; after the block's
+//            barrier every wave chains the pairs of the slices before its own onto the state
+//            entering the block: the state q entering its slice. The last wave leaves the next
+//            block's entering state;
+//   output   y_t = sum_n C_t[n] (h_t + a_1 .. a_t q): the kept a_t are multiplied up, no second
+//            exp. The 16 sums over n are formed in four exchange steps (row mirror, half mirror,
+//            quad permutes) that halve the steps each lane carries: lane (c, t) ends with y_t,
+//            whose u, z it holds.
+// exp(dt' A) is evaluated once per element, and there is one barrier per block. Bound by vector
+// issue: about 230 vector instructions per slice and wave, 19 of them exp (1150 cycles; 1600
+// measured with three waves per SIMD). Measured on MI355X, single or chunked passes -> this (us):
+// 512 channels x 256 steps 15.7 -> 5.6, 1024 x 200 15.9 -> 5.4, 1536 x 512 22.8 -> 13.6, two
+// sequences of 1536 x 1000 42.4 -> 32.7.
+template <int W>
+struct ScanT16 {
+    static constexpr int TB = 16 * W;    // steps per block
+    static constexpr int PT = 20;        // [n][t] pitch of a wave's B and C tiles
+    struct Smem {
+        float bt[W][16][PT], ct[W][16][PT];
+        float2 end[2][W][64];            // (end state, decay) per slice
+        float cin[2][64];                // state entering the block
+    };
+};
+
+// Values v[t] of 16 steps in each lane of a 16-lane row -> their sums over the row, the sum of
+// step t in lane t.
+__device__ __forceinline__ float row_reduce16(float (&v)[16], int j) {
+    const bool b3 = (j & 8) != 0, b2 = (j & 4) != 0, b1 = (j & 2) != 0, b0 = (j & 1) != 0;
+    auto dpp = [](float x, auto ctrl) {
+        return __int_as_float(
+            __builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    float r8[8], r4[4], r2[2];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {       // lanes i and 15 - i
+        const float keep = b3 ? v[8 + i] : v[i], send = b3 ? v[i] : v[8 + i];
+        r8[i] = keep + dpp(send, std::integral_constant<int, 0x140>());
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {       // lanes i and 7 - i of each half
+        const float keep = b2 ? r8[4 + i] : r8[i], send = b2 ? r8[i] : r8[4 + i];
+        r4[i] = keep + dpp(send, std::integral_constant<int, 0x141>());
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {       // lanes i ^ 2
+        const float keep = b1 ? r4[2 + i] : r4[i], send = b1 ? r4[i] : r4[2 + i];
+        r2[i] = keep + dpp(send, std::integral_constant<int, 0x4E>());
+    }
+    const float keep = b0 ? r2[1] : r2[0], send = b0 ? r2[0] : r2[1];
+    return keep + dpp(send, std::integral_constant<int, 0xB1>());
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) void scan_t16_kernel(ScanArgs a) {
+    using S = ScanT16<W>;
+    constexpr int TB = S::TB;
+    __shared__ __attribute__((aligned(16))) typename S::Smem sm;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane >> 4, j = lane & 15;
+    const int D = a.D, L = a.L;
+    // contiguous channel groups per XCD: the groups that share a row's lines share an L2
+    const int nwg = (int)gridDim.x, nb = (D + 3) / 4;
+    const int xcd = blockIdx.x % 8, q8 = nwg / 8, rem = nwg % 8;
+    const int tile = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + blockIdx.x / 8;
+    const int b = tile / nb, d = (tile % nb) * 4 + c;
+    const bool dok = d < D;
+    const int dc = dok ? d : D - 1;
+    const unsigned dmask = dok ? 0u : 0x80000000u;   // a channel past D reads and stores nothing
+    const float A2 = a.A[(long)dc * 16 + j] * ssm::kLog2e;
+    const float bias = a.dt_bias ? a.dt_bias[dc] : 0.f;
+    const float Dd = a.Dsk ? a.Dsk[dc] : 0.f;
+    if (w == 0) sm.cin[0][lane] = (dok && a.h0) ? a.h0[((long)b * D + d) * 16 + j] : 0.f;
+
+    // Rows k TB .. of sequence b: a base that advances a block at a time and the block's bytes
+    // (32-bit offsets however long the sequence); rows past L read zeros, take no stores.
+    struct Span {
+        const char* base;
+        long step;
+        int ld, width;
+    };
+    auto span = [&](const float* p, long ld, int width) {
+        return Span{(const char*)(p + (long)b * L * ld), (long)TB * ld * 4, (int)ld, width};
+    };
+    auto blk = [&](const Span& s, int rows) {   // rows: left in the sequence from this block on
+        const int n = min(rows, TB);
+        return ssm::rsrc(s.base, n > 0 ? (unsigned)((n - 1) * s.ld + s.width) * 4u : 0u);
+    };
+    Span su = span(a.u, a.ldu, D), sd = span(a.dt, a.lddt, D),
+         sz = span(a.z ? a.z : a.u, a.z ? a.ldz : 0, a.z ? D : 0), sb = span(a.Bm, a.ldb, 16),
+         sc = span(a.Cm, a.ldc, 16), sy = span(a.y, a.ldy, D);
+    const unsigned t = 16u * w + j;      // this lane's step within a block, as an input lane
+    const unsigned tb = 16u * w + c;     // B / C: lane (c, n) loads steps 4 i + c of the slice
+    const unsigned du_ = (unsigned)d * 4u;
+    const unsigned ou = (t * (unsigned)a.ldu * 4u + du_) | dmask,
+                   od = (t * (unsigned)a.lddt * 4u + du_) | dmask,
+                   oz = (t * (unsigned)sz.ld * 4u + du_) | dmask,
+                   oy = (t * (unsigned)a.ldy * 4u + du_) | dmask;
+    unsigned ob[4], oc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        ob[i] = ((tb + 4u * i) * (unsigned)a.ldb + (unsigned)j) * 4u;
+        oc[i] = ((tb + 4u * i) * (unsigned)a.ldc + (unsigned)j) * 4u;
+    }
+    float uv, dv, zv, bv[4], cv[4];
+    auto load = [&](int rows) {          // the block at the spans' bases, which then advance
+        const auto ru = blk(su, rows), rd = blk(sd, rows), rz = blk(sz, a.z ? rows : 0),
+                   rb = blk(sb, rows), rc = blk(sc, rows);
+        uv = ssm::bload4(ru, ou);
+        dv = ssm::bload4(rd, od);
+        zv = ssm::bload4(rz, oz);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            bv[i] = ssm::bload4(rb, ob[i]);
+            cv[i] = ssm::bload4(rc, oc[i]);
+        }
+        su.base += su.step; sd.base += sd.step; sz.base += sz.step; sb.base += sb.step;
+        sc.base += sc.step;
+    };
+    load(L);
+    int buf = 0;
+    for (int rows = L; rows > 0; rows -= TB, buf ^= 1) {
+        const float un = uv, zn = zv;
+        float dl = dv + bias;
+        if (a.softplus) dl = ssm::softplus_sel(dl);
+        dl = (int)t < rows ? dl : 0.f;            // past L: dt' = 0, the state is kept
+        const float du = dl * un;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            sm.bt[w][j][4 * i + c] = bv[i];
+            sm.ct[w][j][4 * i + c] = cv[i];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the wave's own tiles
+        load(rows - TB);                           // past the last block: zeros, not used
+        float bq[16], cq[16];
+#pragma unroll
+        for (int q = 0; q < 16; q += 4) {
+            const float4 b4 = *reinterpret_cast<const float4*>(&sm.bt[w][j][q]);
+            const float4 c4 = *reinterpret_cast<const float4*>(&sm.ct[w][j][q]);
+            bq[q] = b4.x; bq[q + 1] = b4.y; bq[q + 2] = b4.z; bq[q + 3] = b4.w;
+            cq[q] = c4.x; cq[q + 1] = c4.y; cq[q + 2] = c4.z; cq[q + 3] = c4.w;
+        }
+        float at[16], hs[16];
+        float h = 0.f;
+#define SCANT_STEP(J)                                     \
+        at[J] = ssm::ex2(row_bcast<J>(dl) * A2);          \
+        h = fmaf(at[J], h, row_bcast<J>(du) * bq[J]);     \
+        hs[J] = h;
+        SCANT_STEP(0) SCANT_STEP(1) SCANT_STEP(2) SCANT_STEP(3)
+        SCANT_STEP(4) SCANT_STEP(5) SCANT_STEP(6) SCANT_STEP(7)
+        SCANT_STEP(8) SCANT_STEP(9) SCANT_STEP(10) SCANT_STEP(11)
+        SCANT_STEP(12) SCANT_STEP(13) SCANT_STEP(14) SCANT_STEP(15)
+#undef SCANT_STEP
+        // sum of dt' over the row (xor 1, 2, 7, 15 exchanges), in every lane
+        float sdt = dl + quad_xor<1>(dl);
+        sdt += quad_xor<2>(sdt);
+        sdt += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sdt), 0x141, 0xF, 0xF, true));
+        sdt += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sdt), 0x140, 0xF, 0xF, true));
+        const float P = ssm::ex2(sdt * A2);
+        sm.end[buf][w][lane] = make_float2(h, P);
+        __syncthreads();
+        float q = sm.cin[buf][lane];
+#pragma unroll
+        for (int v = 0; v < W - 1; ++v) {
+            if (v >= w) break;           // (uniform)
+            const float2 e = sm.end[buf][v][lane];
+            q = fmaf(e.y, q, e.x);
+        }
+        if (w == W - 1) {
+            const float out = fmaf(P, q, h);
+            sm.cin[buf ^ 1][lane] = out;
+            if (rows <= TB && dok && a.hT) a.hT[((long)b * D + d) * 16 + j] = out;
+        }
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            q *= at[s];
+            hs[s] = cq[s] * (hs[s] + q);
+        }
+        float y = fmaf(Dd, un, row_reduce16(hs, j));
+        if (a.z) y *= a.zgated ? zn : ssm::silu_fast(zn);
+        ssm::bstore4(y, blk(sy, rows), oy);
+        sy.base += sy.step;
+    }
+}
+
+// Waves per workgroup: as many slices as the sequence has, up to 16 while each workgroup has a
+// CU to itself; with more workgroups than CUs smaller ones interleave their phases (us, W = 4 /
+// 8 / 16): 64 steps x 512 channels 3.4 / 4.0 / 4.9; 4096 x 256 61.6 / 54.0 / 39.6; 2047 x 1536
+// 45.1 / 44.3 / 46.9; 2 sequences of 1000 x 1536 32.7 / 35.9 / 38.3.
+void launch_t16(const ScanArgs& a, hipStream_t st) {
+    const long nwg = ssm::cdiv(a.D, 4) * a.B;
+    if (a.L <= 64 || nwg > 512) scan_t16_kernel<4><<<(unsigned)nwg, 256, 0, st>>>(a);
+    else if (a.L <= 128 || nwg > 256) scan_t16_kernel<8><<<(unsigned)nwg, 512, 0, st>>>(a);
+    else scan_t16_kernel<16><<<(unsigned)nwg, 1024, 0, st>>>(a);
+}
+
 template <int N, bool EXACT>
 void launch_single(const ScanArgs& a, hipStream_t st) {
     using S = Scan1<N>;
@@ -733,6 +971,14 @@ bool single_ok(int B, int D, int Np) {
 // for one sequence of 1536 channels at 16 to 200 steps, measured).
 constexpr int kShortL = 256;
 bool use_single(int B, int L, int D, int Np) { return L <= kShortL || single_ok(B, D, Np); }
+// N = 16 with fewer channels than the single pass needs: the time-sliced walk up to kSliceL
+// steps. Longer sequences give the chunked passes enough chunks to fill the chip with coalesced
+// 64-channel waves (us, slices / chunks: 512 steps x 1536 channels 13.6 / 22.3, 2 x 1000 x 1536
+// 33.0 / 41.8, 3 x 777 x 1024 26.5 / 40.8, 2047 x 1536 44.5 / 40.2, 4096 x 256 39.8 / 23.7).
+constexpr int kSliceL = 1024;
+bool use_t16(int B, int L, int D, int N) {
+    return N == 16 && !single_ok(B, D, 16) && L <= kSliceL;
+}
 
 // One-token update: one thread per (b, d) with the N state entries in registers. ykb > 0:
 // y goes to fragment order with K = D = 16 ykb (the input of the fused step's out_proj).
@@ -1024,7 +1270,8 @@ size_t chunked_workspace(int B, int L, int D, int N) {
 
 extern "C" size_t ssm_selective_scan_workspace(int B, int L, int D, int N) {
     if (B <= 0 || L <= 0 || D <= 0 || N <= 0 || N > 64) return 0;
-    if (use_single(B, L, D, pad_n(N))) return 0;   // the single pass needs none
+    // the single pass and the time-sliced walk need none
+    if (use_single(B, L, D, pad_n(N)) || use_t16(B, L, D, N)) return 0;
     return chunked_workspace(B, L, D, N);
 }
 
@@ -1056,11 +1303,13 @@ ssm_status selective_scan(const float* u, long ldu, const float* dt, long lddt,
     }
     const int Np = pad_n(N);
     const long ldmax = std::max({ldu, lddt, ldy, z ? ldz : 0L, ldb, ldc});
+    const bool t16 = use_t16(B, L, D, N);
     const bool single = use_single(B, L, D, Np);
-    const long rows = single ? std::min<long>(L, 128) : pick_chunk(B, L, D);
+    const long rows = t16 ? std::min<long>(L, 256) : single ? std::min<long>(L, 128)
+                                                            : pick_chunk(B, L, D);
     SSM_REQUIRE(rows_fit(rows, ldmax, D),
                 "ssm_selective_scan: row stride %ld too large for 32-bit block offsets", ldmax);
-    const size_t need = single ? 0 : chunked_workspace(B, L, D, N);
+    const size_t need = t16 || single ? 0 : chunked_workspace(B, L, D, N);
     SSM_REQUIRE(need == 0 || (workspace && workspace_bytes >= need),
                 "ssm_selective_scan: workspace of %zu bytes needed", need);
     ScanArgs a;
@@ -1074,6 +1323,10 @@ ssm_status selective_scan(const float* u, long ldu, const float* dt, long lddt,
     a.sdt = a.hc + (size_t)B * a.NC * N * D;
     a.h0 = h0; a.hT = hT;
     hipStream_t st = (hipStream_t)stream;
+    if (t16) {
+        launch_t16(a, st);
+        return ssm::check_launch("selective_scan");
+    }
     if (single) {
         const bool exact = N == Np;
         switch (Np) {

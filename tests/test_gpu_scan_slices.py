@@ -1,0 +1,56 @@
+"""The time-sliced Mamba-1 scan (16 states, few channels) against the oracle at the edges of its
+slices (16 steps), blocks (64, 128, 256 steps) and channel groups (4), over every option it
+takes; 1e-4 relative plus 2e-6 of the largest magnitude (fp32 sums of 16 terms, products of up
+to 16 decays)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+from oracle import oracle as O  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def close(got, ref, what):
+    got, ref = got.cpu().numpy().astype(np.float64), np.asarray(ref, np.float64)
+    ratio = float((np.abs(got - ref) / (1e-4 * np.abs(ref) + 2e-6 * np.abs(ref).max())).max())
+    print(f"  {what}: worst |err|/bound {ratio:.3f}", flush=True)
+    assert np.isfinite(got).all() and ratio <= 1.0
+
+
+@pytest.mark.parametrize("B,L,D", [
+    (1, 1, 1), (2, 16, 4), (1, 17, 6),            # one slice, one step of the next, partial group
+    (1, 64, 100), (1, 65, 100), (3, 128, 33),     # 4-wave blocks, the first 8-wave length
+    (1, 129, 64), (1, 256, 512), (2, 300, 130),   # 16-wave blocks
+    (1, 1000, 1030),                              # 8-wave blocks, tail slice of 8 steps
+    (2, 333, 1500),                               # more than 512 groups: 4-wave blocks
+])
+@pytest.mark.parametrize("opts", ["all", "none"])
+def test_matches_oracle(B, L, D, opts):
+    """"all": entering and final state, gate, skip, dt bias, softplus, strided inputs; "none": raw
+    dt and nothing else."""
+    print(f"[case] scan slices B={B} L={L} D={D} {opts}", flush=True)
+    from ssmjs_amd import kernels
+    r = np.random.default_rng(L * D)
+    f = lambda *s: r.standard_normal(s).astype(np.float32)   # noqa: E731
+    u, z, Bm, Cm, Dk, bias = f(B, L, D), f(B, L, D), f(B, L, 16), f(B, L, 16), f(D), f(D) - 1
+    dt = f(B, L, D) - 1
+    A = -r.uniform(0.5, 16, (D, 16)).astype(np.float32)
+    h0 = f(B, D, 16)
+    dev = lambda a: torch.from_numpy(a).cuda()   # noqa: E731
+    if opts == "all":
+        wide = torch.zeros(B, L, D + 40, device="cuda")
+        wide[:, :, :D], wide[:, :, D:D + 16], wide[:, :, D + 20:D + 36] = dev(u), dev(Bm), dev(Cm)
+        hT = torch.empty(B, D, 16, device="cuda")
+        y = kernels.selective_scan(wide[:, :, :D], dev(dt), dev(A), wide[:, :, D:D + 16],
+                                   wide[:, :, D + 20:D + 36], dev(Dk), dev(z), dev(bias), True,
+                                   h0=dev(h0), hT=hT)
+        torch.cuda.synchronize()
+        ref, ref_h = O.selective_scan(u, dt, A, Bm, Cm, Dk, z, bias, True, h0=h0, return_state=True)
+        close(hT, ref_h, "final state")
+    else:
+        dt = np.abs(dt) * 0.1
+        y = kernels.selective_scan(dev(u), dev(dt), dev(A), dev(Bm), dev(Cm), softplus=False)
+        torch.cuda.synchronize()
+        ref = O.selective_scan(u, dt, A, Bm, Cm, None, None, None, False)
+    close(y, ref, "y")
