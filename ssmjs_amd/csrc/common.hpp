@@ -65,6 +65,15 @@ __device__ __forceinline__ float softplus_fast(float x) {
     return x < -8.f ? e : __logf(1.f + e);
 }
 
+// softplus_fast without the rounding of 1 + e^x: with w = fl(1 + e^x), log1p(e^x) = log w + (e^x -
+// (w - 1)) / w to first order (w - 1 is exact); the relative error at x = -3 falls from 1e-6 to
+// 1e-7.
+__device__ __forceinline__ float softplus_corr(float x) {
+    if (x > 20.f) return x;
+    const float e = __expf(x), w = 1.f + e;
+    return x < -8.f ? e - 0.5f * e * e : fmaf(e - (w - 1.f), __builtin_amdgcn_rcpf(w), __logf(w));
+}
+
 // z * sigmoid(z) with v_exp_f32 and v_rcp_f32 (about 1 ulp each).
 __device__ __forceinline__ float silu_fast(float z) {
     return z * __builtin_amdgcn_rcpf(1.f + __expf(-z));

@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     auto scan_put = [&](int cc, float raw_dt, int bf) {
         const int qv = rows_of(cc);
         float dv = raw_dt + dtb;
-        if (a.softplus) dv = ssm::softplus_fast(dv);
+        if (a.softplus) dv = NN <= 32 ? ssm::softplus_corr(dv) : ssm::softplus_fast(dv);
         dv = lane < qv ? fminf(fmaxf(dv, a.dt_min), a.dt_max) : 0.f;
         const float sc = wave_prefix_sum(dv * Ah);
         const float ae = __builtin_bit_cast(
@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
         float acend = 0.f;
         if constexpr (!FULL) {
             float dv = raw.dt + dtb;
-            if (a.softplus) dv = ssm::softplus_fast(dv);
+            if (a.softplus) dv = NN <= 32 ? ssm::softplus_corr(dv) : ssm::softplus_fast(dv);
             dv = lane < qv ? fminf(fmaxf(dv, a.dt_min), a.dt_max) : 0.f;
             const float sc = wave_prefix_sum(dv * Ah);
             acend = __builtin_bit_cast(
