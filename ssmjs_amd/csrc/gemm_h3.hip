@@ -59,7 +59,9 @@ struct PackArgs {
     int* ex;     // per row: the power of two that undoes the scaling
 };
 
-template <int KW>
+// STEP: the order of k of the one-token step's operand (stepproj.hip: lane (q, i) holds k = 4 q ..
+// + 3 of the block's first 16, then of its second 16). VEC: 16-byte loads (rows 16-byte aligned).
+template <int KW, bool STEP, bool VEC>
 __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     __shared__ unsigned red[8][16];
     const int lane = threadIdx.x & 63;
@@ -79,9 +81,15 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
         for (int u = 0; u < KW; ++u)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int k = (kb0 + 8 * u) * kKB + 8 * q + 4 * h;
-                const unsigned oor = k < a.K ? row_oor : 0x80000000u;
-                v[u][h] = ssm::bload16<floatx4>(rx, (base + (unsigned)k * 4u) | oor);
+                const int k = (kb0 + 8 * u) * kKB + (STEP ? 16 * h + 4 * q : 8 * q + 4 * h);
+                const unsigned oor = k < a.K ? row_oor : 0x80000000u;   // (K % 4 == 0)
+                const unsigned o = base + (unsigned)k * 4u;
+                if constexpr (VEC) {
+                    v[u][h] = ssm::bload16<floatx4>(rx, o | oor);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[u][h][e] = ssm::bload4(rx, (o + 4u * e) | oor);
+                }
             }
     };
     auto maxima = [&]() {
@@ -491,20 +499,37 @@ size_t h3_split_floats(int M, int N, int K) {
     return p.ks > 1 ? (size_t)p.ks * M * N : 0;
 }
 
+template <bool STEP, bool VEC>
+static ssm_status launch_pack(const PackArgs& a, hipStream_t st) {
+    const unsigned grid = (unsigned)cdiv(a.R, 16);
+    if (a.KB <= 16) pack_h3_kernel<2, STEP, VEC><<<grid, 512, 0, st>>>(a);
+    else if (a.KB <= 32) pack_h3_kernel<4, STEP, VEC><<<grid, 512, 0, st>>>(a);
+    else if (a.KB <= 64) pack_h3_kernel<8, STEP, VEC><<<grid, 512, 0, st>>>(a);
+    else pack_h3_kernel<16, STEP, VEC><<<grid, 512, 0, st>>>(a);
+    return check_launch("pack_h3");
+}
+
 ssm_status launch_pack_h3(const float* X, long ldx, int rows, int K, void* packed,
                           hipStream_t st) {
     SSM_REQUIRE(X && packed && rows > 0 && K > 0 && K % 4 == 0 && ldx >= K && ldx % 4 == 0 &&
                     ((uintptr_t)X & 15) == 0 && ((uintptr_t)packed & 15) == 0 &&
                     16 * ldx * 4 < (1L << 31),
                 "pack_h3: arguments");
-    PackArgs a{X, ldx, rows, K, (int)cdiv(K, kKB), (char*)packed,
-               (int*)((char*)packed + h3_ex_off(rows, K))};
-    const unsigned grid = (unsigned)cdiv(rows, 16);
-    if (a.KB <= 16) pack_h3_kernel<2><<<grid, 512, 0, st>>>(a);
-    else if (a.KB <= 32) pack_h3_kernel<4><<<grid, 512, 0, st>>>(a);
-    else if (a.KB <= 64) pack_h3_kernel<8><<<grid, 512, 0, st>>>(a);
-    else pack_h3_kernel<16><<<grid, 512, 0, st>>>(a);
-    return check_launch("pack_h3");
+    const PackArgs a{X, ldx, rows, K, (int)cdiv(K, kKB), (char*)packed,
+                     (int*)((char*)packed + h3_ex_off(rows, K))};
+    return launch_pack<false, true>(a, st);
+}
+
+// The step projection's weights (a layer's weights may start at any float offset).
+size_t step_ex_off(int rows, int K) { return h3_ex_off(rows, K) / sizeof(float); }
+size_t step_w_floats(int rows, int K) { return h3_bytes(rows, K) / sizeof(float); }
+ssm_status launch_pack_step(const float* W, long ldw, int N, int K, float* out, hipStream_t st) {
+    SSM_REQUIRE(W && out && N >= 1 && K % 16 == 0 && ldw >= K && ((uintptr_t)out & 15) == 0 &&
+                    16 * ldw * 4 < (1L << 31),
+                "pack_step: K %d / ldw %ld / alignment", K, ldw);
+    const PackArgs a{W, ldw, N, K, (int)cdiv(K, kKB), (char*)out, (int*)(out + step_ex_off(N, K))};
+    return ((uintptr_t)W & 15) == 0 && ldw % 4 == 0 ? launch_pack<true, true>(a, st)
+                                                     : launch_pack<true, false>(a, st);
 }
 
 ssm_status launch_gemm_h3(const void* Xp, const float* X, long ldx, const void* Wp,

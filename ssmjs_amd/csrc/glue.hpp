@@ -42,9 +42,9 @@ ssm_status launch_rowgemm(int mode, const float* X, long ldx, const float* Z, lo
                           hipStream_t st, const float* g2 = nullptr, float* nout = nullptr,
                           long ldn = 0, bool* normed = nullptr);
 
-// One-token step projections (stepproj.hip): v = s[m] * X W^T on 16 x 16 tiles with an
-// epilogue; s[m] = 1 / sqrt(sum_j ssq[m * nssq + j] * inv_div + eps) when ssq is given.
-// X (M rows, padded to whole 16-row tiles) and W (N rows, likewise) are in fragment order.
+// One-token step projections (stepproj.hip): v = s[m] * X W^T with an epilogue;
+// s[m] = 1 / sqrt(sum_j ssq[m * nssq + j] * inv_div + eps) when ssq is given.
+// X (M rows, padded to whole 16-row tiles) is in fragment order.
 constexpr int kStepProjMaxRows = 64;
 constexpr int kStepProjMaxSsq = 256;
 
@@ -54,12 +54,12 @@ constexpr int kStepProjMaxSsq = 256;
 __host__ __device__ inline long frag_off(int m, int k, int KB) {
     return ((long)(m >> 4) * KB + (k >> 4)) * 256 + (((k >> 2) & 3) * 16 + (m & 15)) * 4 + (k & 3);
 }
-size_t frag_floats(int rows, int K);
 
-enum { EPI_STORE = 0, EPI_CONV = 1, EPI_RESID = 2 };
+enum { EPI_STORE = 0, EPI_CONV = 1, EPI_RESID = 2, EPI_HEAD = 3 };
 struct StepProj {
     const float* X = nullptr;              // (M, K) fragment order
-    const float* W = nullptr;              // (N, K) fragment order (launch_pack_frag)
+    const float* W = nullptr;              // (N, K) packed by launch_pack_step
+    const float* Wf = nullptr;             // the same W in fp32, row-major, row stride K
     int M = 0, N = 0, K = 0;
     const float* ssq = nullptr; int nssq = 0; float inv_div = 0.f, eps = 0.f;
     float* Y = nullptr; long ldy = 0; float beta = 0.f;
@@ -77,13 +77,22 @@ struct StepProj {
     // wxt[c, j] with wxt (C, RN) row-major (RN <= kXpartMaxRN, c0 and C multiples of 16); the
     // partials, (C / 16, 16 mt, RN), are added by the step's state update
     const float* wxt = nullptr; int RN = 0; float* xpart = nullptr;
-    int mt = 0, nt = 0, rotate = 0;        // tiles and k-start rotation (set by the launcher)
+    // EPI_HEAD: greedy (value, index) pairs, (M, nparts), one per row and workgroup
+    float* part = nullptr; int nparts = 0;
+    // set by the launcher: row and column tiles, row groups, passes over K, W's row exponents
+    int mt = 0, nt = 0, rg = 0, npass = 0;
+    const int* we = nullptr;
 };
 constexpr int kXpartMaxRN = 128;
 bool stepproj_ok(int M, int N, int K);
 ssm_status launch_stepproj(int epi, StepProj a, hipStream_t st);
-// W (N, K) row stride ldw -> fragment order in out (frag_floats(N, K) floats).
-ssm_status launch_pack_frag(const float* W, long ldw, int N, int K, float* out, hipStream_t st);
+// Workgroups of an EPI_HEAD launch that write a pair per row.
+int step_head_parts(int M, int N, int K);
+// W (N, K) row stride ldw -> the step projection's packed operand in out (step_w_floats(N, K)
+// floats, 16-byte aligned; gemm_h3.hip). The row exponents start at float step_ex_off.
+size_t step_ex_off(int rows, int K);
+size_t step_w_floats(int rows, int K);
+ssm_status launch_pack_step(const float* W, long ldw, int N, int K, float* out, hipStream_t st);
 // Mamba-1 one-token state update (scan_m1.hip): ykb = 0 writes y (B, D) with row stride ldy,
 // ykb > 0 in fragment order with K = 16 ykb. dtr given: the raw dt (before bias and softplus)
 // is formed in the kernel as dtr (B, R) [ld lddtr] times Wdt^T (Wdt (D, R) row-major, 16-byte
@@ -116,14 +125,14 @@ ssm_status launch_pack_t(const float* W, long ldw, int N, int K, float* out, hip
 // W (N, K) row-major (K % 4 == 0) -> quads: out[((k / 4) N + n) 4 + k % 4] = W[n, k].
 ssm_status launch_pack_q4(const float* W, int N, int K, float* out, hipStream_t st);
 // The one-token LM head (head.hip): y (M, V) [ldy] = s[m] xg E^T with xg (M, K) in fragment
-// order, s[m] = 1 / sqrt(inv_div sum_j ssq[m, j] + eps), Ef the fragment-order copy of E
-// (V, K); with argmax, also the greedy pick per row (largest logit, lowest index among equal
-// maxima). part: head_parts(V) pairs per row of workspace.
+// order, s[m] = 1 / sqrt(inv_div sum_j ssq[m, j] + eps), E (V, K) row-major and Ep its
+// launch_pack_step copy; with argmax, also the greedy pick per row (largest logit, lowest index
+// among equal maxima). part: head_parts(V) pairs per row of workspace.
 bool head_ok(int M, int V, int K);
 int head_parts(int V);
 ssm_status launch_head(const float* xg, const float* ssq, int nssq, float inv_div, float eps,
-                       const float* Ef, float* y, long ldy, int M, int V, int K, float* part,
-                       uint32_t* argmax, hipStream_t st);
+                       const float* Ep, const float* E, float* y, long ldy, int M, int V, int K,
+                       float* part, uint32_t* argmax, hipStream_t st);
 // xg = x * g in fragment order (K = d) and ssq (M, d / 16) partial sums of x^2: the first
 // RMSNorm of a step.
 ssm_status launch_xg_ssq(const float* x, long ldx, const float* g, float* xg, float* ssq, int M,

@@ -522,9 +522,9 @@ struct ssm_model {
     // few-row projection split-K workspace (partial products), grown on demand
     char* rg = nullptr;
     size_t rg_bytes = 0;
-    // in_proj / out_proj weights of the layers with a fused one-token step, in the step
-    // projection's fragment order (stepproj.hip); built at the first such step and rebuilt
-    // whenever the weights change
+    // in_proj / out_proj weights of the layers with a fused one-token step, split and packed for
+    // the step projection (stepproj.hip); built at the first such step and rebuilt whenever the
+    // weights change
     float* wp = nullptr;
     std::vector<long> wp_in, wp_out;   // float offsets into wp per layer (-1: not packed)
     std::vector<long> wp_x, wp_dt;     // Mamba-1 layers: x_proj and dt_proj
@@ -1215,7 +1215,7 @@ bool fused_step_ok(const ssm_model* m, const LayerW& Ly, int B, const Ws& w) {
     return B >= 1 && B <= ssm::kStepProjMaxRows && w.xg && w.yf && fusable(m, Ly);
 }
 
-// (Re)builds the fragment-order copies of the fusable layers' in_proj and out_proj.
+// (Re)builds the packed copies of the fusable layers' in_proj and out_proj.
 ssm_status pack_weights(ssm_model* m) {
     const Dims& d = m->dm;
     hipStream_t st = m->ctx->stream;
@@ -1230,23 +1230,23 @@ ssm_status pack_weights(ssm_model* m) {
         for (int l = 0; l < d.nl; ++l) {
             if (!fusable(m, m->layers[l])) continue;
             if (m->layers[l].type == SSM_LAYER_MAMBA1) {
-                m->wp_in[l] = off; off += (long)ssm::frag_floats(2 * d.D, d.d);
+                m->wp_in[l] = off; off += (long)ssm::step_w_floats(2 * d.D, d.d);
                 m->wp_dt[l] = off; off += ((long)d.D * d.R + 63) / 64 * 64;
                 if (m1_step) {   // x_proj rides in in_proj's epilogue: its transpose
                     m->wp_xt[l] = off;
                     off += ((long)d.D * (d.R + 2 * d.N) + 63) / 64 * 64;
                 } else {         // x_proj is its own step projection
                     m->wp_x[l] = off;
-                    off += (long)ssm::frag_floats(d.R + 2 * d.N, d.D);
+                    off += (long)ssm::step_w_floats(d.R + 2 * d.N, d.D);
                 }
             } else {
-                m->wp_in[l] = off; off += (long)ssm::frag_floats(d.nin, d.d);
+                m->wp_in[l] = off; off += (long)ssm::step_w_floats(d.nin, d.d);
             }
-            m->wp_out[l] = off; off += (long)ssm::frag_floats(d.d, d.D);
+            m->wp_out[l] = off; off += (long)ssm::step_w_floats(d.d, d.D);
         }
         if (ssm::head_ok(1, d.V, d.d)) {
             m->wp_emb = off;
-            off += (long)ssm::frag_floats(d.V, d.d);
+            off += (long)ssm::step_w_floats(d.V, d.d);
         }
         if (off == 0) return SSM_OK;
         SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wp, (size_t)off * sizeof(float)));
@@ -1256,10 +1256,10 @@ ssm_status pack_weights(ssm_model* m) {
         const LayerW& Ly = m->layers[l];
         if (Ly.type == SSM_LAYER_MAMBA1) {
             const int RN = d.R + 2 * d.N;
-            SSM_TRY(ssm::launch_pack_frag(m->w + Ly.in_proj, d.d, 2 * d.D, d.d,
+            SSM_TRY(ssm::launch_pack_step(m->w + Ly.in_proj, d.d, 2 * d.D, d.d,
                                           m->wp + m->wp_in[l], st));
             if (m->wp_x[l] >= 0)
-                SSM_TRY(ssm::launch_pack_frag(m->w + Ly.x_proj, d.D, RN, d.D, m->wp + m->wp_x[l],
+                SSM_TRY(ssm::launch_pack_step(m->w + Ly.x_proj, d.D, RN, d.D, m->wp + m->wp_x[l],
                                               st));
             // dt_proj is formed inside the state update: its rows in quads for the three-launch
             // step's update, else an aligned row-major copy
@@ -1273,14 +1273,14 @@ ssm_status pack_weights(ssm_model* m) {
                                            hipMemcpyDeviceToDevice, st));
             }
         } else {
-            SSM_TRY(ssm::launch_pack_frag(m->w + Ly.in_proj, d.d, d.nin, d.d, m->wp + m->wp_in[l],
+            SSM_TRY(ssm::launch_pack_step(m->w + Ly.in_proj, d.d, d.nin, d.d, m->wp + m->wp_in[l],
                                           st));
         }
-        SSM_TRY(ssm::launch_pack_frag(m->w + Ly.out_proj, d.D, d.d, d.D, m->wp + m->wp_out[l],
+        SSM_TRY(ssm::launch_pack_step(m->w + Ly.out_proj, d.D, d.d, d.D, m->wp + m->wp_out[l],
                                       st));
     }
     if (m->wp_emb >= 0)
-        SSM_TRY(ssm::launch_pack_frag(m->w + m->emb, d.d, d.V, d.d, m->wp + m->wp_emb, st));
+        SSM_TRY(ssm::launch_pack_step(m->w + m->emb, d.d, d.V, d.d, m->wp + m->wp_emb, st));
     return SSM_OK;
 }
 
@@ -1311,7 +1311,7 @@ ssm_status mixer_step_fused_m1(ssm_model* m, int l, float* hid, int B, float* ss
     float *xz = w.a, *xc = w.b, *dbl = w.c;
     { Stage g(c, "m1.step.in_proj");
       ssm::StepProj p;
-      p.X = w.xg; p.W = m->wp + m->wp_in[l]; p.M = B; p.N = 2 * d.D; p.K = d.d;
+      p.X = w.xg; p.W = m->wp + m->wp_in[l]; p.Wf = W + Ly.in_proj; p.M = B; p.N = 2 * d.D; p.K = d.d;
       p.ssq = w.ssq_in; p.nssq = d.d / 16; p.inv_div = 1.f / (float)d.d; p.eps = d.eps;
       p.Y = xz; p.ldy = 2 * d.D;
       p.c0 = 0; p.C = d.D; p.Kc = d.K; p.cw = W + Ly.conv_w; p.cb = W + Ly.conv_b;
@@ -1331,7 +1331,7 @@ ssm_status mixer_step_fused_m1(ssm_model* m, int l, float* hid, int B, float* ss
     } else {
         { Stage g(c, "m1.step.x_proj");
           ssm::StepProj p;
-          p.X = w.yf; p.W = m->wp + m->wp_x[l]; p.M = B; p.N = RN; p.K = d.D;
+          p.X = w.yf; p.W = m->wp + m->wp_x[l]; p.Wf = W + Ly.x_proj; p.M = B; p.N = RN; p.K = d.D;
           p.Y = dbl; p.ldy = RN;
           SSM_TRY(ssm::launch_stepproj(ssm::EPI_STORE, p, st)); }
         { Stage g(c, "m1.step.state_update");
@@ -1342,7 +1342,7 @@ ssm_status mixer_step_fused_m1(ssm_model* m, int l, float* hid, int B, float* ss
     }
     { Stage g(c, "m1.step.out_proj");
       ssm::StepProj p;
-      p.X = w.yf; p.W = m->wp + m->wp_out[l]; p.M = B; p.N = d.d; p.K = d.D;
+      p.X = w.yf; p.W = m->wp + m->wp_out[l]; p.Wf = W + Ly.out_proj; p.M = B; p.N = d.d; p.K = d.D;
       p.Y = hid; p.ldy = d.d;
       if (g_next) { p.g2 = g_next; p.xg = w.xg; p.ssq_out = w.ssq_in; }
       SSM_TRY(ssm::launch_stepproj(ssm::EPI_RESID, p, st)); }
@@ -1372,7 +1372,7 @@ ssm_status mixer_step_fused(ssm_model* m, int l, float* hid, int B, float* ssm_s
     const int GN = d.G * d.N;
     { Stage g(c, "m2.step.in_proj");
       ssm::StepProj p;
-      p.X = w.xg; p.W = m->wp + m->wp_in[l]; p.M = B; p.N = d.nin; p.K = d.d;
+      p.X = w.xg; p.W = m->wp + m->wp_in[l]; p.Wf = W + Ly.in_proj; p.M = B; p.N = d.nin; p.K = d.d;
       p.ssq = w.ssq_in; p.nssq = d.d / 16; p.inv_div = 1.f / (float)d.d; p.eps = d.eps;
       p.Y = zx; p.ldy = d.nin;
       p.c0 = d.D; p.C = d.cd; p.Kc = d.K; p.cw = W + Ly.conv_w; p.cb = W + Ly.conv_b;
@@ -1385,7 +1385,7 @@ ssm_status mixer_step_fused(ssm_model* m, int l, float* hid, int B, float* ssm_s
                                           d.P, d.G, d.N, st)); }
     { Stage g(c, "m2.step.out_proj");
       ssm::StepProj p;
-      p.X = w.yf; p.W = m->wp + m->wp_out[l]; p.M = B; p.N = d.d; p.K = d.D;
+      p.X = w.yf; p.W = m->wp + m->wp_out[l]; p.Wf = W + Ly.out_proj; p.M = B; p.N = d.d; p.K = d.D;
       p.ssq = w.ssq_y; p.nssq = ssm::m2_gated_nssq(d.H, d.P, d.N);
       p.inv_div = 1.f / (float)d.D; p.eps = d.eps;
       p.Y = hid; p.ldy = d.d;
@@ -1453,7 +1453,7 @@ ssm_status trunk(ssm_model* m, const uint32_t* d_ids, int B, int L, ssm_state* s
 
 // The own LM head (head.hip) over `rows` final hidden rows x (row stride ldx): the final
 // norm's operand x * g_f in fragment order and its partial sums (xg_ssq_kernel), then the
-// logits on the fragment-order tied embedding with the norm's scale applied per row, and the
+// logits on the packed tied embedding with the norm's scale applied per row, and the
 // greedy picks into d_argmax when given. Replaces the final RMSNorm, the library product and
 // the full-row argmax for up to kStepProjMaxRows rows.
 bool own_head_ok(ssm_model* m, const Ws& w, long rows) {
@@ -1468,7 +1468,8 @@ ssm_status head_rows(ssm_model* m, const Ws& w, const float* x, long ldx, int ro
     Stage g(m->ctx, "head");
     SSM_TRY(ssm::launch_xg_ssq(x, ldx, m->w + m->norm_f, w.xg, w.ssq_in, rows, d.d, st));
     return ssm::launch_head(w.xg, w.ssq_in, d.d / 16, 1.f / (float)d.d, d.eps,
-                            m->wp + m->wp_emb, lg, d.V, rows, d.V, d.d, w.hpart, d_argmax, st);
+                            m->wp + m->wp_emb, m->w + m->emb, lg, d.V, rows, d.V, d.d, w.hpart,
+                            d_argmax, st);
 }
 
 // The LM head over more rows than the own head takes: x already normalised.
@@ -1906,7 +1907,7 @@ ssm_status decode_body(ssm_model* m, ssm_state* s, const uint32_t* d_ids, float*
     const Dims& d = m->dm;
     Ws w;
     SSM_TRY(ensure_ws(m, s->B, 1, false, &w));
-    // the own LM head (head.hip) on the fragment-order embedding, with the final norm's scale
+    // the own LM head (head.hip) on the packed embedding, with the final norm's scale
     // and the greedy pick folded in
     const bool own_head = w.xg && w.hpart && ssm::head_ok(s->B, d.V, d.d) && d.d % 16 == 0;
     if (own_head && !m->wp) SSM_TRY(pack_weights(m));   // eager: the first step never replays
@@ -1914,8 +1915,8 @@ ssm_status decode_body(ssm_model* m, ssm_state* s, const uint32_t* d_ids, float*
     if (own_head) {
         Stage g(m->ctx, "head");
         return ssm::launch_head(w.xg, w.ssq_in, d.d / 16, 1.f / (float)d.d, d.eps,
-                                m->wp + m->wp_emb, lg, d.V, s->B, d.V, d.d, w.hpart, d_argmax,
-                                m->ctx->stream);
+                                m->wp + m->wp_emb, m->w + m->emb, lg, d.V, s->B, d.V, d.d,
+                                w.hpart, d_argmax, m->ctx->stream);
     }
     { Stage g(m->ctx, "head");
       SSM_TRY(proj_rows(m, 1, w.hid, d.d, nullptr, 0, m->w + m->norm_f, m->w + m->emb, lg, d.V,

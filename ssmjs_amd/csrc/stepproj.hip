@@ -1,5 +1,5 @@
-// Projections of the one-token step (decode: one row per sequence, M <= 64) on the gfx950
-// fp32 matrix cores, with the step's neighbouring element-wise work in the epilogue:
+// Projections of the one-token step (decode: one row per sequence, M <= 64) at fp32 precision on
+// the gfx950 fp16 matrix cores, with the step's neighbouring element-wise work in the epilogue:
 //
 //   v[m, n] = s[m] * sum_k X[m, k] W[n, k]          W (N, K)
 //   s[m]    = 1 / sqrt(sum_j ssq[m, j] * inv_div + eps)    (ssq given; else s = 1)
@@ -11,6 +11,9 @@
 //   EPI_RESID  Y[m, n] += v (the residual add); then, when g2 is given, the next RMSNorm's
 //              operand xg[m, n] = Y[m, n] * g2[n] (in fragment order, below) and the row's
 //              partial sum of squares over the tile's 16 columns, ssq_out[m, n / 16]
+//   EPI_HEAD   Y[m, n] = v (the LM head's logits) and, per row and workgroup, the largest logit
+//              with the lowest index among equal maxima (NaN never wins) as a (value, index)
+//              pair; a row's pairs are merged by head_argmax_kernel (head.hip)
 //   Yf         EPI_CONV: the conv outputs also written in fragment order, the operand of the
 //              step's next projection (the Mamba-1 step's x_proj as its own launch)
 //   xpart      EPI_CONV: that next projection summed over each conv tile's 16 channels (one
@@ -23,30 +26,36 @@
 // update (ssd.hip). The partial sums are added in a fixed order, identical in every
 // workgroup, so s[m] is the same wherever it is formed and every result is deterministic.
 //
-// Operand order. An MFMA operand puts 16 different rows in every 16 lanes (lane (i, q) =
-// (lane % 16, lane / 16) holds row i, k = 4q .. 4q+3 of a 16-wide k-block), so loading it
-// from a row-major matrix touches 16 cache lines per 16 lanes for 16 bytes each; measured,
-// that runs at a fraction of the L1's line rate (22 us for the 64 x 4384 x 1024 in_proj).
-// Both operands are therefore stored in fragment order (frag_off in glue.hpp): the 1 KB of
-// a (16-row tile, k-block) is contiguous, lane-major, and one b128 load per lane brings a
-// whole fragment as 8 full lines. W is packed once from the checkpoint layout (pack_frag
-// below, redone when the weights change); X is written in that order by its producer.
+// Split. As in gemm_h3.hip: a row of an operand is scaled by a power of two so that its largest
+// magnitude lies in [2^14, 2^15) and each element is held as fp16 hi + lo; a product is three
+// v_mfma_f32_16x16x32_f16 (lo hi, hi lo, hi hi) into fp32 sums, scaled back exactly. W is packed
+// once per load (launch_pack_step, gemm_h3.hip: a scale per row); X arrives in fp32 and each wave
+// scales and splits its own k range of it in registers, while its W is still on the way from HBM.
+// Elements that are inf or NaN become NaN, and an output that is not finite is formed again from
+// the fp32 operands.
 //
-// Decomposition. A workgroup owns one 16 x 16 output tile and all of K, which its 4 waves
-// split into contiguous quarters; the quarters are added in LDS in wave order. At the decode
-// shapes (64 rows) that is 4 * N / 16 workgroups: 256 for an out_proj into d_model 1024,
-// 1096 for a 4384-column in_proj. Larger tiles reuse operands more, but 64 x 16 tiles give
-// 274 workgroups for 256 CUs, and the 18 CUs that run two set the time (twice the mean); at
-// 16 x 16 the most loaded CU runs 5 tiles against a mean of 4.3. Each wave streams its
-// fragments PD k-blocks ahead; MFMA t of a block takes component t of both fragments
-// (k = 4q + t for lane group q), so its four MFMAs cover the block's 16 k exactly once.
+// Operand order. X is in fragment order (frag_off in glue.hpp): the 1 KB of a (16-row tile,
+// 16-wide k-block) is contiguous, lane-major, lane 16 q + i holding row i, k = 4 q .. + 3, so one
+// b128 load per lane brings 8 full lines. Two k-blocks make one MFMA operand of 32 k: elements
+// 0 .. 3 of lane (q, i) are k = 4 q .. + 3 of the first block, elements 4 .. 7 those of the second;
+// W's packed blocks (hi and lo, 1 KB each) use the same order of k.
 //
-// Tile order: workgroups are dispatched to the 8 XCDs round-robin by linear id, so the row
-// tiles of one column tile get ids 8 apart (same XCD): W, the only operand that comes from
-// HBM, is fetched once into that XCD's L2 and read from there by the other row tiles. W goes
-// through streaming (non-temporal) loads: its lines are wanted only while the row tiles of
-// their column tile run, and X, read by every column tile, keeps the rest of the cache
-// (measured: out_proj 8.00 -> 7.72 us at cfg4, 7.28 -> 6.88 us in the Mamba-1 step).
+// Decomposition. What bounds a step projection is bringing W (18 MB for a 4384 x 1024 in_proj)
+// from HBM once with everything in flight at once: 256 CUs at 6 TB/s and 2 us of latency is
+// 48 KB a CU. A workgroup of eight waves owns 16 MT rows x 16 columns and all of K; wave w takes
+// an eighth of K, issues all its X and W loads up front, keeps the split X in registers (128 at
+// most) and, when there are more column tiles than CUs, walks tiles of
+// stride gridDim with the next tile's W in flight. The waves' partial tiles meet in LDS, added in
+// wave order. MT covers all rows when that still gives every CU a workgroup (W then crosses the
+// L2 once, where 16 x 16 tiles had each W line requested by four row tiles); otherwise the row
+// tiles of a column tile are workgroups of their own, on one XCD (ids 8 apart), sharing W in L2.
+//
+// Measured (MI355X, weights cold, fp32 MFMA tiles of 16 x 16 -> this): 64 x 4384 x 1024 with the
+// conv update 14.8 -> 13.2 us, 64 x 3072 x 768 10.4 -> 9.0, the head 64 x 32000 x 1024 49 -> 32.8;
+// the narrow ones lose a little, 64 x 1024 x 2048 with the residual 7.5 -> 7.9 and 64 x 768 x 1536
+// 6.5 -> 7.0 (every workgroup splits its rows of X anew).
+#include <algorithm>
+
 #include "common.hpp"
 #include "glue.hpp"
 
@@ -54,17 +63,13 @@ namespace ssm {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-constexpr int kNW = 4;                  // waves per workgroup
+constexpr int kNW = 8;                  // waves per workgroup
+constexpr int kNT = 64 * kNW;
 constexpr unsigned kOOR = 0x80000000u;  // a buffer offset past every descriptor's range
-constexpr int kSsqPer = kStepProjMaxSsq / 16;   // partial sums per epilogue thread
-// EPI_CONV with xpart as a kernel of its own (its B fragments need registers that the plain
-// conv epilogue's occupancy target does not leave)
-constexpr int EPI_CONVX = 3;
+// EPI_CONV with xpart as a kernel of its own
+constexpr int EPI_CONVX = 4;
 
 __device__ __forceinline__ float sum16(float v) {
 #pragma unroll
@@ -72,227 +77,447 @@ __device__ __forceinline__ float sum16(float v) {
     return v;
 }
 
-template <int PD, int EPI>
-__global__ __launch_bounds__(64 * kNW, EPI == EPI_CONVX ? 4 : PD > 4 ? (EPI == EPI_CONV ? 4 : 5) : EPI == EPI_CONV ? 6 : 8) void stepproj_kernel(
-    StepProj a) {
+// greedy order: v wins over (best, bi) when larger, or equal with a lower index
+__device__ __forceinline__ void pick(float v, int i, float& best, int& bi) {
+    if (v > best || (v == best && i < bi)) { best = v; bi = i; }
+}
+
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ halfx8 as_h8(u32x4 v) { return __builtin_bit_cast(halfx8, v); }
+
+// Two elements times 2^sh as fp16 hi and lo (round to nearest), packed.
+__device__ __forceinline__ void split2(float a, float b, int sh, unsigned& hi, unsigned& lo) {
+    const float s0 = __builtin_ldexpf(a, sh), s1 = __builtin_ldexpf(b, sh);
+    const halfx2 h = {(_Float16)s0, (_Float16)s1};
+    const halfx2 l = {(_Float16)(s0 - (float)h[0]), (_Float16)(s1 - (float)h[1])};
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, l);
+}
+
+// sum_k X[m, k] W[n, k] from the fp32 operands (X in fragment order), k in order: outputs whose
+// split product is not finite.
+__device__ __noinline__ float step_exact(const float* X, const float* w, int m, int K) {
+    float s = 0.f;
+    for (int k = 0; k < K; ++k) s = fmaf(X[frag_off(m, k, K >> 4)], w[k], s);
+    return s;
+}
+
+// MT row tiles, NC column tiles at a time, KW 32-wide k-blocks per wave and pass; MULTI: a
+// workgroup walks several groups of column tiles (K then takes one pass).
+template <int MT, int NC, int KW, bool MULTI, int EPI>
+__global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     constexpr bool CONV = EPI == EPI_CONV || EPI == EPI_CONVX;
-    __shared__ float red[kNW][16][17];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    constexpr int ROWS = 16 * MT;
+    // epilogue elements of a thread: rows tid / 16 + 32 s, s < RS, of each column tile
+    constexpr int RS = (ROWS + 31) / 32, EPT = RS * NC;
+    __shared__ float red[MULTI ? 2 : 1][kNW][ROWS][16 * NC + 1];
+    __shared__ float sc[64];
+    __shared__ float us[EPI == EPI_CONVX ? ROWS : 1][16 * NC + 1];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, q = lane >> 4;
+    // row group tg and first column group: the row groups of a column group are 8 ids apart (one
+    // XCD); MULTI workgroups go on to the column groups gstep further
     const int b = blockIdx.x, r8 = b >> 3;
-    const int tm = r8 % a.mt, tn = (r8 / a.mt) * 8 + (b & 7);
-    if (tn >= a.nt) return;   // the id space is padded to whole groups of 8 column tiles
-    const int m0 = tm * 16, n0 = tn * 16;
+    const int tg = r8 % a.rg;
+    const int gstep = (int)gridDim.x / a.rg;
+    int tn = NC * ((r8 / a.rg) * 8 + (b & 7));   // first column tile
+    if (tn >= a.nt) return;   // (the id space is padded to whole groups of 8 column groups)
+    const int slot = tn / NC;   // EPI_HEAD: this workgroup's pair
+    const int m0 = tg * ROWS;
+    const int KB = a.K >> 4, KB2 = (KB + 1) >> 1;   // 16-wide blocks of X, 32-wide of W
 
-    // The epilogue's element (thread t: row t / 16, column t % 16 of the tile), and the
-    // partial sums of its row's scale, loaded ahead of the operands so that waiting for them
-    // overlaps the operands' latency (rows past M and sums past nssq read 0).
-    const int ei = tid >> 4, ej = tid & 15;
-    const int em = m0 + ei, en = n0 + ej;
-    float sp[kSsqPer];
-    if (a.ssq) {
-        const auto rs = rsrc(a.ssq, (unsigned)(a.M * a.nssq) * 4u);
+    // ---- operand loads: this wave's k-blocks of pass p are KW (kNW p + w) .. + KW - 1, summed
+    // in this order in every workgroup (equal rows of W give equal results). Every workgroup
+    // reads the same X; those on one XCD start at row tiles of their own.
+    const int irot = (r8 / a.rg) & (MT - 1);
+    const auto ra = rsrc(a.X, (unsigned)(a.mt * KB) * 1024u);
+    auto load_x = [&](float4 (&x)[MT][KW][2], int p) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < kSsqPer; ++u) {
-            const int j = u * 16 + ej;
-            sp[u] = bload4(rs, j < a.nssq ? (unsigned)(em * a.nssq + j) * 4u : kOOR);
-        }
-    }
-
-    // The conv epilogue's inputs (the cached inputs, the taps and the bias of this thread's
-    // channel), loaded here with the operands: they do not depend on the product, and loaded
-    // in the epilogue each would be a memory latency after the last MFMA (the state loads and
-    // the shift stores of one channel alias, so they were also serial there). Widths up to
-    // kConvPre; wider kernels keep the epilogue's own loads.
-    constexpr int kConvPre = 4;
-    const int ec = en - a.c0;
-    const bool conv_pre = CONV && em < a.M && en < a.N && ec >= 0 && ec < a.C && a.Kc <= kConvPre;
-    float csv[kConvPre - 1] = {}, cwv[kConvPre] = {}, cbv = 0.f;
-    if constexpr (CONV) {
-        if (conv_pre) {
-            const float* st = a.cst + ((long)em * a.C + ec) * (a.Kc - 1);
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int k = 0; k < kConvPre - 1; ++k)
-                if (k < a.Kc - 1) csv[k] = st[k];
+            for (int u = 0; u < KW; ++u)
 #pragma unroll
-            for (int k = 0; k < kConvPre; ++k)
-                if (k < a.Kc) cwv[k] = a.cw[(long)ec * a.Kc + k];
-            if (a.cb) cbv = a.cb[ec];
-        }
-    }
-
-    // The residual epilogue's inputs (this thread's element of Y and the next norm's weight),
-    // loaded here for the same reason; only this thread reads and writes that element.
-    float rsv = 0.f, g2v = 0.f;
-    if constexpr (EPI == EPI_RESID) {
-        if (em < a.M && en < a.N) rsv = a.Y[(long)em * a.ldy + en];
-        if (a.g2 && en < a.N) g2v = a.g2[en];
-    }
-
-    // EPI_CONV with xpart: a tile of conv columns (16 channels; c0 and C are multiples of 16)
-    // also projects its 16 x 16 conv outputs onto the next projection's RN columns on the
-    // matrix cores (the tile's outputs as the A operand, its 16 rows of wxt as B). Wave w takes
-    // the 16-column blocks w, w + 4, ...; its B fragments are loaded here (lane (j, k) of
-    // k-step s: wxt[channel 4s + k][16 block + j]) so that they arrive with the operands.
-    constexpr int kXpBlk = kXpartMaxRN / 16 / kNW;   // column blocks per wave
-    const bool xp_tile = EPI == EPI_CONVX && n0 >= a.c0 && n0 < a.c0 + a.C;
-    float wxb[kXpBlk][4];
-    if constexpr (EPI == EPI_CONVX) {
-        if (xp_tile) {
+                for (int h = 0; h < 2; ++h) {
+                    const int k16 = 2 * (KW * (kNW * p + w) + u) + h;
+                    const int tm = tg * MT + ((i + irot) & (MT - 1));
+                    x[i][u][h] = bload16<float4>(
+                        ra, k16 < KB && tm < a.mt ? (unsigned)(tm * KB + k16) * 1024u + 16u * lane
+                                                  : kOOR);
+                }
+    };
+    auto load_w = [&](halfx8 (&wv)[NC][KW][2], int t0, int p) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < kXpBlk; ++t) {
-                const int col = 16 * (w + kNW * t) + l16;
+        for (int j = 0; j < NC; ++j) {
+            const int t = t0 + j;
+            const auto rw = rsrc((const char*)a.W + (long)t * KB2 * 2048,
+                                 t < a.nt ? (unsigned)KB2 * 2048u : 0u);
 #pragma unroll
-                for (int s4 = 0; s4 < 4; ++s4)
-                    wxb[t][s4] = col < a.RN ? a.wxt[(long)(n0 - a.c0 + 4 * s4 + q) * a.RN + col]
-                                            : 0.f;
+            for (int u = 0; u < KW; ++u) {
+                const int kb = KW * (kNW * p + w) + u;
+                const unsigned o = kb < KB2 ? (unsigned)kb * 2048u + 16u * lane : kOOR;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) wv[j][u][h] = ssm::bload16_nt<halfx8>(rw, o + 1024u * h);
             }
         }
-    }
-
-    // this wave's k-blocks [kb0, kb0 + nb); fragment kb of a tile is 1 KB at kb * 1024
-    const int KB = a.K / 16;
-    const int bpw = (KB + kNW - 1) / kNW;
-    const int kb0 = w * bpw;
-    const int nb = min(bpw, KB - kb0);
-    const int ng = nb > 0 ? (nb + PD - 1) / PD : 0;
-    const auto ra = rsrc(a.X + (long)tm * KB * 256, (unsigned)KB * 1024u);
-    const auto rw = rsrc(a.W + (long)tn * KB * 256, (unsigned)KB * 1024u);
-    const unsigned o0 = (unsigned)kb0 * 1024u + (unsigned)lane * 16u;
-    // The column tiles that share an XCD read the same X fragments; each starts its k-blocks
-    // at its own rotation so that they do not all ask one L2 channel for one line at once.
-    // The row tiles of a column tile keep one rotation: they share W's lines in that L2.
-    const int rot = a.rotate && nb > 0 ? (r8 / a.mt) % nb : 0;
-    auto off = [&](int j) -> unsigned {   // j-th k-block of this wave, rotated
-        if (j >= nb) return kOOR;
-        const int jr = j + rot < nb ? j + rot : j + rot - nb;
-        return o0 + (unsigned)jr * 1024u;
+    };
+    // the row's power of two over this wave's k range, and the split operands; ex[i] packs what
+    // undoes the scale of the accumulator's rows 4 q + r of tile i
+    u32x4 xh[MT][KW], xl[MT][KW];   // eight fp16 values each
+    int ex[MT][4];
+    auto split = [&](const float4 (&x)[MT][KW][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            unsigned mx = 0;
+#pragma unroll
+            for (int u = 0; u < KW; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float4 v = x[i][u][h];
+                    const unsigned m1 = max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu);
+                    const unsigned m2 = max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu);
+                    mx = max(mx, max(m1, m2));
+                }
+            mx = max(mx, (unsigned)__shfl_xor((int)mx, 16));
+            mx = max(mx, (unsigned)__shfl_xor((int)mx, 32));
+            const int sh = mx ? 141 - min((int)(mx >> 23), 254) : 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ex[i][r] = -__shfl(sh, 4 * q + r);
+            // (an inf gives hi = inf, lo = NaN, and so NaN in every product of its row)
+#pragma unroll
+            for (int u = 0; u < KW; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float4 v = x[i][u][h];
+                    unsigned h0, l0, h1, l1;
+                    split2(v.x, v.y, sh, h0, l0);
+                    split2(v.z, v.w, sh, h1, l1);
+                    xh[i][u][2 * h] = h0; xh[i][u][2 * h + 1] = h1;
+                    xl[i][u][2 * h] = l0; xl[i][u][2 * h + 1] = l1;
+                }
+        }
+    };
+    floatx4 out[NC][MT];
+    auto multiply = [&](const halfx8 (&wv)[NC][KW][2]) __attribute__((always_inline)) {
+        floatx4 acc[NC][MT];
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        auto mm = [&](int j, int i, u32x4 x, halfx8 y) __attribute__((always_inline)) {
+            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(x), y, acc[j][i], 0, 0, 0);
+        };
+#pragma unroll
+        for (int u = 0; u < KW; ++u) {
+#pragma unroll
+            for (int j = 0; j < NC; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) mm(j, i, xl[i][u], wv[j][u][0]);
+#pragma unroll
+            for (int j = 0; j < NC; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) mm(j, i, xh[i][u], wv[j][u][1]);
+#pragma unroll
+            for (int j = 0; j < NC; ++j)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) mm(j, i, xh[i][u], wv[j][u][0]);
+        }
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = acc[j][i][r];
+                    out[j][i][r] += __builtin_ldexpf(v, ex[i][r]);
+                }
     };
 
-    float4 pa[PD], pb[PD];
-#pragma unroll
-    for (int j = 0; j < PD; ++j) {
-        pa[j] = bload16<float4>(ra, off(j));
-        pb[j] = ssm::bload16_nt<float4>(rw, off(j));   // W: streaming (see below)
-    }
-    float scale = 1.f;
+    float4 xr[MT][KW][2];
+    halfx8 w0[NC][KW][2];
+    load_x(xr, 0);
+    load_w(w0, tn, 0);
+
+    // ---- row scales: eight threads per row, each every eighth partial sum in order
     if (a.ssq) {
-        float t = sp[0];
+        const int srow = tid >> 3, m = m0 + srow;
+        const auto rs = rsrc(a.ssq, (unsigned)(a.M * a.nssq) * 4u);
+        float t = 0.f;
+        if (srow < ROWS) {
+            float sp[8];
 #pragma unroll
-        for (int u = 1; u < kSsqPer; ++u) t += sp[u];
-        t = sum16(t);
-        scale = 1.f / sqrtf(t * a.inv_div + a.eps);
-    }
-    floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    for (int g = 0; g < ng; ++g) {
-#pragma unroll
-        for (int j = 0; j < PD; ++j) {
-            acc0 = mfma4(pa[j].x, pb[j].x, acc0);
-            acc1 = mfma4(pa[j].y, pb[j].y, acc1);
-            acc0 = mfma4(pa[j].z, pb[j].z, acc0);
-            acc1 = mfma4(pa[j].w, pb[j].w, acc1);
-            const int nj = (g + 1) * PD + j;
-            pa[j] = bload16<float4>(ra, off(nj));
-            pb[j] = ssm::bload16_nt<float4>(rw, off(nj));
-            // keep each refill right behind the MFMAs that free its registers, so that PD
-            // blocks stay in flight (left alone, the scheduler sinks all refills to the end
-            // of the group and the next group waits a full memory latency)
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    // lane (l16, q) holds D[4q + r][l16]
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[w][4 * q + r][l16] = acc0[r] + acc1[r];
-    __syncthreads();
-    float v = red[0][ei][ej];
-#pragma unroll
-    for (int k = 1; k < kNW; ++k) v += red[k][ei][ej];
-    v *= scale;
-    const bool ok = em < a.M && en < a.N;
-    if constexpr (EPI == EPI_STORE) {
-        if (ok) {
-            float* y = a.Y + (long)em * a.ldy + en;
-            *y = a.beta != 0.f ? v + a.beta * *y : v;
-        }
-    } else if constexpr (CONV) {
-        const int c = en - a.c0;
-        const bool in_conv = c >= 0 && c < a.C;
-        float u = 0.f;   // the conv output; 0 on padding rows
-        if (ok && !in_conv) a.Y[(long)em * a.ldy + en] = v;
-        if (conv_pre) {
-            // same arithmetic order as the conv update kernel (conv1d.hip), on the prefetched
-            // inputs
-            const int Kc = a.Kc;
-            float* st = a.cst + ((long)em * a.C + c) * (Kc - 1);
-            float acc = cbv;
-#pragma unroll
-            for (int k = 0; k < kConvPre - 1; ++k)
-                if (k < Kc - 1) acc = fmaf(cwv[k], csv[k], acc);
-            float wl = cwv[0];
-#pragma unroll
-            for (int k = 1; k < kConvPre; ++k)
-                if (k == Kc - 1) wl = cwv[k];
-            acc = fmaf(wl, v, acc);
-#pragma unroll
-            for (int k = 1; k < kConvPre - 1; ++k)   // shift the cached inputs down
-                if (k < Kc - 1) st[k - 1] = csv[k];
-            if (Kc > 1) st[Kc - 2] = v;
-            u = silu_fast(acc);
-            a.Yc[(long)em * a.ldyc + c] = u;
-        } else if (ok && in_conv) {
-            // same arithmetic order as the conv update kernel (conv1d.hip)
-            const int Kc = a.Kc;
-            const float* wc = a.cw + (long)c * Kc;
-            float* s = a.cst + ((long)em * a.C + c) * (Kc - 1);
-            float acc = a.cb ? a.cb[c] : 0.f;
-            for (int k = 0; k < Kc - 1; ++k) {   // taps on the cached inputs, shifting them down
-                const float sv = s[k];
-                acc = fmaf(wc[k], sv, acc);
-                if (k > 0) s[k - 1] = sv;
+            for (int u = 0; u < 8; ++u) {
+                const int j = 8 * u + (tid & 7);
+                sp[u] = bload4(rs, j < a.nssq && m < a.M ? (unsigned)(m * a.nssq + j) * 4u : kOOR);
             }
-            acc = fmaf(wc[Kc - 1], v, acc);
-            if (Kc > 1) s[Kc - 2] = v;
-            u = silu_fast(acc);
-            a.Yc[(long)em * a.ldyc + c] = u;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t += sp[u];
+            for (int j = 64 + (tid & 7); j < a.nssq; j += 8)
+                t += bload4(rs, m < a.M ? (unsigned)(m * a.nssq + j) * 4u : kOOR);
         }
-        // padding rows of the fragment-order copy get zeros for the next projection
-        if (a.Yf && in_conv && en < a.N) a.Yf[frag_off(em, c, a.C >> 4)] = u;
-        if constexpr (EPI == EPI_CONVX) {
-            if (xp_tile) {   // uniform over the workgroup
-                __shared__ float us[16][17];
-                us[ei][ej] = u;
-                __syncthreads();
-                // D[i][j] = sum_s sum_k u[i][4s + k] wxt[4s + k][j]; lane (j, q) holds
-                // rows 4q .. 4q + 3
-                const int ct = (n0 - a.c0) >> 4;
+        t += __shfl_xor(t, 1);
+        t += __shfl_xor(t, 2);
+        t += __shfl_xor(t, 4);
+        if ((tid & 7) == 0 && srow < ROWS) sc[srow] = 1.f / sqrtf(t * a.inv_div + a.eps);
+    } else if (tid < ROWS) {
+        sc[tid] = 1.f;
+    }
+
+    // greedy pick so far of this thread's rows (EPI_HEAD; columns ascend from tile to tile)
+    float best[RS];
+    int bidx[RS];
 #pragma unroll
-                for (int t = 0; t < kXpBlk; ++t) {
-                    const int blk = w + kNW * t;
-                    if (16 * blk >= a.RN) break;   // wave-uniform
-                    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < RS; ++s) { best[s] = -INFINITY; bidx[s] = a.N; }
+
+    // descriptors of the epilogue's inputs (empty where absent: their loads give zeros)
+    const auto rwe = rsrc(a.we, (unsigned)a.nt * 64u);
+    const auto rcw = rsrc(a.cw, CONV ? (unsigned)(a.C * a.Kc) * 4u : 0u);
+    const auto rcb = rsrc(a.cb, CONV && a.cb ? (unsigned)a.C * 4u : 0u);
+    const auto rst = rsrc(a.cst, CONV ? (unsigned)(a.M * a.C * (a.Kc - 1)) * 4u : 0u);
+    const auto rg2 = rsrc(a.g2, EPI == EPI_RESID && a.g2 ? (unsigned)a.N * 4u : 0u);
+    const auto ryy = rsrc(a.Y, EPI == EPI_RESID ? (unsigned)((long)(a.M - 1) * a.ldy + a.N) * 4u : 0u);
+
+    // One column tile: W of its first pass is in wc; the next tile's goes into wnx.
+    constexpr int kConvPre = 4;
+    constexpr int kXpBlk = kXpartMaxRN / 16 / kNW;   // x_proj column blocks per wave
+    auto tile = [&](halfx8 (&wc)[NC][KW][2], halfx8 (&wnx)[NC][KW][2], int buf) __attribute__((always_inline)) {
+        // The epilogue's inputs, loaded ahead of the product (they do not depend on it): column
+        // en[j] of column tile j, rows as above.
+        const int ej = tid & 15;
+        int en[NC], wex[NC];
+        bool col_ok[NC], in_conv[NC], pre[NC];
+        float csv[EPT][kConvPre - 1], cwv[NC][kConvPre], cbv[NC], rsv[EPT], g2v[NC];
+        // (through range-checked descriptors: a guarded load would sit behind a branch, and the
+        // waits around those branches held the product back: in_proj 21.4 -> 14.7 us)
 #pragma unroll
-                    for (int s4 = 0; s4 < 4; ++s4)
-                        acc = mfma4(us[l16][4 * s4 + q], wxb[t][s4], acc);
-                    const int col = 16 * blk + l16;
-                    if (col < a.RN) {
-                        float* dst = a.xpart + ((long)ct * 16 * a.mt + m0 + 4 * q) * a.RN + col;
+        for (int j = 0; j < NC; ++j) {
+            en[j] = 16 * (tn + j) + ej;
+            col_ok[j] = en[j] < a.N;
+            const int c = en[j] - a.c0;
+            in_conv[j] = CONV && col_ok[j] && c >= 0 && c < a.C;
+            pre[j] = in_conv[j] && a.Kc <= kConvPre;
+            wex[j] = (int)__float_as_uint(bload4(rwe, col_ok[j] ? 4u * en[j] : kOOR));
+            if constexpr (CONV) {
+                const int Kc1 = a.Kc - 1;
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) dst[(long)r * a.RN] = acc[r];
-                    }
+                for (int k = 0; k < kConvPre; ++k)
+                    cwv[j][k] = bload4(rcw, pre[j] && k < a.Kc ? (unsigned)(c * a.Kc + k) * 4u : kOOR);
+                cbv[j] = bload4(rcb, pre[j] ? (unsigned)c * 4u : kOOR);
+#pragma unroll
+                for (int s = 0; s < RS; ++s) {
+                    const int ei = (tid >> 4) + 32 * s, em = m0 + ei;
+#pragma unroll
+                    for (int k = 0; k < kConvPre - 1; ++k)
+                        csv[j * RS + s][k] = bload4(rst, pre[j] && k < Kc1 && ei < ROWS && em < a.M
+                                                             ? (unsigned)((em * a.C + c) * Kc1 + k) * 4u
+                                                             : kOOR);
+                }
+            }
+            if constexpr (EPI == EPI_RESID) {
+                g2v[j] = bload4(rg2, col_ok[j] ? 4u * en[j] : kOOR);
+#pragma unroll
+                for (int s = 0; s < RS; ++s) {
+                    const int ei = (tid >> 4) + 32 * s, em = m0 + ei;
+                    rsv[j * RS + s] = bload4(ryy, col_ok[j] && ei < ROWS && em < a.M
+                                                      ? (unsigned)((long)em * a.ldy + en[j]) * 4u
+                                                      : kOOR);
                 }
             }
         }
-    } else {   // EPI_RESID
-        float o = 0.f;
-        if (ok) {
-            o = rsv + v;
-            a.Y[(long)em * a.ldy + en] = o;
+        // (c0 and C are multiples of 16 with xpart: a column tile is wholly conv or not at all)
+        bool xp_tile[NC];
+        float wxb[NC][kXpBlk][4];
+        if constexpr (EPI == EPI_CONVX) {
+            const auto rwx = rsrc(a.wxt, (unsigned)(a.C * a.RN) * 4u);
+            // B fragments of the next projection: lane (j, k) of k-step s holds
+            // wxt[channel 4 s + k][16 block + j], block w of the wave
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                const int n0 = 16 * (tn + j);
+                xp_tile[j] = n0 >= a.c0 && n0 < a.c0 + a.C;
+#pragma unroll
+                for (int t = 0; t < kXpBlk; ++t)
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4) {
+                        const int col = 16 * (w + kNW * t) + l16;
+                        wxb[j][t][s4] = bload4(rwx, xp_tile[j] && col < a.RN
+                                                        ? (unsigned)((n0 - a.c0 + 4 * s4 + q) * a.RN + col) * 4u
+                                                        : kOOR);
+                    }
+            }
         }
-        if (a.g2) {
-            // rows past M (up to the tile's 16) get zeros: the next projection reads whole tiles
-            if (en < a.N) a.xg[frag_off(em, en, a.nt)] = ok ? o * g2v : 0.f;
-            const float t = sum16(o * o);
-            if (ej == 0 && em < a.M) a.ssq_out[(long)em * a.nt + tn] = t;
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) out[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (MULTI) {
+            load_w(wnx, tn + NC * gstep, 0);   // past the last tile: an empty range
+            multiply(wc);
+        } else {
+            split(xr);
+            multiply(wc);
+            for (int p = 1; p < a.npass; ++p) {
+                load_x(xr, p);
+                load_w(wc, tn, p);
+                split(xr);
+                multiply(wc);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    red[buf][w][16 * ((i + irot) & (MT - 1)) + 4 * q + r][16 * j + l16] = out[j][i][r];
+        __syncthreads();
+
+        float uo[EPT];
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) {
+            const int j = e / RS;
+            const int ei = (tid >> 4) + 32 * (e % RS), em = m0 + ei, n = en[j], c = n - a.c0;
+            uo[e] = 0.f;
+            if (ei >= ROWS) continue;
+            float v = red[buf][0][ei][16 * j + ej];
+#pragma unroll
+            for (int k = 1; k < kNW; ++k) v += red[buf][k][ei][16 * j + ej];
+            v = __builtin_ldexpf(v, wex[j]);
+            const bool ok = em < a.M && col_ok[j];
+            if (!__builtin_isfinite(v) && ok) v = step_exact(a.X, a.Wf + (long)n * a.K, em, a.K);
+            v *= sc[ei];
+            if constexpr (EPI == EPI_STORE) {
+                if (ok) {
+                    float* y = a.Y + (long)em * a.ldy + n;
+                    *y = a.beta != 0.f ? v + a.beta * *y : v;
+                }
+            } else if constexpr (EPI == EPI_HEAD) {
+                if (ok) a.Y[(long)em * a.ldy + n] = v;
+                // (a row's columns ascend with j and from group to group)
+                const int s = e % RS;
+                if (col_ok[j] && (v > best[s] || (bidx[s] == a.N && v == best[s]))) { best[s] = v; bidx[s] = n; }
+            } else if constexpr (CONV) {
+                if (ok && !in_conv[j]) a.Y[(long)em * a.ldy + n] = v;
+                float u = 0.f;   // the conv output; 0 on padding rows
+                const int Kc = a.Kc;
+                if (ok && pre[j]) {
+                    // same arithmetic order as the conv update kernel (conv1d.hip), on the
+                    // prefetched inputs
+                    float* st = a.cst + ((long)em * a.C + c) * (Kc - 1);
+                    float acc = cbv[j];
+#pragma unroll
+                    for (int k = 0; k < kConvPre - 1; ++k)
+                        if (k < Kc - 1) acc = fmaf(cwv[j][k], csv[e][k], acc);
+                    float wl = cwv[j][0];
+#pragma unroll
+                    for (int k = 1; k < kConvPre; ++k)
+                        if (k == Kc - 1) wl = cwv[j][k];
+                    acc = fmaf(wl, v, acc);
+#pragma unroll
+                    for (int k = 1; k < kConvPre - 1; ++k)   // shift the cached inputs down
+                        if (k < Kc - 1) st[k - 1] = csv[e][k];
+                    if (Kc > 1) st[Kc - 2] = v;
+                    u = silu_fast(acc);
+                    a.Yc[(long)em * a.ldyc + c] = u;
+                } else if (ok && in_conv[j]) {
+                    const float* wcv = a.cw + (long)c * Kc;
+                    float* st = a.cst + ((long)em * a.C + c) * (Kc - 1);
+                    float acc = a.cb ? a.cb[c] : 0.f;
+                    for (int k = 0; k < Kc - 1; ++k) {   // taps on the cached inputs, shifting them
+                        const float sv = st[k];
+                        acc = fmaf(wcv[k], sv, acc);
+                        if (k > 0) st[k - 1] = sv;
+                    }
+                    acc = fmaf(wcv[Kc - 1], v, acc);
+                    if (Kc > 1) st[Kc - 2] = v;
+                    u = silu_fast(acc);
+                    a.Yc[(long)em * a.ldyc + c] = u;
+                }
+                uo[e] = u;
+                // padding rows of the fragment-order copy get zeros for the next projection
+                if (a.Yf && in_conv[j] && em < 16 * a.mt) a.Yf[frag_off(em, c, a.C >> 4)] = u;
+            } else {   // EPI_RESID
+                float o = 0.f;
+                if (ok) {
+                    o = rsv[e] + v;
+                    a.Y[(long)em * a.ldy + n] = o;
+                }
+                if (a.g2) {
+                    // rows past M (up to the tile's 16) get zeros: the next projection reads
+                    // whole tiles
+                    if (col_ok[j] && em < 16 * a.mt) a.xg[frag_off(em, n, a.nt)] = ok ? o * g2v[j] : 0.f;
+                    const float t = sum16(o * o);
+                    if (ej == 0 && em < a.M && col_ok[j]) a.ssq_out[(long)em * a.nt + tn + j] = t;
+                }
+            }
+        }
+        if constexpr (EPI == EPI_CONVX) {
+#pragma unroll
+            for (int e = 0; e < EPT; ++e)
+                if ((tid >> 4) + 32 * (e % RS) < ROWS)
+                    us[(tid >> 4) + 32 * (e % RS)][16 * (e / RS) + ej] = uo[e];
+            __syncthreads();
+            // D[i][j] = sum_s sum_k u[i][4s + k] wxt[4s + k][j] on the fp32 matrix cores;
+            // lane (j, q) holds rows 4q .. 4q + 3
+#pragma unroll
+            for (int j = 0; j < NC; ++j) {
+                if (!xp_tile[j]) continue;   // (uniform over the workgroup)
+                const int ct = tn + j - (a.c0 >> 4);
+#pragma unroll
+                for (int t = 0; t < kXpBlk; ++t) {
+                    const int blk = w + kNW * t, col = 16 * blk + l16;
+                    if (16 * blk >= a.RN) break;   // wave-uniform
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) {
+                        if (tg * MT + i >= a.mt) break;
+                        floatx4 xa = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int s4 = 0; s4 < 4; ++s4)
+                            xa = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                us[16 * i + l16][16 * j + 4 * s4 + q], wxb[j][t][s4], xa, 0, 0, 0);
+                        if (col < a.RN) {
+                            float* dst = a.xpart + ((long)ct * 16 * a.mt + m0 + 16 * i + 4 * q) * a.RN + col;
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) dst[(long)r * a.RN] = xa[r];
+                        }
+                    }
+                }
+            }
+            if constexpr (MULTI) __syncthreads();   // us is written again by the next group
+        }
+    };
+    if constexpr (MULTI) {
+        // tiles in pairs, so that each of the two W buffers is named statically. A wave may run
+        // one barrier ahead of another: red is double-buffered.
+        halfx8 w1[NC][KW][2];
+        split(xr);
+        for (;;) {
+            tile(w0, w1, 0);
+            tn += NC * gstep;
+            if (tn >= a.nt) break;
+            tile(w1, w0, 1);
+            tn += NC * gstep;
+            if (tn >= a.nt) break;
+        }
+    } else {
+        tile(w0, w0, 0);
+    }
+    if constexpr (EPI == EPI_HEAD) {
+        // a row's best over the workgroup's columns (16 lanes), one pair per row
+#pragma unroll
+        for (int s = 0; s < RS; ++s) {
+            const int ei = (tid >> 4) + 32 * s, em = m0 + ei;
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) {
+                const float ov = __shfl_xor(best[s], o, 16);
+                const int oi = __shfl_xor(bidx[s], o, 16);
+                pick(ov, oi, best[s], bidx[s]);
+            }
+            if ((tid & 15) == 0 && ei < ROWS && em < a.M) {
+                float* dst = a.part + ((long)em * a.nparts + slot) * 2;
+                dst[0] = best[s];
+                dst[1] = __int_as_float(bidx[s]);
+            }
         }
     }
 }
@@ -342,27 +567,6 @@ __global__ __launch_bounds__(256) void embed_xg_kernel(const uint32_t* __restric
     if (ok && (n & 15) == 0) ssq[(long)m * (d / 16) + n / 16] = t;
 }
 
-// W (N, K) row stride ldw -> fragment order, N padded with zero rows to whole 16-row tiles.
-// One thread per 16 bytes of the output; W is read as scalars (a layer's weights start at any
-// float offset of the checkpoint buffer, and this runs once per weight change).
-__global__ __launch_bounds__(256) void pack_frag_kernel(const float* __restrict__ W, long ldw,
-                                                        int N, int K, float* __restrict__ out) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;   // float4 index
-    const int KB = K / 16;
-    const long total = (long)((N + 15) / 16) * KB * 64;
-    if (i >= total) return;
-    const int lane = (int)(i & 63);
-    const long blk = i >> 6;
-    const int kb = (int)(blk % KB), tn = (int)(blk / KB);
-    const int n = tn * 16 + (lane & 15), k = kb * 16 + 4 * (lane >> 4);
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (n < N) {
-        const float* r = W + (long)n * ldw + k;
-        v = make_float4(r[0], r[1], r[2], r[3]);
-    }
-    reinterpret_cast<float4*>(out)[i] = v;
-}
-
 // W (N, K) row stride ldw -> W^T (K, N) row-major, out[k N + n] = W[n ldw + k]: the conv
 // epilogue's x_proj slice of a tile is then 16 contiguous rows. One thread per element (runs
 // once per weight change).
@@ -386,15 +590,16 @@ __global__ __launch_bounds__(256) void pack_q4_kernel(const float* __restrict__ 
     out[i] = make_float4(r[0], r[1], r[2], r[3]);
 }
 
-template <int PD>
-ssm_status launch_pd(int epi, const StepProj& a, unsigned grid, hipStream_t st) {
+template <int MT, int NC, int KW, bool MULTI>
+ssm_status launch_mk(int epi, const StepProj& a, unsigned grid, hipStream_t st) {
     switch (epi) {
-        case EPI_STORE: stepproj_kernel<PD, EPI_STORE><<<grid, 64 * kNW, 0, st>>>(a); break;
+        case EPI_STORE: stepproj_kernel<MT, NC, KW, MULTI, EPI_STORE><<<grid, kNT, 0, st>>>(a); break;
         case EPI_CONV:
-            if (a.xpart) stepproj_kernel<PD, EPI_CONVX><<<grid, 64 * kNW, 0, st>>>(a);
-            else stepproj_kernel<PD, EPI_CONV><<<grid, 64 * kNW, 0, st>>>(a);
+            if (a.xpart) stepproj_kernel<MT, NC, KW, MULTI, EPI_CONVX><<<grid, kNT, 0, st>>>(a);
+            else stepproj_kernel<MT, NC, KW, MULTI, EPI_CONV><<<grid, kNT, 0, st>>>(a);
             break;
-        default: stepproj_kernel<PD, EPI_RESID><<<grid, 64 * kNW, 0, st>>>(a); break;
+        case EPI_HEAD: stepproj_kernel<MT, NC, KW, MULTI, EPI_HEAD><<<grid, kNT, 0, st>>>(a); break;
+        default: stepproj_kernel<MT, NC, KW, MULTI, EPI_RESID><<<grid, kNT, 0, st>>>(a); break;
     }
     return check_launch("stepproj");
 }
@@ -404,17 +609,6 @@ ssm_status launch_pd(int epi, const StepProj& a, unsigned grid, hipStream_t st) 
 bool stepproj_ok(int M, int N, int K) {
     return M >= 1 && M <= kStepProjMaxRows && N >= 1 && K >= 16 && K % 16 == 0 &&
            (long)K * 64 < (1L << 31);
-}
-
-size_t frag_floats(int rows, int K) { return (size_t)((rows + 15) / 16) * 16 * K; }
-
-ssm_status launch_pack_frag(const float* W, long ldw, int N, int K, float* out, hipStream_t st) {
-    SSM_REQUIRE(K % 16 == 0 && ldw >= K && ((uintptr_t)out & 15) == 0,
-                "pack_frag: K %d / ldw %ld / alignment", K, ldw);
-    const long n4 = (long)frag_floats(N, K) / 4;
-    if (n4 == 0) return SSM_OK;
-    pack_frag_kernel<<<(unsigned)cdiv(n4, 256), 256, 0, st>>>(W, ldw, N, K, out);
-    return check_launch("pack_frag");
 }
 
 ssm_status launch_pack_t(const float* W, long ldw, int N, int K, float* out, hipStream_t st) {
@@ -432,6 +626,40 @@ ssm_status launch_pack_q4(const float* W, int N, int K, float* out, hipStream_t 
     return check_launch("pack_q4");
 }
 
+// Row tiles (rt) and column tiles (nc) per workgroup: as many rows as still give most CUs a
+// workgroup (W then crosses the L2 fewer times, but each workgroup loads and splits its rows of
+// X). Three and four row tiles go as two groups of two with two column tiles each: half the X
+// per workgroup for the same W (64 rows of 4384 x 1024: 14.7 us with all rows and one column
+// tile, 13.2 this way). 64 rows of 2048 -> 1024 leave one row tile each, 256 workgroups. per:
+// 32-wide k-blocks per wave and pass, what the registers hold of X next to W.
+namespace {
+constexpr int kStepMaxWG = 256;   // workgroups that walk column groups: one per CU
+struct StepPlan {
+    int rt, nc, rg, per, npass;
+    bool multi;
+    unsigned grid;
+};
+StepPlan step_plan(int M, int N, int K) {
+    const int mt = (M + 15) / 16, nt = (N + 15) / 16;
+    const int kw = (int)cdiv(cdiv(K, 32), kNW);   // k-blocks per wave
+    StepPlan p;
+    p.rt = mt <= 1 || (long)nt * cdiv(mt, 2) < 192 ? 1 : 2;
+    p.rg = (int)cdiv(mt, p.rt);
+    p.nc = p.rt == 2 && p.rg == 2 && nt >= 192 ? 2 : 1;
+    p.per = p.rt > 1 || kw <= 4 ? 4 : 8;
+    p.npass = (int)cdiv(kw, p.per);
+    const long groups = cdiv(nt, p.nc), padded = 8L * cdiv(groups, 8);
+    p.multi = p.npass == 1 && padded * p.rg > kStepMaxWG && kStepMaxWG % (8 * p.rg) == 0;
+    p.grid = p.multi ? (unsigned)kStepMaxWG : (unsigned)(padded * p.rg);
+    return p;
+}
+}  // namespace
+
+int step_head_parts(int M, int N, int K) {
+    const StepPlan p = step_plan(M, N, K);
+    return p.multi ? (int)p.grid / p.rg : (int)cdiv((N + 15) / 16, p.nc);
+}
+
 ssm_status launch_stepproj(int epi, StepProj a, hipStream_t st) {
     SSM_REQUIRE(stepproj_ok(a.M, a.N, a.K) && ((uintptr_t)a.X & 15) == 0 &&
                     ((uintptr_t)a.W & 15) == 0,
@@ -446,19 +674,28 @@ ssm_status launch_stepproj(int epi, StepProj a, hipStream_t st) {
     SSM_REQUIRE(!a.xpart || (epi == EPI_CONV && a.wxt && a.RN >= 1 && a.RN <= kXpartMaxRN &&
                              a.c0 % 16 == 0 && a.C % 16 == 0),
                 "stepproj: x_proj partial arguments");
+    SSM_REQUIRE(a.Wf && (epi != EPI_HEAD || a.part), "stepproj: arguments");
+    // 32-bit offsets of the epilogue's operands
+    SSM_REQUIRE((long)a.M * a.C * a.Kc * 4 < (1L << 31) && (long)a.C * a.RN * 4 < (1L << 31) &&
+                    (long)a.M * a.ldy * 4 < (1L << 31),
+                "stepproj: operand too large");
     a.mt = (a.M + 15) / 16;
     a.nt = (a.N + 15) / 16;
-    const unsigned grid = (unsigned)(8L * a.mt * ((a.nt + 7) / 8));
-    // Measured at 64 rows (K 1024 .. 2048): with about one tile per CU, 8 k-blocks in flight
-    // per wave and no rotation (5.5 us for 1024 x 2048, against 6.3 rotated and 6.4 with 16
-    // blocks); with several tiles per CU, 4 blocks and rotated starts (12.8 us for 4384 x 1024,
-    // against 13.5 with 8 blocks and 14.3 unrotated).
-    if ((long)a.mt * a.nt <= 512) {
-        a.rotate = 0;
-        return launch_pd<8>(epi, a, grid, st);
+    a.we = (const int*)(a.W + step_ex_off(a.N, a.K));
+    const StepPlan p = step_plan(a.M, a.N, a.K);
+    a.rg = p.rg; a.npass = p.npass;
+    SSM_REQUIRE(epi != EPI_HEAD || a.nparts == step_head_parts(a.M, a.N, a.K),
+                "stepproj: head pairs");
+    if (p.multi) {
+        if (p.nc == 2) return launch_mk<2, 2, 4, true>(epi, a, p.grid, st);
+        if (p.rt == 2) return launch_mk<2, 1, 4, true>(epi, a, p.grid, st);
+        return p.per == 4 ? launch_mk<1, 1, 4, true>(epi, a, p.grid, st)
+                          : launch_mk<1, 1, 8, true>(epi, a, p.grid, st);
     }
-    a.rotate = 1;
-    return launch_pd<4>(epi, a, grid, st);
+    if (p.nc == 2) return launch_mk<2, 2, 4, false>(epi, a, p.grid, st);
+    if (p.rt == 2) return launch_mk<2, 1, 4, false>(epi, a, p.grid, st);
+    return p.per == 4 ? launch_mk<1, 1, 4, false>(epi, a, p.grid, st)
+                      : launch_mk<1, 1, 8, false>(epi, a, p.grid, st);
 }
 
 ssm_status launch_embed_xg(const uint32_t* ids, const float* emb, float* hid, const float* g,
