@@ -94,6 +94,7 @@ struct SmemF32 {
     float c[FULL ? 2 : 1][FULL ? QF : 1][BP];            // C (i, n), two chunks
     float m[HPW][FULL ? QF : 1][MP];                     // M^T (i, j) per head
     float ac[2][HPW][QF];    // acum_t in log2 units
+    float al[NN <= 32 ? 2 : 1][HPW][NN <= 32 ? QF : 1];   // d_state <= 32: its low part
     float dv[2][HPW][QF];    // dt'_t
     float wj[2][HPW][QF];    // w_t = 2^(acum_end - acum_t) dt'_t
     float ae[2][HPW];        // acum_end
@@ -121,6 +122,35 @@ __device__ __forceinline__ float wave_prefix_sum(float v) {
     v = add_dpp<0x142, 0xa>(v);
     v = add_dpp<0x143, 0xc>(v);
     return v;
+}
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ double add_dpp(double x) {
+    const u32x2 v = __builtin_bit_cast(u32x2, x);
+    u32x2 y;
+    y[0] = __builtin_amdgcn_update_dpp(0, v[0], CTRL, ROW_MASK, 0xf, true);
+    y[1] = __builtin_amdgcn_update_dpp(0, v[1], CTRL, ROW_MASK, 0xf, true);
+    return x + __builtin_bit_cast(double, y);
+}
+
+// The same over the first 32 lanes (a chunk) in double.
+__device__ __forceinline__ double wave_prefix_sum(double v) {
+    v = add_dpp<0x111, 0xf>(v);
+    v = add_dpp<0x112, 0xf>(v);
+    v = add_dpp<0x114, 0xf>(v);
+    v = add_dpp<0x118, 0xf>(v);
+    v = add_dpp<0x142, 0xa>(v);
+    return v;
+}
+
+__device__ __forceinline__ double lane_of(double v, int lane) {
+    const u32x2 b = __builtin_bit_cast(u32x2, v);
+    u32x2 r;
+    r[0] = __builtin_amdgcn_readlane((int)b[0], lane);
+    r[1] = __builtin_amdgcn_readlane((int)b[1], lane);
+    return __builtin_bit_cast(double, r);
 }
 
 __device__ __forceinline__ float4 as_f4(floatx4 v) { return make_float4(v[0], v[1], v[2], v[3]); }
@@ -309,21 +339,40 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     }
     bool state_live = init != nullptr || (CHAIN && seg > 0);
     float decay_sum = 0.f;
-    // dt' of chunk cc (0 past the segment), its running sum times A_h and the weights w_t into
-    // LDS buffer bf (lane = time step)
-    auto scan_put = [&](int cc, float raw_dt, int bf) {
-        const int qv = rows_of(cc);
+    // dt' of a chunk of qv steps (0 past them), its running sum times A_h and the weights w_t
+    // into LDS buffer bf of head k (lane = time step; `put`: this wave writes); returns the
+    // chunk's whole sum. With d_state <= 32 the running sum is kept to double precision, as
+    // hi + lo: decays are differences of it, and a head of fast decay reaches 60 log2 units in a
+    // chunk, where one fp32 rounding of the sum is 1.3e-6 of the decay (relative error of the
+    // final state 1.3e-6 -> 1e-7, against 4e-7 of a product of the steps' decays, which these
+    // shapes had before the matrix-core kernel; the scan's time is hidden).
+    auto scan_dt = [&](float raw_dt, int qv, int bf, int k, bool put) __attribute__((always_inline)) {
         float dv = raw_dt + dtb;
         if (a.softplus) dv = NN <= 32 ? ssm::softplus_corr(dv) : ssm::softplus_fast(dv);
         dv = lane < qv ? fminf(fmaxf(dv, a.dt_min), a.dt_max) : 0.f;
-        const float sc = wave_prefix_sum(dv * Ah);
-        const float ae = __builtin_bit_cast(
-            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sc), QF - 1));
-        if (lane < QF) {
-            sm.ac[bf][hw][lane] = sc;
-            sm.dv[bf][hw][lane] = dv;
-            sm.wj[bf][hw][lane] = ssm::ex2(ae - sc) * dv;
+        float sc, ae, we;
+        if constexpr (NN <= 32) {
+            const double sd = wave_prefix_sum((double)dv * (double)Ah);
+            const double ad = lane_of(sd, QF - 1);
+            sc = (float)sd;
+            ae = (float)ad;
+            we = (float)(ad - sd);
+            if (put && lane < QF) sm.al[bf][k][lane] = (float)(sd - (double)sc);
+        } else {
+            sc = wave_prefix_sum(dv * Ah);
+            ae = __builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sc), QF - 1));
+            we = ae - sc;
         }
+        if (put && lane < QF) {
+            sm.ac[bf][k][lane] = sc;
+            sm.dv[bf][k][lane] = dv;
+            sm.wj[bf][k][lane] = ssm::ex2(we) * dv;
+        }
+        return ae;
+    };
+    auto scan_put = [&](int cc, float raw_dt, int bf) __attribute__((always_inline)) {
+        const float ae = scan_dt(raw_dt, rows_of(cc), bf, hw, true);
         if (lane == 0) sm.ae[bf][hw] = ae;
     };
 
@@ -355,18 +404,8 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
         // step; the full pass formed them a chunk earlier)
         float acend = 0.f;
         if constexpr (!FULL) {
-            float dv = raw.dt + dtb;
-            if (a.softplus) dv = NN <= 32 ? ssm::softplus_corr(dv) : ssm::softplus_fast(dv);
-            dv = lane < qv ? fminf(fmaxf(dv, a.dt_min), a.dt_max) : 0.f;
-            const float sc = wave_prefix_sum(dv * Ah);
-            acend = __builtin_bit_cast(
-                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sc), QF - 1));
+            acend = scan_dt(raw.dt, qv, buf, 0, w == 0);
             decay_sum += acend;
-            if (w == 0 && lane < QF) {
-                sm.ac[buf][0][lane] = sc;
-                sm.dv[buf][0][lane] = dv;
-                sm.wj[buf][0][lane] = ssm::ex2(acend - sc) * dv;
-            }
         }
         // ---- stage B (and C) rows
 #pragma unroll
@@ -449,13 +488,22 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
                     const float4 dvj = *reinterpret_cast<const float4*>(&sm.dv[buf][k][16 * jb + 4 * q4]);
                     const float acja[4] = {acj.x, acj.y, acj.z, acj.w};
                     const float dvja[4] = {dvj.x, dvj.y, dvj.z, dvj.w};
+                    float dl[4] = {aci - acja[0], aci - acja[1], aci - acja[2], aci - acja[3]};
+                    if constexpr (NN <= 32) {
+                        const float ali = sm.al[buf][k][i];
+                        const float4 alj = *reinterpret_cast<const float4*>(&sm.al[buf][k][16 * jb + 4 * q4]);
+                        dl[0] += ali - alj.x;
+                        dl[1] += ali - alj.y;
+                        dl[2] += ali - alj.z;
+                        dl[3] += ali - alj.w;
+                    }
                     float mv[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int j = 16 * jb + 4 * q4 + r;
                         // the masked (j > i) exponent may overflow: select, never multiply by 0
                         const float cbs = cb_wave ? cbv[r] : acc0[r] + acc1[r];
-                        const float f = cbs * (ssm::ex2(aci - acja[r]) * dvja[r]);
+                        const float f = cbs * (ssm::ex2(dl[r]) * dvja[r]);
                         mv[r] = j < i ? f : (j == i ? f + Dh[k] : 0.f);
                     }
                     *reinterpret_cast<float4*>(&sm.m[k][i][16 * jb + 4 * q4]) =

@@ -88,3 +88,31 @@ def test_mixer_matches_oracle(H, N):
         close(y, om.mixer(0, x), f"mixer B={B} L={L}")
     m.destroy()
     dev.destroy()
+
+
+@pytest.mark.parametrize("B,L,H,N,P", [(1, 64, 8, 16, 64), (2, 333, 12, 16, 128), (1, 90, 4, 32, 64)])
+def test_fast_decay_keeps_precision(B, L, H, N, P):
+    """Heads whose decay reaches tens of log2 units within a chunk: y and the final state against
+    float64 in the 2-norm. A step's decay and weight are a rounded exponent difference d (d 2^-24
+    ln 2, at most 0.53 2^-24 after its weight 2^-d), 2^x, softplus and three products: 5 roundings
+    of 2^-24, and the last 16-wide sum's few; 6e-7 together. (A running sum in fp32 loses 1.3e-6.)"""
+    print(f"[case] ssd fast decay B={B} L={L} H={H} N={N} P={P}", flush=True)
+    from ssmjs_amd import kernels
+    x, dt, _, Bm, Cm, D, h0 = inputs(L, B, L, H, P, 1, N)
+    A = -np.linspace(12, 16, H).astype(np.float32)
+    dt += 1
+    t = [torch.from_numpy(a).cuda() for a in (x, dt, A, Bm, Cm, D, h0)]
+    out = torch.empty(B, H, P, N, device="cuda")
+    y = kernels.ssd_chunk_scan(*t[:6], h0=t[6], hT=out)
+    torch.cuda.synchronize()
+    x, dt, A, Bm, Cm, D, h = (a.astype(np.float64) for a in (x, dt, A, Bm, Cm, D, h0))
+    d = np.log1p(np.exp(dt))
+    ref = np.empty_like(x)
+    for i in range(L):
+        h = (np.exp(d[:, i] * A)[:, :, None, None] * h +
+             (d[:, i, :, None] * x[:, i])[..., None] * Bm[:, i, 0][:, None, None])
+        ref[:, i] = (h * Cm[:, i, 0][:, None, None]).sum(-1) + D[:, None] * x[:, i]
+    for got, want, what in ((y, ref, "y"), (out, h, "final state")):
+        rel = np.linalg.norm(got.cpu().numpy() - want) / np.linalg.norm(want)
+        print(f"  {what}: relative 2-norm {rel:.2e}", flush=True)
+        assert rel <= 6e-7
