@@ -1204,7 +1204,7 @@ bool fusable(const ssm_model* m, const LayerW& Ly) {
                ssm::stepproj_ok(1, d.d, d.D);
     }
     if (Ly.type != SSM_LAYER_MAMBA2 || d.G != 1) return false;
-    if (!(d.N == 64 || d.N == 128 || d.N == 256) || d.K > 8) return false;
+    if (!(d.N == 16 || d.N == 32 || d.N == 64 || d.N == 128 || d.N == 256) || d.K > 8) return false;
     if (d.d % 16 != 0 || d.d / 16 > ssm::kStepProjMaxSsq) return false;
     if (ssm::m2_gated_nssq(d.H, d.P, d.N) > ssm::kStepProjMaxSsq) return false;
     if (d.D % 16 != 0 || d.cd % 4 != 0) return false;   // whole k-blocks; 16-byte B, C rows

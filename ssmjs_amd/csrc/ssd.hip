@@ -1267,11 +1267,13 @@ extern "C" ssm_status ssm_m2_state_update(const float* x, long ldx, const float*
 
 namespace ssm {
 
-// Two state rows per thread, as in ssm_m2_state_update: P / (2 * 256 / (N / 4)) workgroups
-// per (b, h), each one partial sum.
+// State rows per thread: two, as in ssm_m2_state_update, and one for d_state 16 (the session
+// presets: 64 rows fill a workgroup). A (b, h) state takes P / (rows * 256 / (N / 4)) workgroups,
+// each one partial sum.
+static int m2_gated_rows(int N) { return N == 16 ? 1 : 2; }
 int m2_gated_nssq(int H, int P, int N) {
     const int rpp = 256 / (N / 4);
-    return H * (int)cdiv(P, rpp * 2);
+    return H * (int)cdiv(P, rpp * m2_gated_rows(N));
 }
 
 ssm_status launch_m2_update_gated(const float* x, long ldx, const float* dt, long lddt,
@@ -1281,17 +1283,18 @@ ssm_status launch_m2_update_gated(const float* x, long ldx, const float* dt, lon
                                   int B, int H, int Pd, int G, int N, hipStream_t st) {
     SSM_REQUIRE(x && dt && A && Bm && Cm && z && gn && y && ssq && h, "m2_update_gated: null");
     SSM_REQUIRE((H * Pd) % 16 == 0, "m2_update_gated: d_inner %d not a multiple of 16", H * Pd);
-    SSM_REQUIRE(N == 64 || N == 128 || N == 256, "m2_update_gated: d_state %d", N);
+    SSM_REQUIRE(N == 16 || N == 32 || N == 64 || N == 128 || N == 256,
+                "m2_update_gated: d_state %d", N);
     SSM_REQUIRE(ldb % 4 == 0 && ldc % 4 == 0 && (uintptr_t)Bm % 16 == 0 &&
                     (uintptr_t)Cm % 16 == 0 && (uintptr_t)h % 16 == 0,
                 "m2_update_gated: B/C/state must be 16-byte aligned");
     if (B == 0) return SSM_OK;
-    constexpr int R = 2;
+    const int R = m2_gated_rows(N);
     const int lpr = N / 4, rpp = 256 / lpr;
     const int bph = (int)cdiv(Pd, rpp * R);
     const unsigned grid = (unsigned)((long)B * H * bph);
     const bool full = Pd % (rpp * R) == 0;
-#define M2G(LPR)                                                                            \
+#define M2G(LPR, R)                                                                         \
     (full ? m2_update_kernel<LPR, R, true, true><<<grid, 256, 0, st>>>(                    \
                 x, ldx, dt, lddt, dt_bias, 1, 0.f, INFINITY, A, Bm, ldb, Cm, ldc, Dsk, z,    \
                 ldz, gn, ssq, y, 0, h, H, Pd, G, N, bph)                                    \
@@ -1299,9 +1302,11 @@ ssm_status launch_m2_update_gated(const float* x, long ldx, const float* dt, lon
                 x, ldx, dt, lddt, dt_bias, 1, 0.f, INFINITY, A, Bm, ldb, Cm, ldc, Dsk, z,    \
                 ldz, gn, ssq, y, 0, h, H, Pd, G, N, bph))
     switch (lpr) {
-        case 16: M2G(16); break;
-        case 32: M2G(32); break;
-        default: M2G(64); break;
+        case 4: M2G(4, 1); break;
+        case 8: M2G(8, 2); break;
+        case 16: M2G(16, 2); break;
+        case 32: M2G(32, 2); break;
+        default: M2G(64, 2); break;
     }
 #undef M2G
     return check_launch("m2_update_gated");
