@@ -1270,8 +1270,9 @@ size_t chunked_workspace(int B, int L, int D, int N) {
 
 extern "C" size_t ssm_selective_scan_workspace(int B, int L, int D, int N) {
     if (B <= 0 || L <= 0 || D <= 0 || N <= 0 || N > 64) return 0;
-    // the single pass and the time-sliced walk need none
-    if (use_single(B, L, D, pad_n(N)) || use_t16(B, L, D, N)) return 0;
+    // (the time-sliced walk touches none, but takes its shapes from the chunked passes only where
+    // the row strides suit it, so longer sequences come with the chunked passes' workspace)
+    if (use_single(B, L, D, pad_n(N))) return 0;
     return chunked_workspace(B, L, D, N);
 }
 
@@ -1303,13 +1304,12 @@ ssm_status selective_scan(const float* u, long ldu, const float* dt, long lddt,
     }
     const int Np = pad_n(N);
     const long ldmax = std::max({ldu, lddt, ldy, z ? ldz : 0L, ldb, ldc});
-    const bool t16 = use_t16(B, L, D, N);
+    const bool t16 = use_t16(B, L, D, N) && rows_fit(std::min<long>(L, 256), ldmax, D);
     const bool single = use_single(B, L, D, Np);
-    const long rows = t16 ? std::min<long>(L, 256) : single ? std::min<long>(L, 128)
-                                                            : pick_chunk(B, L, D);
+    const long rows = single ? std::min<long>(L, 128) : pick_chunk(B, L, D);
     SSM_REQUIRE(rows_fit(rows, ldmax, D),
                 "ssm_selective_scan: row stride %ld too large for 32-bit block offsets", ldmax);
-    const size_t need = t16 || single ? 0 : chunked_workspace(B, L, D, N);
+    const size_t need = single ? 0 : chunked_workspace(B, L, D, N);
     SSM_REQUIRE(need == 0 || (workspace && workspace_bytes >= need),
                 "ssm_selective_scan: workspace of %zu bytes needed", need);
     ScanArgs a;
