@@ -17,6 +17,8 @@ from . import _lib
 from .backend import sample_supported  # noqa: F401  (re-export)
 
 _NULL = None
+_device = getattr(torch._C, "_cuda_getDevice", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _p(t):
@@ -29,7 +31,16 @@ def _p(t):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current device's current stream, without a Stream object around it (1 us of
+    each call)."""
+    return _raw_stream(_device())
+
+
+def _scratch(nbytes, device):
+    """A call's workspace as (tensor or None, bytes): shapes that need none pay no allocation."""
+    if nbytes == 0:
+        return None, 0
+    return torch.empty(nbytes, device=device, dtype=torch.uint8), nbytes
 
 
 def _rows(t, width):
@@ -38,6 +49,14 @@ def _rows(t, width):
     if t.stride(-1) != 1:
         raise ValueError("last dimension must be contiguous")
     return t.stride(-2) if t.dim() >= 2 else width
+
+
+def _seq_ld(t):
+    """Row stride of a (B,L,X) view whose sequences follow one another."""
+    s = t.stride()
+    if len(s) == 3 and s[0] != t.shape[1] * s[1] and t.shape[1] > 1:
+        raise ValueError("row-strided (B,L,X) views only")
+    return s[1]
 
 
 def _f32(t):
@@ -51,9 +70,9 @@ def causal_conv1d(x, w, bias=None, silu=True, state_in=None, state_out=None, out
     K = w.shape[1]
     _f32(x)
     y = out if out is not None else torch.empty(B, L, Cc, device=x.device, dtype=torch.float32)
-    if x.stride(2) != 1 or (L > 1 and x.stride(0) != L * x.stride(1)):
+    sb, ldx, sc = x.stride()
+    if sc != 1 or (L > 1 and sb != L * ldx):
         raise ValueError("x must be a row-strided (B,L,C) view")
-    ldx = x.stride(1)
     _lib.call("ssm_causal_conv1d", _p(x), ldx, _p(w.contiguous()), _p(bias), _p(y), y.stride(1),
               B, L, Cc, K, int(silu), _p(state_in), _p(state_out), _stream())
     return y
@@ -72,15 +91,11 @@ def selective_scan(u, dt, A, Bm, Cm, D=None, z=None, dt_bias=None, softplus=True
     B, L, Dd = u.shape
     N = A.shape[1]
     y = out if out is not None else torch.empty(B, L, Dd, device=u.device, dtype=torch.float32)
-    nbytes = _lib.lib().ssm_selective_scan_workspace(B, L, Dd, N)
-    ws = torch.empty(max(nbytes, 4), device=u.device, dtype=torch.uint8)
-    for t in (u, dt, Bm, Cm, z):
-        if t is not None and t.dim() == 3 and t.shape[1] > 1 and t.stride(0) != t.shape[1] * t.stride(1):
-            raise ValueError("row-strided (B,L,X) views only")
-    _lib.call("ssm_selective_scan", _p(u), u.stride(1), _p(dt), dt.stride(1), _p(dt_bias),
-              int(softplus), _p(A.contiguous()), _p(Bm), Bm.stride(1), _p(Cm), Cm.stride(1),
-              _p(D), _p(z), z.stride(1) if z is not None else 0, _p(y), y.stride(1), B, L, Dd, N,
-              _p(h0), _p(hT), _p(ws), ws.numel(), _stream())
+    ws, nbytes = _scratch(_lib.lib().ssm_selective_scan_workspace(B, L, Dd, N), u.device)
+    _lib.call("ssm_selective_scan", _p(u), _seq_ld(u), _p(dt), _seq_ld(dt), _p(dt_bias),
+              int(softplus), _p(A.contiguous()), _p(Bm), _seq_ld(Bm), _p(Cm), _seq_ld(Cm),
+              _p(D), _p(z), _seq_ld(z) if z is not None else 0, _p(y), y.stride(1), B, L, Dd, N,
+              _p(h0), _p(hT), _p(ws), nbytes, _stream())
     return y
 
 
@@ -114,12 +129,15 @@ def ssd_chunk_scan(x, dt, A, Bm, Cm, D=None, dt_bias=None, softplus=True, dt_min
     if Bm.dtype != x.dtype or Cm.dtype != x.dtype:
         raise TypeError("x, B and C must share a dtype")
     y = out if out is not None else torch.empty(B, L, H, P, device=x.device, dtype=torch.float32)
-    ws = workspace if workspace is not None else ssd_workspace(B, L, H, P, G, N, x.device)
+    if workspace is not None:
+        ws, nbytes = workspace, workspace.numel()
+    else:
+        ws, nbytes = _scratch(_lib.lib().ssm_ssd_workspace(B, L, H, P, G, N), x.device)
     ldx = x.stride(1)
     _lib.call("ssm_ssd_chunk_scan", dtype, _p(x), ldx, _p(dt), dt.stride(1), _p(dt_bias),
               int(softplus), float(dt_min), float(dt_max), _p(A), _p(Bm), Bm.stride(1), _p(Cm),
               Cm.stride(1), _p(D), _p(y), y.stride(1), B, L, H, P, G, N, _p(h0), _p(hT), _p(ws),
-              ws.numel(), _stream())
+              nbytes, _stream())
     return y
 
 
