@@ -69,7 +69,8 @@ struct F32Args {
     const float* Dsk;
     float* y; long ldy;
     int B, L, H, G;     // H counts 64-row heads: P / 64 of them per head of the call
-    int hs;             // P / 64: head h reads dt, A, dt_bias and D of h / hs
+    int hs;             // P / 64: head h reads dt, A, dt_bias and D of h / hs (call_head)
+    unsigned hs_inv;    // ceil(2^32 / hs), 0 for hs = 1
     int nchunks, nseg, chunks_per_seg;
     const float* h0;
     float* hT;
@@ -86,6 +87,11 @@ struct F32Args {
     float* ssq;
 };
 
+// h / hs by its reciprocal (exact for h hs < 2^32; four integer divisions per workgroup before).
+__device__ __forceinline__ int call_head(const F32Args& a, int h) {
+    return a.hs_inv ? (int)__umulhi((unsigned)h, a.hs_inv) : h;
+}
+
 template <int NN, bool FULL, bool GATED, int HPW>
 struct SmemF32 {
     static constexpr int BP = NN + 4;    // B / C row pitch (floats): b128 rows conflict-free
@@ -94,11 +100,12 @@ struct SmemF32 {
     float c[FULL ? 2 : 1][FULL ? QF : 1][BP];            // C (i, n), two chunks
     float m[HPW][FULL ? QF : 1][MP];                     // M^T (i, j) per head
     float ac[2][HPW][QF];    // acum_t in log2 units
-    float al[NN <= 32 ? 2 : 1][HPW][NN <= 32 ? QF : 1];   // d_state <= 32: its low part
     float dv[2][HPW][QF];    // dt'_t
     float wj[2][HPW][QF];    // w_t = 2^(acum_end - acum_t) dt'_t
     float ae[2][HPW];        // acum_end
     float sq[GATED ? 2 : 1][HPW][GATED ? 4 : 1][GATED ? QF : 1];   // per-wave sums of u^2 per row
+    // d_state <= 32: the low part of ac
+    alignas(16) float al[NN <= 32 ? 2 : 1][HPW][NN <= 32 ? QF : 1];
 };
 
 using ssm::bload16;
@@ -190,7 +197,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     const int h = h0w + hw;
     const int bh = b * a.H + h;
     const int g = h / (a.H / a.G);
-    const int hp = h / a.hs;             // head of the call
+    const int hp = call_head(a, h);      // head of the call
     const int l16 = lane & 15, q4 = lane >> 4;
     const int p0 = 16 * wl;
     const int sr = tid / RL, sc4 = 4 * (tid % RL);   // staging row / column
@@ -200,7 +207,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     const float dtb = a.dt_bias ? a.dt_bias[hp] : 0.f;
     float Dh[HPW];   // D of the workgroup's heads (the C B^T tiles serve them all)
 #pragma unroll
-    for (int k = 0; k < HPW; ++k) Dh[k] = a.Dsk ? a.Dsk[(h0w + k) / a.hs] : 0.f;
+    for (int k = 0; k < HPW; ++k) Dh[k] = a.Dsk ? a.Dsk[call_head(a, h0w + k)] : 0.f;
     // gated output: this lane's four norm weights (columns p0 + 4 q4 .. + 3 of the head)
     float4 gw = make_float4(0.f, 0.f, 0.f, 0.f);
     if constexpr (GATED) gw = *reinterpret_cast<const float4*>(a.gn + (long)h * PF + p0 + 4 * q4);
@@ -786,6 +793,7 @@ ssm_status ssd_f32(const float* x, long ldx, const float* dt, long lddt, const f
                    long ldz, const float* gn, float* ssq) {
     F32Args a{};
     a.hs = Pd / PF;
+    a.hs_inv = a.hs > 1 ? (unsigned)(((1ull << 32) + a.hs - 1) / a.hs) : 0u;
     H *= a.hs;
     a.z = z; a.ldz = ldz; a.gn = gn; a.ssq = ssq;
     if (ssq) {
