@@ -139,8 +139,9 @@ ssm_status ssm_m1_state_update(const float* x, long ldx, const float* dt, long l
  *   S_t = exp(dt'_t A_h) S_{t-1} + dt'_t x_t B_t^T  (P x N);  y_t = S_t C_t + Dsk_h x_t.
  * x: (B,L,H,P) elements of `in_dtype` with row stride ldx; dt: (B,L,H) float, row stride
  * lddt; Bm, Cm: (B,L,G,N) of `in_dtype`, row strides ldb/ldc; y: (B,L,H,P) float, ldy;
- * h0/hT: (B,H,P,N) float (may be NULL). P = 64 with N in {64, 128} runs the fused MFMA
- * kernel. Other shapes: with G = 1, N <= 64, float inputs, a dt clamp that cannot bind and
+ * h0/hT: (B,H,P,N) float (may be NULL; hT may alias h0). P = 64 with N in {64, 128} runs the
+ * fused MFMA kernel; so do float inputs with P a multiple of 64 and N in {16, 32, 64, 128} when
+ * all rows are 16-byte aligned and the workspace is given. Other shapes: with G = 1, N <= 64, float inputs, a dt clamp that cannot bind and
  * the workspace, the Mamba-1 chunked scan over H*P channels; otherwise a sequential kernel
  * (no workspace needed). The chunk length of the reference config (chunkLen) does not change
  * the result; the kernel uses its own internal chunk. `workspace` holds

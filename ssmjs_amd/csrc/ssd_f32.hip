@@ -300,14 +300,27 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     // entering state: S^T tile nb holds S[p0 + l16][16 nb + 4 q4 + r] in register r. With
     // NN <= 32 a segment's entering state is formed here from the local states and decays of
     // the segments before it (a few float4 per lane from L2, loaded ahead of the chain);
-    // larger states come combined from ssd_f32_seg_prefix.
+    // larger states come combined from ssd_f32_seg_prefix. The chain starts from the state pass's
+    // copy of h0, in the last segment's slot (which has no local state): the final state may be
+    // written in place of h0 while other segments still start.
     constexpr bool CHAIN = FULL && NN <= 32;
     const float* init = nullptr;
     if (FULL) {
-        if (a.nseg > 1 && !CHAIN) init = a.seg_state + ((long)bh * a.nseg + seg) * PF * NN;
+        const int slot = CHAIN ? a.nseg - 1 : seg;
+        if (a.nseg > 1 && (!CHAIN || a.h0)) init = a.seg_state + ((long)bh * a.nseg + slot) * PF * NN;
         else if (a.h0) init = a.h0 + (long)bh * PF * NN;
     }
     const long lane_off = (long)(p0 + l16) * NN + 4 * q4;
+    if constexpr (!FULL && NN <= 32) {
+        if (a.h0 && seg == 0) {
+            const float* from = a.h0 + (long)bh * PF * NN + lane_off;
+            float* to = a.seg_state + ((long)bh * a.nseg + a.nseg - 1) * PF * NN + lane_off;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+                *reinterpret_cast<float4*>(to + 16 * nb) =
+                    *reinterpret_cast<const float4*>(from + 16 * nb);
+        }
+    }
     floatx4 S[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {

@@ -116,3 +116,19 @@ def test_fast_decay_keeps_precision(B, L, H, N, P):
         rel = np.linalg.norm(got.cpu().numpy() - want) / np.linalg.norm(want)
         print(f"  {what}: relative 2-norm {rel:.2e}", flush=True)
         assert rel <= 6e-7
+
+
+@pytest.mark.parametrize("B,L,H,N,P", [(1, 33, 2, 16, 64), (1, 2000, 12, 16, 128),
+                                       (4, 3000, 9, 32, 128)])
+def test_state_in_place(B, L, H, N, P):
+    """hT in the place of h0 (a session's state, as the mixer calls it): the same bits as with two
+    buffers, though the last segment's workgroup may end before another segment's starts."""
+    print(f"[case] ssd state in place B={B} L={L} H={H} N={N} P={P}", flush=True)
+    from ssmjs_amd import kernels
+    t = [torch.from_numpy(a).cuda() for a in inputs(L, B, L, H, P, 1, N)]
+    hT = torch.empty_like(t[6])
+    y = kernels.ssd_chunk_scan(*t[:6], h0=t[6], hT=hT)
+    state = t[6].clone()
+    y2 = kernels.ssd_chunk_scan(*t[:6], h0=state, hT=state)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2) and torch.equal(hT, state)
