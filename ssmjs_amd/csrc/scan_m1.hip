@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kWave) void scan_chunk_state(
 template <int kPreW, int kPer>
 __global__ __launch_bounds__(64 * kPreW) void scan_chunk_prefix(
     const float* __restrict__ A, int D, int N, int NC, float* __restrict__ hc,
-    const float* __restrict__ sdt, const float* __restrict__ h0, float* __restrict__ hT) {
+    const float* __restrict__ sdt, const float* h0, float* hT) {   // (hT may be h0)
     __shared__ float2 seg[2][kPreW][64];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -155,7 +155,9 @@ __global__ __launch_bounds__(64 * kPreW) void scan_chunk_prefix(
             P *= av[u];
         }
         seg[buf][w][lane] = make_float2(P, H);
-        __syncthreads();   // (also: every wave's loads of the round are done before its stores)
+        // every wave's loads (h0's too) are done before any wave's stores
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+        __syncthreads();
         float e = carry;
 #pragma unroll
         for (int v = 0; v < kPreW; ++v) {

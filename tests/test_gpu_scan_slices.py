@@ -54,3 +54,20 @@ def test_matches_oracle(B, L, D, opts):
         torch.cuda.synchronize()
         ref = O.selective_scan(u, dt, A, Bm, Cm, None, None, None, False)
     close(y, ref, "y")
+
+
+@pytest.mark.parametrize("B,L,D", [(1, 300, 130),     # time slices
+                                   (1, 1100, 70), (2, 2047, 600), (1, 8192, 256)])   # chunks
+def test_state_in_place(B, L, D):
+    """hT in the place of h0 (a session's state): the same bits as with two buffers."""
+    print(f"[case] scan state in place B={B} L={L} D={D}", flush=True)
+    from ssmjs_amd import kernels
+    r = np.random.default_rng(L)
+    dev = lambda *s: torch.from_numpy(r.standard_normal(s).astype(np.float32)).cuda()   # noqa: E731
+    u, dt, Bm, Cm, h0 = dev(B, L, D), dev(B, L, D) - 1, dev(B, L, 16), dev(B, L, 16), dev(B, D, 16)
+    A = -dev(D, 16).abs()
+    hT, state = torch.empty_like(h0), h0.clone()
+    y = kernels.selective_scan(u, dt, A, Bm, Cm, h0=h0, hT=hT)
+    y2 = kernels.selective_scan(u, dt, A, Bm, Cm, h0=state, hT=state)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2) and torch.equal(hT, state)
