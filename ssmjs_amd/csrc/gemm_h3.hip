@@ -315,6 +315,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
             compute(s3);
         }
     }
+    // the loads past the last block end before the LDS they write is given back
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
 
     if constexpr (RS) {
         for (int r = threadIdx.x; r < BM; r += 64 * NW) {
