@@ -52,7 +52,11 @@ import sys
 import time
 
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, GB/s
-PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0}   # dense MFMA, TFLOP/s
+# dense MFMA, TFLOP/s; f32x3: fp32-precision products as three fp16 MFMAs each (gemm_h3.hip,
+# stepproj.hip), a third of the fp16 peak
+PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0, "f32x3": 2500.0 / 3}
+SPLIT_STAGES = {"m1.in_proj", "m1.x_proj", "m1.out_proj", "m2.in_proj", "m2.out_proj",
+                "m1.step.in_proj", "m1.step.out_proj", "m2.step.in_proj", "m2.step.out_proj"}
 
 METRIC = "SSM tokens/s on 1×MI355X (prefill + decode) + % of HBM/MFMA roofline"
 
@@ -63,11 +67,9 @@ METRIC = "SSM tokens/s on 1×MI355X (prefill + decode) + % of HBM/MFMA roofline"
 # read 1.0000 GiB each way). The commands and per-kernel counts sit with the rocprof summaries
 # in profiles/. Re-measured when the kernels change; None where not measured.
 TRAFFIC = {
-    ("cfg2", "m1.in_proj"): 345_239_515,               # gemm_f32_kernel<4>
     ("cfg2", "m1.conv"): 103_171_772,                  # conv1d_fwd
     ("cfg2", "m1.x_dt_proj"): 111_457_347,             # xproj_dt_kernel
     ("cfg2", "m1.scan"): 205_006_791,                  # scan_w16_kernel
-    ("cfg2", "m1.out_proj"): 159_930_259,              # gemm_f32_kernel<3>
     ("cfg3", "bf16"): 847_398_173,                     # ssd_kernel (two heads per workgroup)
     ("cfg3", "f32"): 1_135_702_044,                    # ssd_f32_kernel (the C B^T pre-pass, ssd_f32_cb_kernel, adds 36.7 MB)
     ("cfg4", "m2.step.state_update"): 136_414_850,     # m2_update_kernel (timed on its own)
@@ -188,6 +190,8 @@ def profiled_stages(dev, torch, fn, steps):
 def roofline(name, avg_ms, flops=None, nbytes=None, prec="f32", bound=None, traffic=None,
              traffic_key=None):
     """Achieved rate of one kernel/stage against its binding peak."""
+    if prec == "f32" and name in SPLIT_STAGES:
+        prec = "f32x3"
     t = avg_ms * 1e-3
     if bound is None:
         ai = flops / nbytes if (flops and nbytes) else 0.0
@@ -557,7 +561,9 @@ def w_cfg3layer(torch, np, dev, args):
         prec = "bf16" if kk.startswith("m2b.") else "f32"
         stages[kk] = roofline(kk, avg, f, b, prec, "hbm" if f is None else None)
     dom = max(stages.values(), key=lambda r: r["avg_ms"])
-    layer_flops = sum(alg[kk][0] for kk in st if alg[kk][0])
+    # the layer's products at their units' peaks, over its time
+    peak_s = sum(alg[kk][0] / (PEAK_TFLOPS["bf16" if bf else "f32x3" if kk in SPLIT_STAGES
+                                           else "f32"] * 1e12) for kk in st if alg[kk][0])
     out = {"value": T / (ms * 1e-3), "ms_per_step": ms, "steps": steps, "warmup": warm,
            "dtype": "bf16" if bf else "f32",
            "config": {"workload": "cfg3 layer: Mamba-2 layer prefill (in_proj, conv1d+SiLU over "
@@ -566,8 +572,7 @@ def w_cfg3layer(torch, np, dev, args):
                       "batch": B, "seq_len": L, "d_model": d, "heads": H, "head_dim": P,
                       "d_state": N, "groups": 1, "tokens_per_step": T},
            "roofline": dom, "stages": stages,
-           "layer_mfma_frac": round(layer_flops / (ms * 1e-3) / 1e12
-                                    / PEAK_TFLOPS["bf16" if bf else "f32"], 4)}
+           "layer_mfma_frac": round(peak_s / (ms * 1e-3), 4)}
     m.destroy()
     return out
 
