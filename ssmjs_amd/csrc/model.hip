@@ -663,24 +663,32 @@ ssm_status build_wh(ssm_model* m) {
         }
         SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh, off ? (size_t)off : 1));
     }
-    for (int l = 0; l < d.nl; ++l) {
+    auto pack = [&](long at, long w, int rows, int K) {
+        return at < 0 ? SSM_OK : ssm::launch_pack_h3(m->w + w, K, rows, K, m->wh + at, st);
+    };
+    ssm_status e = SSM_OK;
+    for (int l = 0; l < d.nl && e == SSM_OK; ++l) {
         const LayerW& Ly = m->layers[l];
         const bool m1 = Ly.type == SSM_LAYER_MAMBA1;
-        if (m->wh_in[l] >= 0)
-            SSM_TRY(ssm::launch_pack_h3(m->w + Ly.in_proj, d.d, m1 ? 2 * d.D : d.nin, d.d,
-                                        m->wh + m->wh_in[l], st));
-        if (m->wh_out[l] >= 0)
-            SSM_TRY(ssm::launch_pack_h3(m->w + Ly.out_proj, d.D, d.d, d.D, m->wh + m->wh_out[l],
-                                        st));
-        if (m->wh_x[l] >= 0)
-            SSM_TRY(ssm::launch_pack_h3(m->w + Ly.x_proj, d.D, RN, d.D, m->wh + m->wh_x[l], st));
+        e = pack(m->wh_in[l], Ly.in_proj, m1 ? 2 * d.D : d.nin, d.d);
+        if (e == SSM_OK) e = pack(m->wh_out[l], Ly.out_proj, d.d, d.D);
+        if (e == SSM_OK) e = pack(m->wh_x[l], Ly.x_proj, RN, d.D);
     }
-    return SSM_OK;
+    if (e != SSM_OK) {   // no half-packed copies: the next call builds them anew
+        hipFree(m->wh);
+        m->wh = nullptr;
+    }
+    return e;
 }
 ssm_status build_wh_emb(ssm_model* m) {
     const Dims& d = m->dm;
     if (!m->wh_emb) SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh_emb, ssm::h3_bytes(d.V, d.d)));
-    return ssm::launch_pack_h3(m->w + m->emb, d.d, d.V, d.d, m->wh_emb, m->ctx->stream);
+    const ssm_status e = ssm::launch_pack_h3(m->w + m->emb, d.d, d.V, d.d, m->wh_emb, m->ctx->stream);
+    if (e != SSM_OK) {
+        hipFree(m->wh_emb);
+        m->wh_emb = nullptr;
+    }
+    return e;
 }
 
 // bf16 (round to nearest even) copies of the Mamba-2 layers' in_proj and out_proj.

@@ -91,6 +91,30 @@ def test_launch_failure_then_recovery(device, inject):
     m.destroy()
 
 
+def test_failed_weight_packing_is_built_anew(device, inject):
+    """A launch failure while the projections' packed weights are built (the first mixer call of
+    more than 64 rows): the next call packs them from the start."""
+    case("injected fault: launch, weight packing")
+    from ssmjs_amd import _lib, backend
+    m = backend.Model(device, CFG, seed=2)
+    om = O.Model(m.export_weights())
+    d = CFG["dModel"]
+    x = np.random.default_rng(0).standard_normal((1, 90, d)).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    y = torch.empty_like(xd)
+    torch.cuda.synchronize()
+    args = ("ssm_mixer_forward_device", m.handle, 0, xd.data_ptr(), y.data_ptr(), 1, 90)
+    inject("launch")
+    with pytest.raises(_lib.SsmError):
+        _lib.call(*args)
+    inject(None)
+    _lib.call(*args)
+    device.synchronize()
+    ref = om.mixer(0, x)
+    assert np.abs(y.cpu().numpy() - ref).max() <= 1e-4 * np.abs(ref).max()
+    m.destroy()
+
+
 def test_session_create_reports_model_failure(inject):
     """MambaSession.create with every allocation failing: the device opens (no allocation), the
     model construction fails and the session raises SessionError('UNKNOWN') as session.ts
