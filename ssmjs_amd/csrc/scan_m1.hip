@@ -843,16 +843,21 @@ __global__ __launch_bounds__(64 * W) void scan_t16_kernel(ScanArgs a) {
          sc = span(a.Cm, a.ldc, 16), sy = span(a.y, a.ldy, D);
     const unsigned t = 16u * w + j;      // this lane's step within a block, as an input lane
     const unsigned tb = 16u * w + c;     // B / C: lane (c, n) loads steps 4 i + c of the slice
-    const unsigned du_ = (unsigned)d * 4u;
-    const unsigned ou = (t * (unsigned)a.ldu * 4u + du_) | dmask,
-                   od = (t * (unsigned)a.lddt * 4u + du_) | dmask,
-                   oz = (t * (unsigned)sz.ld * 4u + du_) | dmask,
-                   oy = (t * (unsigned)a.ldy * 4u + du_) | dmask;
+    // Steps past a sequence shorter than a block are out of range by their own bit: the host
+    // checks that min(L, 256) rows fit 32-bit offsets, and a later row's offset may wrap into the
+    // descriptor's range.
+    auto past = [&](unsigned step) { return step < (unsigned)L ? 0u : 0x80000000u; };
+    const unsigned du_ = (unsigned)d * 4u, tmask = dmask | past(t);
+    const unsigned ou = (t * (unsigned)a.ldu * 4u + du_) | tmask,
+                   od = (t * (unsigned)a.lddt * 4u + du_) | tmask,
+                   oz = (t * (unsigned)sz.ld * 4u + du_) | tmask,
+                   oy = (t * (unsigned)a.ldy * 4u + du_) | tmask;
     unsigned ob[4], oc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        ob[i] = ((tb + 4u * i) * (unsigned)a.ldb + (unsigned)j) * 4u;
-        oc[i] = ((tb + 4u * i) * (unsigned)a.ldc + (unsigned)j) * 4u;
+        const unsigned ti = tb + 4u * i;
+        ob[i] = ((ti * (unsigned)a.ldb + (unsigned)j) * 4u) | past(ti);
+        oc[i] = ((ti * (unsigned)a.ldc + (unsigned)j) * 4u) | past(ti);
     }
     float uv, dv, zv, bv[4], cv[4];
     auto load = [&](int rows) {          // the block at the spans' bases, which then advance
