@@ -335,6 +335,14 @@ struct Scan1 {
     };
 };
 
+// Out-of-range bit of a block's step: set past a sequence shorter than the block. The host checks
+// that the sequence's own rows fit 32-bit offsets; a later step's offset may wrap into the
+// descriptor's range. (Constant over a sequence's blocks: a longer one has whole blocks' rows
+// checked, and its last block ends at the descriptor's range.)
+__device__ __forceinline__ unsigned past_row(unsigned step, int L) {
+    return step < (unsigned)L ? 0u : 0x80000000u;
+}
+
 // Value of lane j of this lane's 16-lane row (DPP row_newbcast); as an operand of a VALU
 // instruction the compiler folds it into that instruction.
 template <int J>
@@ -403,16 +411,17 @@ __global__ __launch_bounds__(64 * Scan1<N>::W) void scan_single_kernel(ScanArgs 
 #pragma unroll
         for (int e = 0; e < UE; ++e) {
             const unsigned t = (unsigned)(st0 + e * SR);
-            uv[e] = ssm::bload4(ru, (t * (unsigned)a.ldu + (unsigned)sd) * 4u);
-            dv[e] = ssm::bload4(rd, (t * (unsigned)a.lddt + (unsigned)sd) * 4u);
-            zv[e] = ssm::bload4(rz, (t * (unsigned)ldz + (unsigned)sd) * 4u);
+            const unsigned pm = past_row(t, L);
+            uv[e] = ssm::bload4(ru, (t * (unsigned)a.ldu + (unsigned)sd) * 4u | pm);
+            dv[e] = ssm::bload4(rd, (t * (unsigned)a.lddt + (unsigned)sd) * 4u | pm);
+            zv[e] = ssm::bload4(rz, (t * (unsigned)ldz + (unsigned)sd) * 4u | pm);
         }
 #pragma unroll
         for (int j = 0; j < BE; ++j) {
             const int i = (tid + NT * j) % (TK * N), nn = i % N;
-            const unsigned t = (unsigned)(i / N);
-            bv[j] = ssm::bload4(rb, (t * (unsigned)a.ldb + (unsigned)nn) * 4u);
-            cv[j] = ssm::bload4(rc, (t * (unsigned)a.ldc + (unsigned)nn) * 4u);
+            const unsigned t = (unsigned)(i / N), pm = past_row(t, L);
+            bv[j] = ssm::bload4(rb, (t * (unsigned)a.ldb + (unsigned)nn) * 4u | pm);
+            cv[j] = ssm::bload4(rc, (t * (unsigned)a.ldc + (unsigned)nn) * 4u | pm);
         }
     };
 
@@ -500,7 +509,7 @@ __global__ __launch_bounds__(64 * Scan1<N>::W) void scan_single_kernel(ScanArgs 
             // rows past L fall outside the descriptor (dropped); so does a channel past D
             const int st = st0 + e * SR;
             const unsigned off = ((unsigned)st * (unsigned)a.ldy + (unsigned)sd) * 4u;
-            ssm::bstore4(sm.ys[st][sc], ry, off | (sdok ? 0u : 0x80000000u));
+            ssm::bstore4(sm.ys[st][sc], ry, off | (sdok ? 0u : 0x80000000u) | past_row(st, L));
         }
     }
     if (live && a.hT) a.hT[((long)b * D + d) * Nr + n] = h;
@@ -605,18 +614,19 @@ __global__ __launch_bounds__(64 * W) void scan_w16_kernel(ScanArgs a) {
         for (int e = 0; e < UE; ++e) {
             const int i = st + NST * e;
             const unsigned t = (unsigned)(i / CW), sd = (unsigned)min(c0 + i % CW, D - 1);
-            uv[e] = ssm::bload4(ru, (t * (unsigned)a.ldu + sd) * 4u);
-            dv[e] = ssm::bload4(rd, (t * (unsigned)a.lddt + sd) * 4u);
-            zv[e] = ssm::bload4(rz, (t * (unsigned)a.ldz + sd) * 4u);
+            const unsigned pm = past_row(t, L);
+            uv[e] = ssm::bload4(ru, (t * (unsigned)a.ldu + sd) * 4u | pm);
+            dv[e] = ssm::bload4(rd, (t * (unsigned)a.lddt + sd) * 4u | pm);
+            zv[e] = ssm::bload4(rz, (t * (unsigned)a.ldz + sd) * 4u | pm);
         }
 #pragma unroll
         for (int e = 0; e < BE; ++e) {
             // value i = step i / 16, state i % 16; threads past the block's values repeat the
             // first ones (the same value to the same place)
             const int i = (st + NST * e) % (TK * 16);
-            const unsigned t = (unsigned)(i >> 4), nn = (unsigned)(i & 15);
-            bv[e] = ssm::bload4(rb, (t * (unsigned)a.ldb + nn) * 4u);
-            cv[e] = ssm::bload4(rc, (t * (unsigned)a.ldc + nn) * 4u);
+            const unsigned t = (unsigned)(i >> 4), nn = (unsigned)(i & 15), pm = past_row(t, L);
+            bv[e] = ssm::bload4(rb, (t * (unsigned)a.ldb + nn) * 4u | pm);
+            cv[e] = ssm::bload4(rc, (t * (unsigned)a.ldc + nn) * 4u | pm);
         }
     };
     auto stage = [&](int k, int buf) {
@@ -683,7 +693,8 @@ __global__ __launch_bounds__(64 * W) void scan_w16_kernel(ScanArgs a) {
             const float kk = x1 ? r1s : r0s, ss = x1 ? r0s : r1s;
             const float ysum = kk + quad_xor<1>(ss);
             ssm::bstore4((ysum + dx) * gz, ry,
-                         (((unsigned)(16 * s + j) * (unsigned)a.ldy + (unsigned)d) * 4u) | dmask);
+                         (((unsigned)(16 * s + j) * (unsigned)a.ldy + (unsigned)d) * 4u) | dmask |
+                             past_row(16 * s + j, L));
         };
         read_in(0, in, bq);
         float gzp = 0.f, dxp = 0.f;
@@ -843,11 +854,7 @@ __global__ __launch_bounds__(64 * W) void scan_t16_kernel(ScanArgs a) {
          sc = span(a.Cm, a.ldc, 16), sy = span(a.y, a.ldy, D);
     const unsigned t = 16u * w + j;      // this lane's step within a block, as an input lane
     const unsigned tb = 16u * w + c;     // B / C: lane (c, n) loads steps 4 i + c of the slice
-    // Steps past a sequence shorter than a block are out of range by their own bit: the host
-    // checks that min(L, 256) rows fit 32-bit offsets, and a later row's offset may wrap into the
-    // descriptor's range.
-    auto past = [&](unsigned step) { return step < (unsigned)L ? 0u : 0x80000000u; };
-    const unsigned du_ = (unsigned)d * 4u, tmask = dmask | past(t);
+    const unsigned du_ = (unsigned)d * 4u, tmask = dmask | past_row(t, L);
     const unsigned ou = (t * (unsigned)a.ldu * 4u + du_) | tmask,
                    od = (t * (unsigned)a.lddt * 4u + du_) | tmask,
                    oz = (t * (unsigned)sz.ld * 4u + du_) | tmask,
@@ -856,8 +863,8 @@ __global__ __launch_bounds__(64 * W) void scan_t16_kernel(ScanArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const unsigned ti = tb + 4u * i;
-        ob[i] = ((ti * (unsigned)a.ldb + (unsigned)j) * 4u) | past(ti);
-        oc[i] = ((ti * (unsigned)a.ldc + (unsigned)j) * 4u) | past(ti);
+        ob[i] = ((ti * (unsigned)a.ldb + (unsigned)j) * 4u) | past_row(ti, L);
+        oc[i] = ((ti * (unsigned)a.ldc + (unsigned)j) * 4u) | past_row(ti, L);
     }
     float uv, dv, zv, bv[4], cv[4];
     auto load = [&](int rows) {          // the block at the spans' bases, which then advance

@@ -73,28 +73,30 @@ def test_state_in_place(B, L, D):
     assert torch.equal(y, y2) and torch.equal(hT, state)
 
 
-@pytest.mark.parametrize("L", [2, 3])
-def test_row_stride_past_the_offset_range(L):
-    """Rows 72 MB apart: step 60 of the 64-step block lies 2^32 bytes and a little on, which 32-bit
+@pytest.mark.parametrize("L,D,N", [(2, 5, 16), (3, 5, 16),                        # time slices
+                                   (2, 4112, 16), (2, 5, 4), (2, 5, 8), (2, 5, 32),   # single pass
+                                   (2, 5, 64)])
+def test_row_stride_past_the_offset_range(L, D, N):
+    """Rows 72 MB apart: step 60 of a 64- or 128-step block lies 2^32 bytes and a little on, which 32-bit
     offsets would bring back between the first two rows. The outputs agree with the oracle, and
     what lies between the rows (NaN) is neither read nor written."""
-    print(f"[case] scan row stride L={L}", flush=True)
+    print(f"[case] scan row stride L={L} D={D} N={N}", flush=True)
     from ssmjs_amd import kernels
-    B, D, ld = 1, 5, 18_000_000
+    B, ld = 1, 18_000_000
     assert 60 * ld * 4 - 2 ** 32 in range(4 * D, 4 * ld)
     r = np.random.default_rng(L)
     f = lambda *s: r.standard_normal(s).astype(np.float32)   # noqa: E731
-    u, Bm, Cm = f(B, L, D), f(B, L, 16), f(B, L, 16)
+    u, Bm, Cm = f(B, L, D), f(B, L, N), f(B, L, N)
     dt = np.abs(f(B, L, D)) * 0.1
-    A = -r.uniform(0.5, 16, (D, 16)).astype(np.float32)
+    A = -r.uniform(0.5, 16, (D, N)).astype(np.float32)
 
     def far(a):
-        buf = torch.full(((L - 1) * ld + 16,), float("nan"), device="cuda")
+        buf = torch.full(((L - 1) * ld + D + 64,), float("nan"), device="cuda")
         v = torch.as_strided(buf, a.shape, (L * ld, ld, 1))
         v.copy_(torch.from_numpy(a))
         return buf, v
     (_, ud), (_, dd), (_, bd), (_, cd), (ybuf, y) = (far(a) for a in (u, dt, Bm, Cm, 0 * u))
-    hT = torch.empty(B, D, 16, device="cuda")
+    hT = torch.empty(B, D, N, device="cuda")
     kernels.selective_scan(ud, dd, torch.from_numpy(A).cuda(), bd, cd, softplus=False, out=y, hT=hT)
     torch.cuda.synchronize()
     ref, ref_h = O.selective_scan(u, dt, A, Bm, Cm, None, None, None, False, return_state=True)
