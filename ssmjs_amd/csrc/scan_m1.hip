@@ -445,9 +445,10 @@ __global__ __launch_bounds__(64 * Scan1<N>::W) void scan_single_kernel(ScanArgs 
             // threads past the block's TK x N values repeat the first ones (the same value to
             // the same place), so no thread branches around its write
             const int i = (tid + NT * j) % (TK * N);
-            const float nm = (EXACT || i % N < Nr) ? 1.f : 0.f;
-            sm.bt[i % N][i / N] = nm * bv[j];
-            sm.ct[i / N][i % N] = nm * cv[j];
+            // (a state past Nr was loaded from what follows the row, which may be inf or NaN)
+            const bool nm = EXACT || i % N < Nr;
+            sm.bt[i % N][i / N] = nm ? bv[j] : 0.f;
+            sm.ct[i / N][i % N] = nm ? cv[j] : 0.f;
         }
         load(k + 1);   // the next block's loads have this whole block to arrive
         __syncthreads();

@@ -75,7 +75,7 @@ def test_state_in_place(B, L, D):
 
 @pytest.mark.parametrize("L,D,N", [(2, 5, 16), (3, 5, 16),                        # time slices
                                    (2, 4112, 16), (2, 5, 4), (2, 5, 8), (2, 5, 32),   # single pass
-                                   (2, 5, 64)])
+                                   (2, 5, 64), (2, 5, 13)])
 def test_row_stride_past_the_offset_range(L, D, N):
     """Rows 72 MB apart: step 60 of a 64- or 128-step block lies 2^32 bytes and a little on, which 32-bit
     offsets would bring back between the first two rows. The outputs agree with the oracle, and
