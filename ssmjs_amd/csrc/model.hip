@@ -516,6 +516,10 @@ struct ssm_model {
     size_t nfloats = 0, nA = 0;
     float* w = nullptr;      // weights in checkpoint payload order
     float* Ab = nullptr;     // A = -exp(A_log), per layer
+    // What is derived from the weights holds the current ones: set after a build's last launch,
+    // cleared before the weights change or a build starts. A copy that lost its flag keeps its
+    // memory (captured steps hold its address) and is built anew before its next use.
+    bool A_ok = false, wp_ok = false, wb_ok = false, wh_ok = false, wh_emb_ok = false;
     // workspace, grown on demand
     char* ws = nullptr;
     size_t ws_bytes = 0;
@@ -643,6 +647,7 @@ ssm_status build_wh(ssm_model* m) {
     const Dims& d = m->dm;
     hipStream_t st = m->ctx->stream;
     const int RN = d.R + 2 * d.N;
+    m->wh_ok = false;
     auto ok = [&](long off, int K) { return K % 4 == 0 && ((uintptr_t)(m->w + off) & 15) == 0; };
     if (!m->wh) {
         m->wh_in.assign(d.nl, -1);
@@ -666,35 +671,30 @@ ssm_status build_wh(ssm_model* m) {
     auto pack = [&](long at, long w, int rows, int K) {
         return at < 0 ? SSM_OK : ssm::launch_pack_h3(m->w + w, K, rows, K, m->wh + at, st);
     };
-    ssm_status e = SSM_OK;
-    for (int l = 0; l < d.nl && e == SSM_OK; ++l) {
+    for (int l = 0; l < d.nl; ++l) {
         const LayerW& Ly = m->layers[l];
         const bool m1 = Ly.type == SSM_LAYER_MAMBA1;
-        e = pack(m->wh_in[l], Ly.in_proj, m1 ? 2 * d.D : d.nin, d.d);
-        if (e == SSM_OK) e = pack(m->wh_out[l], Ly.out_proj, d.d, d.D);
-        if (e == SSM_OK) e = pack(m->wh_x[l], Ly.x_proj, RN, d.D);
+        SSM_TRY(pack(m->wh_in[l], Ly.in_proj, m1 ? 2 * d.D : d.nin, d.d));
+        SSM_TRY(pack(m->wh_out[l], Ly.out_proj, d.d, d.D));
+        SSM_TRY(pack(m->wh_x[l], Ly.x_proj, RN, d.D));
     }
-    if (e != SSM_OK) {   // no half-packed copies: the next call builds them anew
-        hipFree(m->wh);
-        m->wh = nullptr;
-    }
-    return e;
+    m->wh_ok = true;
+    return SSM_OK;
 }
 ssm_status build_wh_emb(ssm_model* m) {
     const Dims& d = m->dm;
+    m->wh_emb_ok = false;
     if (!m->wh_emb) SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh_emb, ssm::h3_bytes(d.V, d.d)));
-    const ssm_status e = ssm::launch_pack_h3(m->w + m->emb, d.d, d.V, d.d, m->wh_emb, m->ctx->stream);
-    if (e != SSM_OK) {
-        hipFree(m->wh_emb);
-        m->wh_emb = nullptr;
-    }
-    return e;
+    SSM_TRY(ssm::launch_pack_h3(m->w + m->emb, d.d, d.V, d.d, m->wh_emb, m->ctx->stream));
+    m->wh_emb_ok = true;
+    return SSM_OK;
 }
 
 // bf16 (round to nearest even) copies of the Mamba-2 layers' in_proj and out_proj.
 ssm_status build_wb(ssm_model* m) {
     const Dims& d = m->dm;
     hipStream_t st = m->ctx->stream;
+    m->wb_ok = false;
     if (!m->wb) {
         m->wb_in.assign(d.nl, -1);
         m->wb_out.assign(d.nl, -1);
@@ -715,20 +715,37 @@ ssm_status build_wb(ssm_model* m) {
         SSM_TRY(ssm::launch_cast_bf16(m->w + Ly.out_proj, d.D, m->wb + m->wb_out[l], d.D, d.d,
                                       d.D, st));
     }
+    m->wb_ok = true;
     return SSM_OK;
 }
 
-// Everything derived from the weights: A = -exp(A_log) and, once built, the packed copies.
-ssm_status refresh_A(ssm_model* m) {
+// Everything derived from the weights, after a change of them: A = -exp(A_log) and, once built,
+// the packed copies.
+void drop_derived(ssm_model* m) {
+    m->A_ok = m->wp_ok = m->wb_ok = m->wh_ok = m->wh_emb_ok = false;
+}
+ssm_status build_A(ssm_model* m) {
     hipStream_t st = m->ctx->stream;
     for (const LayerW& L : m->layers) {
         const long n = L.type == SSM_LAYER_MAMBA1 ? (long)m->dm.D * m->dm.N : m->dm.H;
         SSM_TRY(ssm::launch_neg_exp(m->w + L.A_log, m->Ab + L.A, n, st));
     }
+    m->A_ok = true;
+    return SSM_OK;
+}
+ssm_status refresh_derived(ssm_model* m) {
+    drop_derived(m);
+    SSM_TRY(build_A(m));
     if (m->wb) SSM_TRY(build_wb(m));
     if (m->wh) SSM_TRY(build_wh(m));
     if (m->wh_emb) SSM_TRY(build_wh_emb(m));
     return m->wp ? pack_weights(m) : SSM_OK;
+}
+// Before a call computes with the model: what a failed refresh left behind (A, and the step's
+// copies, which captured steps read without asking).
+ssm_status derived_current(ssm_model* m) {
+    if (!m->A_ok) SSM_TRY(build_A(m));
+    return m->wp && !m->wp_ok ? pack_weights(m) : SSM_OK;
 }
 
 ssm_status random_init(ssm_model* m, uint64_t seed) {
@@ -765,7 +782,7 @@ ssm_status random_init(ssm_model* m, uint64_t seed) {
         }
     }
     SSM_TRY(I(m->norm_f, d.d, SSM_INIT_CONST, 1.f, 0.f));
-    return refresh_A(m);
+    return refresh_derived(m);
 }
 
 // Workspace plan for T = B*L tokens (bytes, 256-aligned carve-outs).
@@ -946,10 +963,10 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
     const float* W = m->w;
     const float* A = m->Ab + Ly.A;
     const bool few = few_rows(T);
-    if (h3_rows(T) && !m->wh) SSM_TRY(build_wh(m));
+    if (h3_rows(T) && !m->wh_ok) SSM_TRY(build_wh(m));
     const long l = &Ly - m->layers.data();
     auto packed = [&](const std::vector<long>& at) -> const void* {
-        return m->wh && at[l] >= 0 ? m->wh + at[l] : nullptr;
+        return m->wh_ok && at[l] >= 0 ? m->wh + at[l] : nullptr;
     };
     const void *Wp_in = packed(m->wh_in), *Wp_out = packed(m->wh_out), *Wp_x = packed(m->wh_x);
     auto proj = [&](int N, int K, const float* X, long ldx, const float* Wt, const void* Wp,
@@ -1059,7 +1076,7 @@ ssm_status mixer_bf16(ssm_model* m, int l, const float* x, float* out, int B, in
     const float* A = m->Ab + Ly.A;
     const int GN = d.G * d.N;
     SSM_REQUIRE(Ly.type == SSM_LAYER_MAMBA2, "bf16 mixer: layer %d is not a Mamba-2 layer", l);
-    if (!m->wb) SSM_TRY(build_wb(m));
+    if (!m->wb_ok) SSM_TRY(build_wb(m));
     __bf16* x16 = (__bf16*)w.hid;        // (T, d)
     float* zx = w.a;                     // (T, nin) fp32
     __bf16* xbc16 = (__bf16*)w.b;        // (T, cd)
@@ -1227,6 +1244,7 @@ bool fused_step_ok(const ssm_model* m, const LayerW& Ly, int B, const Ws& w) {
 ssm_status pack_weights(ssm_model* m) {
     const Dims& d = m->dm;
     hipStream_t st = m->ctx->stream;
+    m->wp_ok = false;
     if (!m->wp) {
         long off = 0;
         m->wp_in.assign(d.nl, -1);
@@ -1289,6 +1307,7 @@ ssm_status pack_weights(ssm_model* m) {
     }
     if (m->wp_emb >= 0)
         SSM_TRY(ssm::launch_pack_step(m->w + m->emb, d.d, d.V, d.d, m->wp + m->wp_emb, st));
+    m->wp_ok = true;
     return SSM_OK;
 }
 
@@ -1430,7 +1449,7 @@ ssm_status trunk(ssm_model* m, const uint32_t* d_ids, int B, int L, ssm_state* s
             const LayerW* nx = l + 1 < d.nl ? &m->layers[l + 1] : nullptr;
             const bool next_fused = nx && fused_step_ok(m, *nx, B, w);
             if (fused_step_ok(m, Ly, B, w)) {
-                if (!m->wp) SSM_TRY(pack_weights(m));   // eager: the first step never replays
+                if (!m->wp_ok) SSM_TRY(pack_weights(m));   // eager: the first step never replays
                 if (!pre)
                     SSM_TRY(ssm::launch_xg_ssq(w.hid, d.d, m->w + Ly.norm, w.xg, w.ssq_in, B, d.d,
                                                st));
@@ -1472,7 +1491,7 @@ ssm_status head_rows(ssm_model* m, const Ws& w, const float* x, long ldx, int ro
                      uint32_t* d_argmax) {
     const Dims& d = m->dm;
     hipStream_t st = m->ctx->stream;
-    if (!m->wp) SSM_TRY(pack_weights(m));
+    if (!m->wp_ok) SSM_TRY(pack_weights(m));
     Stage g(m->ctx, "head");
     SSM_TRY(ssm::launch_xg_ssq(x, ldx, m->w + m->norm_f, w.xg, w.ssq_in, rows, d.d, st));
     return ssm::launch_head(w.xg, w.ssq_in, d.d / 16, 1.f / (float)d.d, d.eps,
@@ -1484,7 +1503,7 @@ ssm_status head_rows(ssm_model* m, const Ws& w, const float* x, long ldx, int ro
 ssm_status head_many(ssm_model* m, const Ws& w, const float* x, int rows, float* lg) {
     const Dims& d = m->dm;
     const float* E = m->w + m->emb;
-    if (h3_rows(rows) && w.xh && d.d % 4 == 0 && !m->wh_emb) SSM_TRY(build_wh_emb(m));
+    if (h3_rows(rows) && w.xh && d.d % 4 == 0 && !m->wh_emb_ok) SSM_TRY(build_wh_emb(m));
     if (h3_product_ok(w, m->wh_emb, rows, d.V, d.d, x, d.d, E, d.V))
         return proj_h3(m, w, rows, d.V, d.d, x, d.d, E, m->wh_emb, lg, d.V, 0.f);
     return gemm(m->ctx, rows, d.V, d.d, x, d.d, E, lg, d.V, 0.f);
@@ -1656,6 +1675,7 @@ extern "C" ssm_status ssm_model_load_weights(ssm_model* m, const void* buf, size
     if (const char* why = ssmw::validate(buf, bytes, ssmw_expect(m, types), &h))
         return ssm::fail(SSM_ERR_CHECKPOINT_INVALID, "%s", why);
     if (h.eps > 0.f) m->dm.eps = h.eps;
+    drop_derived(m);
     if (h.dtype == 0) {
         SSM_HIP_TRY(hipMemcpyAsync(m->w, p + h.header_bytes, m->nfloats * 4,
                                    hipMemcpyHostToDevice, m->ctx->stream));
@@ -1667,7 +1687,7 @@ extern "C" ssm_status ssm_model_load_weights(ssm_model* m, const void* buf, size
                                    m->ctx->stream));
         SSM_HIP_TRY(hipStreamSynchronize(m->ctx->stream));
     }
-    SSM_TRY(refresh_A(m));
+    SSM_TRY(refresh_derived(m));
     SSM_HIP_TRY(hipStreamSynchronize(m->ctx->stream));
     return SSM_OK;
 }
@@ -1678,6 +1698,7 @@ extern "C" ssm_status ssm_forward_device(ssm_model* m, const uint32_t* d_ids, in
     SSM_TRY(model_enter(m, lk));
     SSM_REQUIRE(d_ids && d_logits && B >= 0 && L >= 0, "ssm_forward_device: bad args");
     if (B == 0 || L == 0) return SSM_OK;
+    SSM_TRY(derived_current(m));
     Ws w;
     SSM_TRY(ensure_ws(m, B, L, false, &w));
     const long T = (long)B * L;
@@ -1693,6 +1714,7 @@ extern "C" ssm_status ssm_forward(ssm_model* m, const uint32_t* ids, int B, int 
     SSM_TRY(model_enter(m, lk));
     SSM_REQUIRE(ids && logits && B >= 0 && L >= 0, "ssm_forward: bad args");
     if (B == 0 || L == 0) return SSM_OK;
+    SSM_TRY(derived_current(m));
     const size_t T = (size_t)B * L;
     SSM_TRY(ensure_ids(m, T));
     Ws w;
@@ -1714,6 +1736,7 @@ extern "C" ssm_status ssm_mixer_forward_device(ssm_model* m, int layer, const fl
     SSM_REQUIRE(layer >= 0 && layer < m->dm.nl && d_x && d_y && B >= 0 && L >= 0,
                 "ssm_mixer_forward_device: bad args");
     if (B == 0 || L == 0) return SSM_OK;
+    SSM_TRY(derived_current(m));
     Ws w;
     SSM_TRY(ensure_ws(m, B, L, false, &w));
     return mixer(m, m->layers[layer], d_x, d_y, 0.f, B, L, nullptr, nullptr, w);
@@ -1726,6 +1749,7 @@ extern "C" ssm_status ssm_mixer_forward_device_bf16(ssm_model* m, int layer, con
     SSM_REQUIRE(layer >= 0 && layer < m->dm.nl && d_x && d_y && B >= 0 && L >= 0,
                 "ssm_mixer_forward_device_bf16: bad args");
     if (B == 0 || L == 0) return SSM_OK;
+    SSM_TRY(derived_current(m));
     Ws w;
     SSM_TRY(ensure_ws(m, B, L, false, &w));
     return mixer_bf16(m, layer, d_x, d_y, B, L, w);
@@ -1855,6 +1879,7 @@ namespace {
 ssm_status prefill_device(ssm_model* m, ssm_state* s, const uint32_t* d_ids, int L,
                           uint32_t* d_argmax) {
     const Dims& d = m->dm;
+    SSM_TRY(derived_current(m));
     Ws w;
     SSM_TRY(ensure_ws(m, s->B, L, false, &w));
     // the own LM head on the B last positions (their final norm folded in), else the final
@@ -1918,7 +1943,7 @@ ssm_status decode_body(ssm_model* m, ssm_state* s, const uint32_t* d_ids, float*
     // the own LM head (head.hip) on the packed embedding, with the final norm's scale
     // and the greedy pick folded in
     const bool own_head = w.xg && w.hpart && ssm::head_ok(s->B, d.V, d.d) && d.d % 16 == 0;
-    if (own_head && !m->wp) SSM_TRY(pack_weights(m));   // eager: the first step never replays
+    if (own_head && !m->wp_ok) SSM_TRY(pack_weights(m));   // eager: the first step never replays
     SSM_TRY(trunk(m, d_ids, s->B, 1, s, w, false, own_head));
     if (own_head) {
         Stage g(m->ctx, "head");
@@ -2003,6 +2028,7 @@ extern "C" ssm_status ssm_decode_step_device(ssm_model* m, ssm_state* s, const u
     SSM_TRY(state_enter(s, lk));
     SSM_REQUIRE(s->m == m && d_ids, "ssm_decode_step_device: bad args");
     float* lg = d_logits ? d_logits : s->d_logits;
+    SSM_TRY(derived_current(m));
     if (!graphs_on(m->ctx)) return decode_body(m, s, d_ids, lg, d_argmax);
     return decode_graphed(m, s, d_ids, lg, d_argmax);
 }

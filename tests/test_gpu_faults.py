@@ -115,6 +115,79 @@ def test_failed_weight_packing_is_built_anew(device, inject):
     m.destroy()
 
 
+def test_failed_step_packing_is_built_anew(device, inject):
+    """A launch failure while the one-token step's packed weights are built (a decode's first
+    launches): the next step packs them from the start."""
+    case("injected fault: launch, step weight packing")
+    from ssmjs_amd import _lib, backend
+    m = backend.Model(device, CFG, seed=3)
+    om = O.Model(m.export_weights())
+    ids = np.array([5, 9], np.uint32)
+    st = m.new_state(2)
+    inject("launch")
+    with pytest.raises(_lib.SsmError):
+        st.decode(ids)
+    inject(None)
+    st.reset()
+    got = st.decode(ids)[0]
+    ref = om.forward(ids[:, None])[:, 0]
+    assert np.abs(got - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
+    m.destroy()
+
+
+def test_failed_bf16_cast_is_built_anew(device, inject):
+    """The same for the bf16 layer's weights (its call's first launches)."""
+    case("injected fault: launch, bf16 weights")
+    from ssmjs_amd import _lib, backend
+    cfg = dict(CFG, dState=64, nHeads=2, layers=[{"type": "mamba2"}] * 2)
+    outs = []
+    for fail in (False, True):
+        m = backend.Model(device, cfg, seed=4)
+        x = torch.from_numpy(np.random.default_rng(0).standard_normal((1, 90, cfg["dModel"]))
+                             .astype(np.float32)).cuda()
+        y = torch.empty_like(x)
+        torch.cuda.synchronize()
+        args = ("ssm_mixer_forward_device_bf16", m.handle, 0, x.data_ptr(), y.data_ptr(), 1, 90)
+        if fail:
+            inject("launch")
+            with pytest.raises(_lib.SsmError):
+                _lib.call(*args)
+            inject(None)
+        _lib.call(*args)
+        device.synchronize()
+        outs.append(y.cpu().numpy())
+        m.destroy()
+    np.testing.assert_array_equal(outs[0], outs[1])
+
+
+def test_failed_reload_leaves_no_old_copies(device, inject):
+    """Weights loaded while every launch fails, into a model whose derived copies all exist and
+    whose step is captured: the next calls (decode, long and short prefill) use the new weights."""
+    case("injected fault: launch, reload")
+    from ssmjs_amd import _lib, backend
+    m, other = backend.Model(device, CFG, seed=5), backend.Model(device, CFG, seed=6)
+    blob = other.export_weights()
+    om = O.Model(blob)
+    st = m.new_state(2)
+    ids = np.array([5, 9], np.uint32)
+    for _ in range(3):            # eager, captured, replayed
+        st.reset()
+        st.decode(ids)
+    long_ids = (np.arange(100, dtype=np.uint32) * 7 % 64)[None]
+    m.forward(long_ids)
+    inject("launch")
+    with pytest.raises(_lib.SsmError):
+        m.load_weights(blob)
+    inject(None)
+    st.reset()
+    for got, ref in ((st.decode(ids)[0], om.forward(ids[:, None])[:, 0]),
+                     (m.forward(long_ids), om.forward(long_ids)),
+                     (m.forward(long_ids[:, :20]), om.forward(long_ids[:, :20]))):
+        assert np.abs(got - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
+    m.destroy()
+    other.destroy()
+
+
 def test_session_create_reports_model_failure(inject):
     """MambaSession.create with every allocation failing: the device opens (no allocation), the
     model construction fails and the session raises SessionError('UNKNOWN') as session.ts
