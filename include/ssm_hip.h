@@ -56,7 +56,7 @@ int ssm_abi_version(void);
 /* Failure injection for tests of the error contract (no counterpart in the reference; its
  * GPU_UNAVAILABLE / CHECKPOINT_INVALID paths are session.ts:262-270,393-401): kind
  * "nodevice" (ssm_ctx_create finds no device), "alloc" (every device allocation of the
- * library fails with SSM_ERR_OUT_OF_MEMORY), "launch" (every launch check reports
+ * library fails with SSM_ERR_OUT_OF_MEMORY), "alloc:N" (the N-th from now does), "launch" (every launch check reports
  * SSM_ERR_HIP after the kernel ran normally), "" (none). It holds for the whole process until
  * the next call; NULL hands control back to the environment variable SSM_HIP_FAULT, which
  * each ssm_ctx_create then reads. Unknown kinds: SSM_ERR_INVALID_ARG. */

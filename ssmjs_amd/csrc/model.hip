@@ -64,20 +64,27 @@ ssm_status from_hip(hipError_t e, const char* what) {
 
 // Fault injection for tests of the error contract (session.ts:262-270,393-401): a failure the
 // library reports as if HIP had returned it. "nodevice": ssm_ctx_create finds no device;
-// "alloc": every device allocation of the library fails (out of memory); "launch": every
-// launch check reports a failed launch after the (normally running) kernel was queued.
+// "alloc": every device allocation of the library fails (out of memory), "alloc:N": the N-th
+// from now does; "launch": every launch check reports a failed launch after the (normally
+// running) kernel was queued.
 // The kind lives in an atomic: ssm_set_fault_injection sets it (and pins it against the
 // environment until it is called with NULL); otherwise each ssm_ctx_create latches the
 // environment variable SSM_HIP_FAULT into it. Nothing reads the environment per launch or
 // allocation (getenv is not safe against a concurrent setenv on another thread).
-enum FaultKind { kFaultNone = 0, kFaultNoDevice, kFaultAlloc, kFaultLaunch, kFaultUnknown };
+enum FaultKind { kFaultNone = 0, kFaultNoDevice, kFaultAlloc, kFaultAllocNth,
+                 kFaultLaunch, kFaultUnknown };
 std::atomic<int> g_fault{kFaultNone};
 std::atomic<bool> g_fault_pinned{false};
+std::atomic<int> g_fault_nth{0};
 
 int parse_fault(const char* f) {
     if (!f || !*f) return kFaultNone;
     if (std::strcmp(f, "nodevice") == 0) return kFaultNoDevice;
     if (std::strcmp(f, "alloc") == 0) return kFaultAlloc;
+    if (std::strncmp(f, "alloc:", 6) == 0 && std::atoi(f + 6) > 0) {
+        g_fault_nth.store(std::atoi(f + 6));
+        return kFaultAllocNth;
+    }
     if (std::strcmp(f, "launch") == 0) return kFaultLaunch;
     return kFaultUnknown;
 }
@@ -90,7 +97,7 @@ void latch_fault_env() {
 bool fault(int kind) { return g_fault.load(std::memory_order_relaxed) == kind; }
 
 hipError_t dev_malloc(void** p, size_t bytes) {
-    if (fault(kFaultAlloc)) {
+    if (fault(kFaultAlloc) || (fault(kFaultAllocNth) && g_fault_nth.fetch_sub(1) == 1)) {
         *p = nullptr;
         return hipErrorOutOfMemory;
     }
@@ -544,6 +551,10 @@ struct ssm_model {
     char* wh = nullptr;
     std::vector<long> wh_in, wh_out, wh_x;
     char* wh_emb = nullptr;
+    // set when the device had no room for a packed copy or for a workspace with the packed
+    // activations: the prefill's products then run on the unpacked fp32 operands (gemm()), until
+    // the next load of weights
+    bool unpacked = false;
     int* d_flag = nullptr;   // out-of-range token id flag
     uint32_t* d_ids = nullptr;
     size_t ids_cap = 0;
@@ -641,6 +652,15 @@ void build_layout(ssm_model* m) {
 
 ssm_status pack_weights(ssm_model* m);
 
+// Memory for a packed copy of weights; without it the model goes on unpacked.
+bool room_for(ssm_model* m, void** p, size_t bytes) {
+    if (ssm::dev_malloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    m->unpacked = true;
+    return false;
+}
+
 // Packed copies (gemm_h3.hip) of the layers' in_proj and out_proj, and of the Mamba-1 layers'
 // x_proj. Weights that kernel does not take (rows not 16-byte aligned) have none.
 ssm_status build_wh(ssm_model* m) {
@@ -666,7 +686,7 @@ ssm_status build_wh(ssm_model* m) {
             take(m->wh_out[l], Ly.out_proj, d.d, d.D);
             if (m1) take(m->wh_x[l], Ly.x_proj, RN, d.D);
         }
-        SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh, off ? (size_t)off : 1));
+        if (!room_for(m, (void**)&m->wh, off ? (size_t)off : 1)) return SSM_OK;
     }
     auto pack = [&](long at, long w, int rows, int K) {
         return at < 0 ? SSM_OK : ssm::launch_pack_h3(m->w + w, K, rows, K, m->wh + at, st);
@@ -684,7 +704,7 @@ ssm_status build_wh(ssm_model* m) {
 ssm_status build_wh_emb(ssm_model* m) {
     const Dims& d = m->dm;
     m->wh_emb_ok = false;
-    if (!m->wh_emb) SSM_HIP_TRY(ssm::dev_malloc((void**)&m->wh_emb, ssm::h3_bytes(d.V, d.d)));
+    if (!m->wh_emb && !room_for(m, (void**)&m->wh_emb, ssm::h3_bytes(d.V, d.d))) return SSM_OK;
     SSM_TRY(ssm::launch_pack_h3(m->w + m->emb, d.d, d.V, d.d, m->wh_emb, m->ctx->stream));
     m->wh_emb_ok = true;
     return SSM_OK;
@@ -723,6 +743,7 @@ ssm_status build_wb(ssm_model* m) {
 // the packed copies.
 void drop_derived(ssm_model* m) {
     m->A_ok = m->wp_ok = m->wb_ok = m->wh_ok = m->wh_emb_ok = false;
+    m->unpacked = false;
 }
 ssm_status build_A(ssm_model* m) {
     hipStream_t st = m->ctx->stream;
@@ -859,7 +880,7 @@ size_t plan_ws(ssm_model* m, int B, int L, bool full_logits, Ws* out) {
     const size_t nhp = nhead * (size_t)ssm::head_parts(d.V) * 2;
     size_t o_hp = off; off += al(4 * nhp);
     size_t ngp = 0, nxh = 0;
-    if (h3_rows((long)T) && T <= (size_t)INT32_MAX) {
+    if (h3_rows((long)T) && T <= (size_t)INT32_MAX && !m->unpacked) {
         const int t = (int)T;
         auto product = [&](int rows, int n, int k) {
             ngp = std::max(ngp, ssm::h3_split_floats(rows, n, k));
@@ -901,13 +922,23 @@ size_t plan_ws(ssm_model* m, int B, int L, bool full_logits, Ws* out) {
 }
 
 ssm_status ensure_ws(ssm_model* m, int B, int L, bool full_logits, Ws* w) {
-    const size_t need = plan_ws(m, B, L, full_logits, nullptr);
+    size_t need = plan_ws(m, B, L, full_logits, nullptr);
     if (need > m->ws_bytes) {
         SSM_HIP_TRY(hipStreamSynchronize(m->ctx->stream));
         if (m->ws) SSM_HIP_TRY(hipFree(m->ws));
         m->ws = nullptr;
         m->ws_bytes = 0;
-        SSM_HIP_TRY(ssm::dev_malloc((void**)&m->ws, need));
+        if (ssm::dev_malloc((void**)&m->ws, need) != hipSuccess) {
+            (void)hipGetLastError();
+            const bool was = m->unpacked;
+            m->unpacked = true;
+            need = plan_ws(m, B, L, full_logits, nullptr);
+            const hipError_t e = ssm::dev_malloc((void**)&m->ws, need);
+            if (e != hipSuccess) {
+                m->unpacked = was;
+                SSM_HIP_TRY(e);
+            }
+        }
         m->ws_bytes = need;
     }
     plan_ws(m, B, L, full_logits, w);
@@ -963,7 +994,7 @@ ssm_status mixer(ssm_model* m, const LayerW& Ly, const float* x, float* out, flo
     const float* W = m->w;
     const float* A = m->Ab + Ly.A;
     const bool few = few_rows(T);
-    if (h3_rows(T) && !m->wh_ok) SSM_TRY(build_wh(m));
+    if (h3_rows(T) && !m->wh_ok && !m->unpacked) SSM_TRY(build_wh(m));
     const long l = &Ly - m->layers.data();
     auto packed = [&](const std::vector<long>& at) -> const void* {
         return m->wh_ok && at[l] >= 0 ? m->wh + at[l] : nullptr;
@@ -1503,7 +1534,8 @@ ssm_status head_rows(ssm_model* m, const Ws& w, const float* x, long ldx, int ro
 ssm_status head_many(ssm_model* m, const Ws& w, const float* x, int rows, float* lg) {
     const Dims& d = m->dm;
     const float* E = m->w + m->emb;
-    if (h3_rows(rows) && w.xh && d.d % 4 == 0 && !m->wh_emb_ok) SSM_TRY(build_wh_emb(m));
+    if (h3_rows(rows) && w.xh && d.d % 4 == 0 && !m->wh_emb_ok && !m->unpacked)
+        SSM_TRY(build_wh_emb(m));
     if (h3_product_ok(w, m->wh_emb, rows, d.V, d.d, x, d.d, E, d.V))
         return proj_h3(m, w, rows, d.V, d.d, x, d.d, E, m->wh_emb, lg, d.V, 0.f);
     return gemm(m->ctx, rows, d.V, d.d, x, d.d, E, lg, d.V, 0.f);

@@ -188,6 +188,37 @@ def test_failed_reload_leaves_no_old_copies(device, inject):
     other.destroy()
 
 
+@pytest.mark.parametrize("nth,what", [(2, "workspace"), (3, "layers"), (4, "embedding")])
+def test_no_room_for_packed_operands(device, inject, nth, what):
+    """A long prompt when the device has no room for the workspace with the packed activations,
+    the packed weights or the packed embedding (the allocations after the ids): it runs on the
+    unpacked operands and agrees with the oracle; so does the same prompt after the weights are
+    loaded again, packed."""
+    case(f"injected fault: one allocation, {what}")
+    from ssmjs_amd import _lib, backend
+    m = backend.Model(device, CFG, seed=7)
+    ids = (np.arange(100, dtype=np.uint32) * 7 % 64)[None]
+    ref = O.Model(m.export_weights()).forward(ids)
+
+    def check():
+        assert np.abs(m.forward(ids) - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
+    inject(f"alloc:{nth}")
+    check()
+    inject("alloc")
+    check()                       # (the failure was met: nothing more is allocated)
+    inject(None)
+    m.load_weights(m.export_weights())
+    check()
+    m.destroy()
+    m = backend.Model(device, CFG, seed=7)
+    inject("alloc:1")             # the ids: no call without them
+    with pytest.raises(_lib.SsmError):
+        m.forward(ids)
+    inject(None)
+    check()
+    m.destroy()
+
+
 def test_session_create_reports_model_failure(inject):
     """MambaSession.create with every allocation failing: the device opens (no allocation), the
     model construction fails and the session raises SessionError('UNKNOWN') as session.ts
