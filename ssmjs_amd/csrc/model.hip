@@ -895,7 +895,9 @@ size_t plan_ws(ssm_model* m, int B, int L, bool full_logits, Ws* out) {
             product(t, d.nin, d.d);
             product(t, d.d, d.D);
         }
-        if (nhead == 0) product(full_logits ? t : B, d.V, d.d);
+        // head_many: a forward's T positions, a wide batch's last ones
+        product(t, d.V, d.d);
+        if (h3_rows(B)) product(B, d.V, d.d);
     }
     size_t o_xh = off; off += al(nxh);
     size_t o_gp = off; off += al(4 * ngp);

@@ -60,6 +60,7 @@ def reference(E, ids):
     (150, 8000, 1024),   # wide: 128-column tiles
     (4090, 4084, 64),    # 256 x 256 tiles, ragged edges
     (2050, 4100, 2052),  # 128 x 128 tiles, K in more than 64 blocks, K tail
+    (90, 150, 4180),     # K past what the packing keeps in registers, K tail
 ])
 def test_matches_float64(device, T, V, d):
     print(f"[case] split product T={T} V={V} d={d}", flush=True)
@@ -98,3 +99,23 @@ def test_scales_and_non_finite(device):
     np.testing.assert_array_equal(np.isnan(got[:, 171:175]), np.isnan(ref[:, 171:175]))
     for c in (171, 172):
         np.testing.assert_array_equal(got[:, c], ref[:, c].astype(np.float32))
+
+
+def test_non_finite_in_split_slices(device):
+    """inf, -inf and NaN in a product split over K: a row with one of them, and rows with inf and
+    -inf in different slices, whose sum is NaN only after the slices are added."""
+    print("[case] split product non-finite slices", flush=True)
+    r = np.random.default_rng(5)
+    T, V, d = 70, 64, 1024
+    E = r.standard_normal((V, d)).astype(np.float32)
+    E[60, 3], E[61, 1000], E[62, 500] = np.inf, -np.inf, np.nan
+    E[63, 3], E[63, 1000] = np.inf, -np.inf
+    ids = r.integers(0, 60, T).astype(np.uint32)
+    x = np.sign(E[ids][:, [3, 1000]])
+    got = logits_of(device, E, ids)
+    ref, bound = reference(E[:60], ids)
+    assert float((np.abs(got[:, :60] - ref) / bound).max()) <= 1.0
+    np.testing.assert_array_equal(got[:, 60], x[:, 0] * np.inf)
+    np.testing.assert_array_equal(got[:, 61], -x[:, 1] * np.inf)
+    assert np.isnan(got[:, 62]).all()
+    np.testing.assert_array_equal(got[:, 63], np.where(x[:, 0] == x[:, 1], np.nan, x[:, 0] * np.inf))
