@@ -5,15 +5,22 @@
 // magnitude lies in [2^14, 2^15), and each scaled element v is held as two fp16 values,
 // hi = fp16(v) and lo = fp16(v - hi), both rounded to nearest: v - hi is exact in fp32, and
 // hi + lo is v to 2^-23 |v| or 2^-25 (2^-39 of the row's largest magnitude), whichever is
-// larger. The product of a row pair is summed as lo hi + hi lo + hi hi in fp32 accumulators
+// larger (the excess over 2^-23 |v|, summed over the row, is kept as rho). The product of a row pair is summed as lo hi + hi lo + hi hi in fp32 accumulators
 // (v_mfma_f32_16x16x32_f16, whose products are exact in fp32), leaving out lo lo (2^-22 of a
 // product at most); the sum is scaled back exactly in the epilogue. Three MFMAs at 16 times the fp32
 // matrix rate replace one, and 3 K / 32 roundings of the running sum replace K / 4.
 //
+// Range. Elements 2^-17 of their row's largest magnitude and smaller lose bits, which matters
+// where the large elements meet zeros or tiny ones, so that the small ones make up the sum.
+// Every output is held against rho (below) and, where its sum is not large enough to
+// cover the loss, formed again from the fp32 operands on the fp32 matrix cores, 16 x 16 outputs
+// at a time: the error is at most (3 K / 32) 2^-24 + 2^-22 3 + 2^-22 of S = sum |x w| for any
+// operands (or the fp32 product's K / 4 roundings of 2^-24). Normal data takes no such path.
+//
 // Non-finite values. An inf or NaN element becomes a NaN in hi, so that every output of its
-// row (column) comes out NaN; an output that is not finite is formed again from the fp32
-// operands, term by term, and so gets fp32 arithmetic's own inf or NaN. Rows whose largest
-// magnitude is tiny or huge are scaled by ldexp, which covers the whole fp32 range.
+// row (column) comes out NaN; an output that is not finite is formed again in the same way, and
+// so gets fp32 arithmetic's own inf or NaN. Rows whose largest magnitude is tiny or huge are
+// scaled by ldexp, which covers the whole fp32 range.
 //
 // Packed order. Both operands are read in the MFMA's own order: the 16-row block rb and the
 // 32-k block kb hold two 1 KB fragments (hi, lo), lane 16 q + i of which has row 16 rb + i,
@@ -47,6 +54,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 constexpr int kKB = 32;              // k per block (one MFMA)
 constexpr int kFragB = 1024;         // bytes per fragment
 constexpr int kPairB = 2 * kFragB;   // hi and lo of a (row block, k block)
+constexpr float kRhoZero = -1e30f;   // rho of a row of zeros: its sums are exact
 
 // ---------------------------------------------------------------- packing
 // Workgroup rb packs rows 16 rb .. + 15 (zeros past R): eight waves share the row block's k
@@ -57,6 +65,7 @@ struct PackArgs {
     int R, K, KB;
     char* P;
     int* ex;     // per row: the power of two that undoes the scaling
+    float* rho;  // per row: what hi + lo leave out beyond 2^-23 of an element, summed (scaled)
 };
 
 // STEP: the order of k of the one-token step's operand (stepproj.hip: lane (q, i) holds k = 4 q ..
@@ -64,6 +73,7 @@ struct PackArgs {
 template <int KW, bool STEP, bool VEC>
 __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     __shared__ unsigned red[8][16];
+    __shared__ float rred[8][16];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, i16 = lane & 15;
@@ -118,6 +128,8 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     const int E = min((int)(mx >> 23), 254);
     const int sh = mx ? 141 - E : 0;
     if (w == 0 && q == 0) a.ex[16 * rb + i16] = -sh;
+    float rho = 0.f;
+    const bool low = __any(sh < 0);   // elements of such a row may scale to zero
     for (int kb0 = w; kb0 < a.KB; kb0 += 8 * KW) {
         if (!once) fetch(kb0);
 #pragma unroll
@@ -131,21 +143,36 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
                 const float s = __builtin_ldexpf(x, sh);
                 const bool fin = (__builtin_bit_cast(unsigned, x) & 0x7f800000u) != 0x7f800000u;
                 const _Float16 hh = (_Float16)s;
+                const float d = s - (float)hh;
+                const _Float16 ll = (_Float16)d;
                 hi[e] = fin ? hh : (_Float16)__builtin_nanf("");
-                lo[e] = fin ? (_Float16)(s - (float)hh) : (_Float16)0.f;
+                lo[e] = fin ? ll : (_Float16)0.f;
+                // (a row with inf or NaN: its outputs are formed from the fp32 operands anyway)
+                rho += fmaxf(fmaf(-0x1p-23f, fabsf(s), fabsf(d - (float)ll)), 0.f);
+                if (low && s == 0.f && x != 0.f) rho += 0x1p-126f;
             }
             halfx8* o = reinterpret_cast<halfx8*>(a.P + ((long)rb * a.KB + kb) * kPairB) + lane;
             o[0] = hi;
             o[64] = lo;
         }
     }
+    rho += __shfl_xor(rho, 16);
+    rho += __shfl_xor(rho, 32);
+    if (q == 0) rred[w][i16] = rho;
+    __syncthreads();
+    if (w == 0 && q == 0) {
+        rho = rred[0][i16];
+#pragma unroll
+        for (int k = 1; k < 8; ++k) rho += rred[k][i16];
+        a.rho[16 * rb + i16] = mx ? rho : kRhoZero;
+    }
 }
 
 // ---------------------------------------------------------------- product
 struct H3Args {
-    const char* Xp; const int* xe;
-    const char* Wp; const int* we;
-    const float* X; long ldx;      // the fp32 operands (outputs that are not finite)
+    const char* Xp; const int* xe; const float* xr;
+    const char* Wp; const int* we; const float* wr;
+    const float* X; long ldx;      // the fp32 operands (outputs formed again)
     const float* W; long ldw;
     float* Y; long ldy;
     int M, N, K, KB;
@@ -175,10 +202,30 @@ __device__ __forceinline__ void h3_step() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-__device__ __noinline__ float h3_exact(const float* x, const float* w, int k0, int k1) {
-    float s = 0.f;
-    for (int k = k0; k < k1; ++k) s = fmaf(x[k], w[k], s);
-    return s;
+// The 16 x 16 outputs of a wave from the fp32 operands, k in [k0, k1), on the fp32 matrix cores:
+// x and w are the lane's rows (row / column lane & 15), k quads 4 (lane >> 4) of each 16.
+__device__ __noinline__ floatx4 h3_exact(const float* x, const float* w, int k0, int k1) {
+    const int q4 = 4 * ((threadIdx.x & 63) >> 4);
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int U = 4;
+    for (int k = k0; k < k1; k += 16 * U) {
+        float4 xv[U], wv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kk = k + 16 * u + q4;   // (k0, k1 are multiples of 4)
+            const bool in = kk < k1;
+            xv[u] = in ? *reinterpret_cast<const float4*>(x + kk) : make_float4(0.f, 0.f, 0.f, 0.f);
+            wv[u] = in ? *reinterpret_cast<const float4*>(w + kk) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u].x, wv[u].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u].y, wv[u].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u].z, wv[u].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u].w, wv[u].w, acc, 0, 0, 0);
+        }
+    }
+    return acc;
 }
 
 // WM x WN waves, each with TI x TJ 16 x 16 tiles: a workgroup owns (16 TI WM) x (16 TJ WN) of
@@ -286,33 +333,82 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
         }
     };
 
+    // Whether a running sum is large enough for its split: it bounds S = sum |x w| of the scaled
+    // operands from below, and 2^15 (rho_x + rho_w) bounds what the split's range leaves out, which
+    // is then at most 2^-22 S. Tested halfway (okm: tiles whose sums all are), and at the end for
+    // the others: a row's rho is mostly 0 or a few 2^-26 and its sums 2^27 and more, so an output
+    // fails both only where large elements meet small ones.
+    auto rho_x = [&](int i, float (&v)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * (TI * wm + i) + 4 * q + r;
+            const float rho = a.xr[m0 + min(row, rows - 1)];
+            v[r] = row < rows ? rho : kRhoZero;
+        }
+    };
+    auto rho_w = [&](float (&v)[TJ]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int c = 16 * (TJ * wn + j) + i16;
+            const float rho = a.wr[n0 + min(c, cols - 1)];
+            v[j] = c < cols ? rho : kRhoZero;
+        }
+    };
+    auto large = [&](float s, float rx, float rw) __attribute__((always_inline)) {
+        return fabsf(s) >= 0x1p37f * (rx + rw);
+    };
+    static_assert(TI * TJ <= 32, "a bit per tile");
+    unsigned okm = 0;
+    const int kbm = kb0 + (kb1 - kb0) / (2 * NS) * NS;   // whole turns of the loop below
+    int kb = kb0, end = kbm;
     if constexpr (NS == 2) {
         load(s0, kb0);
-        for (int kb = kb0; kb < kb1; kb += 2) {
-            h3_step<0>();
-            load(s1, kb + 1);
-            compute(s0);
-            h3_step<0>();
-            load(s0, kb + 2);
-            if (kb + 1 < kb1) compute(s1);
-        }
     } else {
         load(s0, kb0);
         load(s1, kb0 + 1);
         load(s2, kb0 + 2);
-        for (int kb = kb0; kb < kb1; kb += 4) {   // blocks past kb1 multiply zeros
-            h3_step<2 * PER>();
-            load(s3, kb + 3);
-            compute(s0);
-            h3_step<2 * PER>();
-            load(s0, kb + 4);
-            compute(s1);
-            h3_step<2 * PER>();
-            load(s1, kb + 5);
-            compute(s2);
-            h3_step<2 * PER>();
-            load(s2, kb + 6);
-            compute(s3);
+    }
+    for (;;) {
+        if constexpr (NS == 2) {
+            for (; kb < end; kb += 2) {
+                h3_step<0>();
+                load(s1, kb + 1);
+                compute(s0);
+                h3_step<0>();
+                load(s0, kb + 2);
+                if (kb + 1 < kb1) compute(s1);
+            }
+        } else {
+            for (; kb < end; kb += 4) {   // blocks past kb1 multiply zeros
+                h3_step<2 * PER>();
+                load(s3, kb + 3);
+                compute(s0);
+                h3_step<2 * PER>();
+                load(s0, kb + 4);
+                compute(s1);
+                h3_step<2 * PER>();
+                load(s1, kb + 5);
+                compute(s2);
+                h3_step<2 * PER>();
+                load(s2, kb + 6);
+                compute(s3);
+            }
+        }
+        if (end == kb1) break;
+        end = kb1;
+        float wr[TJ];
+        rho_w(wr);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+            float xr[4];
+            rho_x(i, xr);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+                bool ok = true;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ok = ok && large(acc[i][j][r], xr[r], wr[j]);
+                okm |= ok ? 1u << (i * TJ + j) : 0u;
+            }
         }
     }
     // the loads past the last block end before the LDS they write is given back
@@ -355,14 +451,35 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
             const int c = 16 * (TJ * wn + j) + i16;
             const unsigned oor = c < cols ? 0u : 0x80000000u;
             const bool gate = !SPLIT && n0 + 16 * (TJ * wn + j) >= a.gate_c0;
+            float vv[4];
+            bool open = !(okm >> (i * TJ + j) & 1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                vv[r] = __builtin_ldexpf(acc[i][j][r], xe[r] + we[j]);
+                open = open || !__builtin_isfinite(vv[r]);
+            }
+            if (__any(open)) {
+                float xr[4], wr[TJ];
+                rho_x(i, xr);
+                rho_w(wr);
+                bool again[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    again[r] = !__builtin_isfinite(vv[r]) || !large(acc[i][j][r], xr[r], wr[j]);
+                if (__any(again[0] || again[1] || again[2] || again[3])) {
+                    const int row = min(16 * (TI * wm + i) + i16, rows - 1);
+                    const floatx4 ev = h3_exact(a.X + (long)(m0 + row) * a.ldx,
+                                                a.W + (long)(n0 + min(c, cols - 1)) * a.ldw,
+                                                kb0 * kKB, min(kb1 * kKB, a.K));
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) vv[r] = again[r] && open ? ev[r] : vv[r];
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * (TI * wm + i) + 4 * q + r;
                 const unsigned o = ((unsigned)(row * ldo + c) * 4u) | oor;
-                float v = __builtin_ldexpf(acc[i][j][r], xe[r] + we[j]);
-                if (!__builtin_isfinite(v) && row < rows && c < cols)
-                    v = h3_exact(a.X + (long)(m0 + row) * a.ldx, a.W + (long)(n0 + c) * a.ldw,
-                                 kb0 * kKB, min(kb1 * kKB, a.K));
+                float v = vv[r];
                 if constexpr (!SPLIT) {
                     if constexpr (RS) v *= rs[row];
                     if constexpr (BETA) v += a.beta * ssm::bload4(ry, o);
@@ -482,8 +599,13 @@ static size_t h3_ex_off(int rows, int K) {
     return (size_t)cdiv(rows, 16) * (size_t)cdiv(K, kKB) * kPairB;
 }
 size_t h3_bytes(int rows, int K) {
-    const size_t b = h3_ex_off(rows, K) + (size_t)cdiv(rows, 16) * 16 * sizeof(int);
+    const size_t b = h3_ex_off(rows, K) + (size_t)cdiv(rows, 16) * 16 * (sizeof(int) + sizeof(float));
     return (b + 255) & ~(size_t)255;
+}
+
+// ... and of the rows' rho behind the exponents.
+static const float* h3_rho(const int* ex, int rows) {
+    return (const float*)(ex + cdiv(rows, 16) * 16);
 }
 
 bool h3_ok(int M, int N, int K, long ldx, long ldw, long ldy) {
@@ -517,8 +639,9 @@ ssm_status launch_pack_h3(const float* X, long ldx, int rows, int K, void* packe
                     ((uintptr_t)X & 15) == 0 && ((uintptr_t)packed & 15) == 0 &&
                     16 * ldx * 4 < (1L << 31),
                 "pack_h3: arguments");
-    const PackArgs a{X, ldx, rows, K, (int)cdiv(K, kKB), (char*)packed,
-                     (int*)((char*)packed + h3_ex_off(rows, K))};
+    int* ex = (int*)((char*)packed + h3_ex_off(rows, K));
+    const PackArgs a{X, ldx, rows, K, (int)cdiv(K, kKB), (char*)packed, ex,
+                     const_cast<float*>(h3_rho(ex, rows))};
     return launch_pack<false, true>(a, st);
 }
 
@@ -529,7 +652,9 @@ ssm_status launch_pack_step(const float* W, long ldw, int N, int K, float* out, 
     SSM_REQUIRE(W && out && N >= 1 && K % 16 == 0 && ldw >= K && ((uintptr_t)out & 15) == 0 &&
                     16 * ldw * 4 < (1L << 31),
                 "pack_step: K %d / ldw %ld / alignment", K, ldw);
-    const PackArgs a{W, ldw, N, K, (int)cdiv(K, kKB), (char*)out, (int*)(out + step_ex_off(N, K))};
+    int* ex = (int*)(out + step_ex_off(N, K));
+    const PackArgs a{W, ldw, N, K, (int)cdiv(K, kKB), (char*)out, ex,
+                     const_cast<float*>(h3_rho(ex, N))};
     return ((uintptr_t)W & 15) == 0 && ldw % 4 == 0 ? launch_pack<true, true>(a, st)
                                                      : launch_pack<true, false>(a, st);
 }
@@ -546,7 +671,9 @@ ssm_status launch_gemm_h3(const void* Xp, const float* X, long ldx, const void* 
     const H3Plan p = pick_h3(M, N, K, ws ? part_floats : 0);
     H3Args a{};
     a.Xp = (const char*)Xp; a.xe = (const int*)((const char*)Xp + h3_ex_off(M, K));
+    a.xr = h3_rho(a.xe, M);
     a.Wp = (const char*)Wp; a.we = (const int*)((const char*)Wp + h3_ex_off(N, K));
+    a.wr = h3_rho(a.we, N);
     a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.Y = Y; a.ldy = ldy;
     a.M = M; a.N = N; a.K = K; a.KB = (int)cdiv(K, kKB); a.beta = beta;
     a.ssq = ssq; a.nssq = nssq; a.inv_div = inv_div; a.eps = eps; a.gate_c0 = gate_c0;

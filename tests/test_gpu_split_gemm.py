@@ -101,6 +101,37 @@ def test_scales_and_non_finite(device):
         np.testing.assert_array_equal(got[:, c], ref[:, c].astype(np.float32))
 
 
+def wide_rows(r, n, d, big, at):
+    """n rows of unit normals, those from n / 2 on with one element of size `big` at column `at`."""
+    E = r.standard_normal((n, d)).astype(np.float32)
+    E[n // 2:, at] = big
+    return E
+
+
+@pytest.mark.parametrize("small", ["inverse", "zero"])
+@pytest.mark.parametrize("big", [1e5, 1e6, 1e8, 2.0 ** 34])
+@pytest.mark.parametrize("T,V,d", [(70, 64, 1024),     # split over K
+                                   (300, 400, 768), (1500, 2050, 256)])
+def test_wide_rows_keep_fp32_precision(device, T, V, d, big, small):
+    """One large element in a row against 1 / it, or 0, in the other operand's row, so that the sum
+    is made of elements far below their row's largest. Outputs formed again take the fp32 matrix
+    cores' K / 4 roundings instead of the split's."""
+    print(f"[case] split product wide rows T={T} V={V} d={d} big={big:g} {small}", flush=True)
+    r = np.random.default_rng(d)
+    E = wide_rows(r, V, d, big, 7)
+    E[:V // 2, 7] = r.standard_normal(V // 2) / big if small == "inverse" else 0.0
+    ids = r.integers(0, V, T).astype(np.uint32)
+    got = logits_of(device, E, ids)
+    ref, bound = reference(E, ids)
+    per = 3 * -(-d // 32) * 2.0 ** -24 + 2.0 ** -20
+    bound *= max(per, d // 4 * 2.0 ** -24 + 2.0 ** -22) / per
+    ratio = float((np.abs(got - ref) / bound).max())
+    meets = np.ix_(ids >= V // 2, np.arange(V) < V // 2)
+    rel = float(np.linalg.norm((got - ref)[meets]) / np.linalg.norm(ref[meets]))
+    print(f"  worst |err| / bound {ratio:.3f}, relative 2-norm of large against small {rel:.2e}")
+    assert np.isfinite(got).all() and ratio <= 1.0 and rel <= 1e-6
+
+
 def test_non_finite_in_split_slices(device):
     """inf, -inf and NaN in a product split over K: a row with one of them, and rows with inf and
     -inf in different slices, whose sum is NaN only after the slices are added."""
