@@ -69,7 +69,8 @@ struct PackArgs {
 };
 
 // STEP: the order of k of the one-token step's operand (stepproj.hip: lane (q, i) holds k = 4 q ..
-// + 3 of the block's first 16, then of its second 16). VEC: 16-byte loads (rows 16-byte aligned).
+// + 3 of the block's first 16, then of its second 16), and the row's exponent and rho in one word
+// (step_ex_off in glue.hpp). VEC: 16-byte loads (rows 16-byte aligned).
 template <int KW, bool STEP, bool VEC>
 __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     __shared__ unsigned red[8][16];
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     // biased exponent of the largest magnitude (inf / NaN rows: the largest finite one)
     const int E = min((int)(mx >> 23), 254);
     const int sh = mx ? 141 - E : 0;
-    if (w == 0 && q == 0) a.ex[16 * rb + i16] = -sh;
+    if (!STEP && w == 0 && q == 0) a.ex[16 * rb + i16] = -sh;
     float rho = 0.f;
     const bool low = __any(sh < 0);   // elements of such a row may scale to zero
     for (int kb0 = w; kb0 < a.KB; kb0 += 8 * KW) {
@@ -164,7 +165,13 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
         rho = rred[0][i16];
 #pragma unroll
         for (int k = 1; k < 8; ++k) rho += rred[k][i16];
-        a.rho[16 * rb + i16] = mx ? rho : kRhoZero;
+        rho = mx ? rho : kRhoZero;
+        if constexpr (STEP) {
+            const unsigned up = __builtin_bit_cast(unsigned, rho) + (mx ? 0xffffu : 0u);
+            a.ex[16 * rb + i16] = (int)((up & 0xffff0000u) | ((unsigned)-sh & 0xffffu));
+        } else {
+            a.rho[16 * rb + i16] = rho;
+        }
     }
 }
 
@@ -652,9 +659,8 @@ ssm_status launch_pack_step(const float* W, long ldw, int N, int K, float* out, 
     SSM_REQUIRE(W && out && N >= 1 && K % 16 == 0 && ldw >= K && ((uintptr_t)out & 15) == 0 &&
                     16 * ldw * 4 < (1L << 31),
                 "pack_step: K %d / ldw %ld / alignment", K, ldw);
-    int* ex = (int*)(out + step_ex_off(N, K));
-    const PackArgs a{W, ldw, N, K, (int)cdiv(K, kKB), (char*)out, ex,
-                     const_cast<float*>(h3_rho(ex, N))};
+    const PackArgs a{W, ldw, N, K, (int)cdiv(K, kKB), (char*)out, (int*)(out + step_ex_off(N, K)),
+                     nullptr};
     return ((uintptr_t)W & 15) == 0 && ldw % 4 == 0 ? launch_pack<true, true>(a, st)
                                                      : launch_pack<true, false>(a, st);
 }

@@ -79,7 +79,7 @@ struct StepProj {
     const float* wxt = nullptr; int RN = 0; float* xpart = nullptr;
     // EPI_HEAD: greedy (value, index) pairs, (M, nparts), one per row and workgroup
     float* part = nullptr; int nparts = 0;
-    // set by the launcher: row and column tiles, row groups, passes over K, W's row exponents
+    // set by the launcher: row and column tiles, row groups, passes over K, W's row words (step_ex_off)
     int mt = 0, nt = 0, rg = 0, npass = 0;
     const int* we = nullptr;
 };
@@ -89,7 +89,8 @@ ssm_status launch_stepproj(int epi, StepProj a, hipStream_t st);
 // Workgroups of an EPI_HEAD launch that write a pair per row.
 int step_head_parts(int M, int N, int K);
 // W (N, K) row stride ldw -> the step projection's packed operand in out (step_w_floats(N, K)
-// floats, 16-byte aligned; gemm_h3.hip). The row exponents start at float step_ex_off.
+// floats, 16-byte aligned; gemm_h3.hip). From float step_ex_off on, a word per row: its exponent (low
+// 16 bits, signed) and its loss rho, rounded up to the high half of a float.
 size_t step_ex_off(int rows, int K);
 size_t step_w_floats(int rows, int K);
 ssm_status launch_pack_step(const float* W, long ldw, int N, int K, float* out, hipStream_t st);

@@ -31,8 +31,12 @@
 // v_mfma_f32_16x16x32_f16 (lo hi, hi lo, hi hi) into fp32 sums, scaled back exactly. W is packed
 // once per load (launch_pack_step, gemm_h3.hip: a scale per row); X arrives in fp32 and each wave
 // scales and splits its own k range of it in registers, while its W is still on the way from HBM.
-// Elements that are inf or NaN become NaN, and an output that is not finite is formed again from
-// the fp32 operands.
+// Range: as there, every output is held against what the split may have lost of elements far
+// below their row's largest (W: the packing's rho; X: 2^-25 for each element of a lane that holds
+// one below 2^-16 of its wave's largest). Its measure is the waves' partial sums taken by
+// magnitude, which are small together only if the operands really are that far apart. Such an
+// output, and one that is not finite (elements that are inf or NaN become NaN), is formed again
+// from the fp32 operands.
 //
 // Operand order. X is in fragment order (frag_off in glue.hpp): the 1 KB of a (16-row tile,
 // 16-wide k-block) is contiguous, lane-major, lane 16 q + i holding row i, k = 4 q .. + 3, so one
@@ -94,12 +98,34 @@ __device__ __forceinline__ void split2(float a, float b, int sh, unsigned& hi, u
     lo = __builtin_bit_cast(unsigned, l);
 }
 
-// sum_k X[m, k] W[n, k] from the fp32 operands (X in fragment order), k in order: outputs whose
-// split product is not finite.
-__device__ __noinline__ float step_exact(const float* X, const float* w, int m, int K) {
-    float s = 0.f;
-    for (int k = 0; k < K; ++k) s = fmaf(X[frag_off(m, k, K >> 4)], w[k], s);
-    return s;
+// sum_k X[m, k] W[n, k] from the fp32 operands (X in fragment order) for the lanes with `again`
+// set, whose split product will not do: the 16 lanes of a row m share one output at a time, each
+// its quads of k in order, then a tree. (All lanes of the wave call it; W rows start anywhere.
+// Inline and not unrolled: it takes few registers, where a call had the multi-tile kernels spill.)
+__device__ __forceinline__ float step_exact(const float* X, const float* W, int m, int n, int K,
+                                         bool again) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15;
+    unsigned todo = (unsigned)(__ballot(again) >> (lane & 48)) & 0xffffu;
+    float out = 0.f;
+    while (__any(todo != 0)) {
+        const int src = todo ? __builtin_ctz(todo) : 0;
+        const float* w = W + (long)__shfl(n, src, 16) * K;
+        float s = 0.f;
+        if (todo) {
+#pragma unroll 1
+            for (int k = 4 * l16; k < K; k += 64) {
+                const float4 x = *reinterpret_cast<const float4*>(X + frag_off(m, k, K >> 4));
+                s = fmaf(x.x, w[k], s);
+                s = fmaf(x.y, w[k + 1], s);
+                s = fmaf(x.z, w[k + 2], s);
+                s = fmaf(x.w, w[k + 3], s);
+            }
+        }
+        s = sum16(s);
+        if (todo && l16 == src) out = s;
+        todo &= todo - 1;
+    }
+    return out;
 }
 
 // MT row tiles, NC column tiles at a time, KW 32-wide k-blocks per wave and pass; MULTI: a
@@ -112,6 +138,7 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     constexpr int RS = (ROWS + 31) / 32, EPT = RS * NC;
     __shared__ float red[MULTI ? 2 : 1][kNW][ROWS][16 * NC + 1];
     __shared__ float sc[64];
+    __shared__ float2 loss[kNW][ROWS];   // (what the split of X may lose, scale) per wave and row
     __shared__ float us[EPI == EPI_CONVX ? ROWS : 1][16 * NC + 1];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -165,22 +192,34 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     // undoes the scale of the accumulator's rows 4 q + r of tile i
     u32x4 xh[MT][KW], xl[MT][KW];   // eight fp16 values each
     int ex[MT][4];
+    float2 lost[MT];                // of row l16 of tile i: the passes' losses and scales, summed
+#pragma unroll
+    for (int i = 0; i < MT; ++i) lost[i] = make_float2(0.f, 0.f);
     auto split = [&](const float4 (&x)[MT][KW][2]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            unsigned mx = 0;
+            unsigned mx = 0, mn = 0x7fffffffu;
 #pragma unroll
             for (int u = 0; u < KW; ++u)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const float4 v = x[i][u][h];
-                    const unsigned m1 = max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu);
-                    const unsigned m2 = max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu);
-                    mx = max(mx, max(m1, m2));
+                    const unsigned b0 = __float_as_uint(v.x) & 0x7fffffffu, b1 = __float_as_uint(v.y) & 0x7fffffffu,
+                                   b2 = __float_as_uint(v.z) & 0x7fffffffu, b3 = __float_as_uint(v.w) & 0x7fffffffu;
+                    mx = max(max(mx, b0), max(b1, max(b2, b3)));
+                    mn = min(min(mn, b0), min(b1, min(b2, b3)));
                 }
             mx = max(mx, (unsigned)__shfl_xor((int)mx, 16));
             mx = max(mx, (unsigned)__shfl_xor((int)mx, 32));
-            const int sh = mx ? 141 - min((int)(mx >> 23), 254) : 0;
+            const int E = min((int)(mx >> 23), 254), sh = mx ? 141 - E : 0;
+            // lanes whose smallest element (a zero counts) is below 2^-2 scaled: up to 2^-25 lost
+            // of each of the lane's elements
+            const unsigned long long small = __ballot((int)(mn >> 23) < max(E - 16, 1));
+            const int lanes = __popcll((small >> l16) & 0x0001000100010001ull);
+            if (mx) {
+                lost[i].x += __builtin_ldexpf((float)(lanes * 8 * KW), -25 - sh);
+                lost[i].y += __builtin_ldexpf(1.f, -sh);
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) ex[i][r] = -__shfl(sh, 4 * q + r);
             // (an inf gives hi = inf, lo = NaN, and so NaN in every product of its row)
@@ -277,6 +316,9 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     const auto rg2 = rsrc(a.g2, EPI == EPI_RESID && a.g2 ? (unsigned)a.N * 4u : 0u);
     const auto ryy = rsrc(a.Y, EPI == EPI_RESID ? (unsigned)((long)(a.M - 1) * a.ldy + a.N) * 4u : 0u);
 
+    // the rows' losses over all waves, summed when the first tile's waves have met
+    float2 rl[RS];
+    bool first = true;
     // One column tile: W of its first pass is in wc; the next tile's goes into wnx.
     constexpr int kConvPre = 4;
     constexpr int kXpBlk = kXpartMaxRN / 16 / kNW;   // x_proj column blocks per wave
@@ -284,7 +326,8 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
         // The epilogue's inputs, loaded ahead of the product (they do not depend on it): column
         // en[j] of column tile j, rows as above.
         const int ej = tid & 15;
-        int en[NC], wex[NC];
+        int en[NC];
+        unsigned wex[NC];   // exponent and loss (rho) of the column's W row
         bool col_ok[NC], in_conv[NC], pre[NC];
         float csv[EPT][kConvPre - 1], cwv[NC][kConvPre], cbv[NC], rsv[EPT], g2v[NC];
         // (through range-checked descriptors: a guarded load would sit behind a branch, and the
@@ -296,7 +339,7 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
             const int c = en[j] - a.c0;
             in_conv[j] = CONV && col_ok[j] && c >= 0 && c < a.C;
             pre[j] = in_conv[j] && a.Kc <= kConvPre;
-            wex[j] = (int)__float_as_uint(bload4(rwe, col_ok[j] ? 4u * en[j] : kOOR));
+            wex[j] = __float_as_uint(bload4(rwe, col_ok[j] ? 4u * en[j] : kOOR));
             if constexpr (CONV) {
                 const int Kc1 = a.Kc - 1;
 #pragma unroll
@@ -370,7 +413,25 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     red[buf][w][16 * ((i + irot) & (MT - 1)) + 4 * q + r][16 * j + l16] = out[j][i][r];
+        if (!MULTI || first) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                if (q == 0) loss[w][16 * ((i + irot) & (MT - 1)) + l16] = lost[i];
+        }
         __syncthreads();
+        if (!MULTI || first) {
+#pragma unroll
+            for (int s = 0; s < RS; ++s) {
+                const int ei = min((tid >> 4) + 32 * s, ROWS - 1);
+                rl[s] = loss[0][ei];
+#pragma unroll
+                for (int k = 1; k < kNW; ++k) {
+                    rl[s].x += loss[k][ei].x;
+                    rl[s].y += loss[k][ei].y;
+                }
+            }
+            first = false;
+        }
 
         float uo[EPT];
 #pragma unroll
@@ -379,12 +440,24 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
             const int ei = (tid >> 4) + 32 * (e % RS), em = m0 + ei, n = en[j], c = n - a.c0;
             uo[e] = 0.f;
             if (ei >= ROWS) continue;
-            float v = red[buf][0][ei][16 * j + ej];
+            float v = red[buf][0][ei][16 * j + ej], mag = fabsf(v);
 #pragma unroll
-            for (int k = 1; k < kNW; ++k) v += red[buf][k][ei][16 * j + ej];
-            v = __builtin_ldexpf(v, wex[j]);
+            for (int k = 1; k < kNW; ++k) {
+                const float t = red[buf][k][ei][16 * j + ej];
+                v += t;
+                mag += fabsf(t);
+            }
+            v = __builtin_ldexpf(v, (int)(short)wex[j]);
             const bool ok = em < a.M && col_ok[j];
-            if (!__builtin_isfinite(v) && ok) v = step_exact(a.X, a.Wf + (long)n * a.K, em, a.K);
+            // the split's loss, at most 2^15 (loss of X + scale * rho of W), against 2^-22 of the
+            // magnitudes (the factor 2^37 in two parts, within fp32's range)
+            const float2 lo = rl[e % RS];
+            const bool covered = mag * 0x1p-20f >= fmaf(lo.y, __uint_as_float(wex[j] & 0xffff0000u), lo.x) * 0x1p17f;
+            const bool again = ok && !(covered && __builtin_isfinite(v));
+            if (__any(again)) {
+                const float t = step_exact(a.X, a.Wf, em, n, a.K, again);
+                v = again ? t : v;
+            }
             v *= sc[ei];
             if constexpr (EPI == EPI_STORE) {
                 if (ok) {

@@ -10,7 +10,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
-from test_gpu_split_gemm import device, logits_of, reference  # noqa: E402,F401
+from test_gpu_split_gemm import device, logits_of, reference, wide_rows  # noqa: E402,F401
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +71,23 @@ def test_scales_and_non_finite(device, T):   # noqa: F811
     np.testing.assert_array_equal(np.isnan(got[:, 171:175]), np.isnan(ref[:, 171:175]))
     for c in (171, 172):
         np.testing.assert_array_equal(got[:, c], ref[:, c].astype(np.float32))
+
+
+@pytest.mark.parametrize("small", ["inverse", "zero"])
+@pytest.mark.parametrize("big", [1e5, 1e6, 1e8, 2.0 ** 34])
+@pytest.mark.parametrize("T,V,d", [(1, 300, 768), (40, 130, 2064), (64, 3100, 1024)])
+def test_wide_rows_keep_fp32_precision(device, T, V, d, big, small):   # noqa: F811
+    """As in the prefill's test: one large element in a row against 1 / it, or 0, in the other
+    operand's row. Outputs formed again add K / 16 terms in order and 4 levels of a tree."""
+    print(f"[case] step projection wide rows T={T} V={V} d={d} big={big:g} {small}", flush=True)
+    r = np.random.default_rng(d)
+    E = wide_rows(r, V, d, big, 7)
+    E[:V // 2, 7] = r.standard_normal(V // 2) / big if small == "inverse" else 0.0
+    for ids in (r.integers(V // 2, V, T), r.integers(0, V // 2, T)):
+        got = logits_of(device, E, ids.astype(np.uint32))
+        ref, bound = bounded(E, ids)
+        meets = np.arange(V) < V // 2 if ids[0] >= V // 2 else np.arange(V) >= V // 2
+        ratio = float((np.abs(got - ref) / bound).max())
+        rel = float(np.linalg.norm((got - ref)[:, meets]) / np.linalg.norm(ref[:, meets]))
+        print(f"  worst |err| / bound {ratio:.3f}, relative 2-norm of large against small {rel:.2e}")
+        assert np.isfinite(got).all() and ratio <= 1.0 and rel <= 1e-6
