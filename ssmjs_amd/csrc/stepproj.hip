@@ -154,9 +154,18 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     const int m0 = tg * ROWS;
     const int KB = a.K >> 4, KB2 = (KB + 1) >> 1;   // 16-wide blocks of X, 32-wide of W
 
-    // ---- operand loads: this wave's k-blocks of pass p are KW (kNW p + w) .. + KW - 1, summed
-    // in this order in every workgroup (equal rows of W give equal results). Every workgroup
-    // reads the same X; those on one XCD start at row tiles of their own.
+    // ---- operand loads: a wave's k-blocks go in groups of four, each scaled and summed by itself,
+    // and the groups' sums are added in order: the same in every workgroup (equal rows of W give
+    // equal results) and whether a pass takes two groups or, with more row tiles in the registers,
+    // one (a row's result does not depend on the rows beside it). Past four k-blocks a wave, two
+    // groups are adjacent. Every workgroup reads the same X; those on one XCD start at row tiles of
+    // their own.
+    constexpr int KG = 4, NG = KW / KG;
+    static_assert(KW == KG || KW == 2 * KG, "one or two groups");
+    const bool halves = KW == KG && a.npass > 1;   // (uniform) a pass takes one of two adjacent groups
+    auto block = [&](int p, int u) __attribute__((always_inline)) {
+        return halves ? 2 * KG * (kNW * (p >> 1) + w) + KG * (p & 1) + u : KW * (kNW * p + w) + u;
+    };
     const int irot = (r8 / a.rg) & (MT - 1);
     const auto ra = rsrc(a.X, (unsigned)(a.mt * KB) * 1024u);
     auto load_x = [&](float4 (&x)[MT][KW][2], int p) __attribute__((always_inline)) {
@@ -166,7 +175,7 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
             for (int u = 0; u < KW; ++u)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const int k16 = 2 * (KW * (kNW * p + w) + u) + h;
+                    const int k16 = 2 * block(p, u) + h;
                     const int tm = tg * MT + ((i + irot) & (MT - 1));
                     x[i][u][h] = bload16<float4>(
                         ra, k16 < KB && tm < a.mt ? (unsigned)(tm * KB + k16) * 1024u + 16u * lane
@@ -181,50 +190,58 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
                                  t < a.nt ? (unsigned)KB2 * 2048u : 0u);
 #pragma unroll
             for (int u = 0; u < KW; ++u) {
-                const int kb = KW * (kNW * p + w) + u;
+                const int kb = block(p, u);
                 const unsigned o = kb < KB2 ? (unsigned)kb * 2048u + 16u * lane : kOOR;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) wv[j][u][h] = ssm::bload16_nt<halfx8>(rw, o + 1024u * h);
             }
         }
     };
-    // the row's power of two over this wave's k range, and the split operands; ex[i] packs what
-    // undoes the scale of the accumulator's rows 4 q + r of tile i
+    // the split operands, by the row's power of two over the group; ex[g][i] undoes the scale of the
+    // accumulator's rows 4 q + r of tile i
     u32x4 xh[MT][KW], xl[MT][KW];   // eight fp16 values each
-    int ex[MT][4];
+    int ex[NG][MT][4];
     float2 lost[MT];                // of row l16 of tile i: the passes' losses and scales, summed
 #pragma unroll
     for (int i = 0; i < MT; ++i) lost[i] = make_float2(0.f, 0.f);
     auto split = [&](const float4 (&x)[MT][KW][2]) __attribute__((always_inline)) {
+        // (no branch, and step by step over all groups: their exchanges overlap)
+        unsigned mx[NG * MT], mn[NG * MT];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            unsigned mx = 0, mn = 0x7fffffffu;
+        for (int gi = 0; gi < NG * MT; ++gi) {
+            mx[gi] = 0;
+            mn[gi] = 0x7fffffffu;
 #pragma unroll
-            for (int u = 0; u < KW; ++u)
+            for (int u = KG * (gi / MT); u < KG * (gi / MT + 1); ++u)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const float4 v = x[i][u][h];
+                    const float4 v = x[gi % MT][u][h];
                     const unsigned b0 = __float_as_uint(v.x) & 0x7fffffffu, b1 = __float_as_uint(v.y) & 0x7fffffffu,
                                    b2 = __float_as_uint(v.z) & 0x7fffffffu, b3 = __float_as_uint(v.w) & 0x7fffffffu;
-                    mx = max(max(mx, b0), max(b1, max(b2, b3)));
-                    mn = min(min(mn, b0), min(b1, min(b2, b3)));
+                    mx[gi] = max(max(mx[gi], b0), max(b1, max(b2, b3)));
+                    mn[gi] = min(min(mn[gi], b0), min(b1, min(b2, b3)));
                 }
-            mx = max(mx, (unsigned)__shfl_xor((int)mx, 16));
-            mx = max(mx, (unsigned)__shfl_xor((int)mx, 32));
-            const int E = min((int)(mx >> 23), 254), sh = mx ? 141 - E : 0;
+        }
+#pragma unroll
+        for (int o = 16; o <= 32; o *= 2)
+#pragma unroll
+            for (int gi = 0; gi < NG * MT; ++gi)
+                mx[gi] = max(mx[gi], (unsigned)__shfl_xor((int)mx[gi], o));
+#pragma unroll
+        for (int gi = 0; gi < NG * MT; ++gi) {
+            const int g = gi / MT, i = gi % MT;
+            const int E = min((int)(mx[gi] >> 23), 254), sh = mx[gi] ? 141 - E : 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ex[g][i][r] = -__shfl(sh, 4 * q + r);
             // lanes whose smallest element (a zero counts) is below 2^-2 scaled: up to 2^-25 lost
             // of each of the lane's elements
-            const unsigned long long small = __ballot((int)(mn >> 23) < max(E - 16, 1));
+            const unsigned long long small = __ballot((int)(mn[gi] >> 23) < max(E - 16, 1));
             const int lanes = __popcll((small >> l16) & 0x0001000100010001ull);
-            if (mx) {
-                lost[i].x += __builtin_ldexpf((float)(lanes * 8 * KW), -25 - sh);
-                lost[i].y += __builtin_ldexpf(1.f, -sh);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ex[i][r] = -__shfl(sh, 4 * q + r);
+            lost[i].x += mx[gi] ? __builtin_ldexpf((float)(lanes * 8 * KG), -25 - sh) : 0.f;
+            lost[i].y += mx[gi] ? __builtin_ldexpf(1.f, -sh) : 0.f;
             // (an inf gives hi = inf, lo = NaN, and so NaN in every product of its row)
 #pragma unroll
-            for (int u = 0; u < KW; ++u)
+            for (int u = KG * g; u < KG * (g + 1); ++u)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const float4 v = x[i][u][h];
@@ -238,38 +255,41 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     };
     floatx4 out[NC][MT];
     auto multiply = [&](const halfx8 (&wv)[NC][KW][2]) __attribute__((always_inline)) {
-        floatx4 acc[NC][MT];
 #pragma unroll
-        for (int j = 0; j < NC; ++j)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-        auto mm = [&](int j, int i, u32x4 x, halfx8 y) __attribute__((always_inline)) {
-            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(x), y, acc[j][i], 0, 0, 0);
-        };
-#pragma unroll
-        for (int u = 0; u < KW; ++u) {
+        for (int g = 0; g < NG; ++g) {
+            floatx4 acc[NC][MT];
 #pragma unroll
             for (int j = 0; j < NC; ++j)
 #pragma unroll
-                for (int i = 0; i < MT; ++i) mm(j, i, xl[i][u], wv[j][u][0]);
+                for (int i = 0; i < MT; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+            auto mm = [&](int j, int i, u32x4 x, halfx8 y) __attribute__((always_inline)) {
+                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(x), y, acc[j][i], 0, 0, 0);
+            };
+#pragma unroll
+            for (int u = KG * g; u < KG * (g + 1); ++u) {
+#pragma unroll
+                for (int j = 0; j < NC; ++j)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) mm(j, i, xl[i][u], wv[j][u][0]);
+#pragma unroll
+                for (int j = 0; j < NC; ++j)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) mm(j, i, xh[i][u], wv[j][u][1]);
+#pragma unroll
+                for (int j = 0; j < NC; ++j)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) mm(j, i, xh[i][u], wv[j][u][0]);
+            }
 #pragma unroll
             for (int j = 0; j < NC; ++j)
 #pragma unroll
-                for (int i = 0; i < MT; ++i) mm(j, i, xh[i][u], wv[j][u][1]);
+                for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NC; ++j)
-#pragma unroll
-                for (int i = 0; i < MT; ++i) mm(j, i, xh[i][u], wv[j][u][0]);
+                    for (int r = 0; r < 4; ++r) {
+                        const float v = acc[j][i][r];
+                        out[j][i][r] += __builtin_ldexpf(v, ex[g][i][r]);
+                    }
         }
-#pragma unroll
-        for (int j = 0; j < NC; ++j)
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float v = acc[j][i][r];
-                    out[j][i][r] += __builtin_ldexpf(v, ex[i][r]);
-                }
     };
 
     float4 xr[MT][KW][2];
@@ -720,7 +740,7 @@ StepPlan step_plan(int M, int N, int K) {
     p.rg = (int)cdiv(mt, p.rt);
     p.nc = p.rt == 2 && p.rg == 2 && nt >= 192 ? 2 : 1;
     p.per = p.rt > 1 || kw <= 4 ? 4 : 8;
-    p.npass = (int)cdiv(kw, p.per);
+    p.npass = kw > 4 && p.per == 4 ? 2 * (int)cdiv(kw, 8) : (int)cdiv(kw, p.per);
     const long groups = cdiv(nt, p.nc), padded = 8L * cdiv(groups, 8);
     p.multi = p.npass == 1 && padded * p.rg > kStepMaxWG && kStepMaxWG % (8 * p.rg) == 0;
     p.grid = p.multi ? (unsigned)kStepMaxWG : (unsigned)(padded * p.rg);

@@ -91,3 +91,16 @@ def test_wide_rows_keep_fp32_precision(device, T, V, d, big, small):   # noqa: F
         rel = float(np.linalg.norm((got - ref)[:, meets]) / np.linalg.norm(ref[:, meets]))
         print(f"  worst |err| / bound {ratio:.3f}, relative 2-norm of large against small {rel:.2e}")
         assert np.isfinite(got).all() and ratio <= 1.0 and rel <= 1e-6
+
+
+@pytest.mark.parametrize("V,d", [(300, 768), (4099, 1040), (4099, 2064), (3100, 4096)])
+def test_rows_do_not_depend_on_their_batch(device, V, d):   # noqa: F811
+    """A row's logits have the same bits in batches of 1 to 64, which take one or two row tiles per
+    workgroup and one or several passes over K."""
+    print(f"[case] step projection batches V={V} d={d}", flush=True)
+    r = np.random.default_rng(d)
+    E = r.standard_normal((V, d)).astype(np.float32)
+    ids = r.integers(0, V, 64).astype(np.uint32)
+    whole = logits_of(device, E, ids)
+    for T in (1, 16, 17, 40):
+        np.testing.assert_array_equal(logits_of(device, E, ids[:T]), whole[:T])
