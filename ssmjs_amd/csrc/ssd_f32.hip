@@ -92,7 +92,7 @@ __device__ __forceinline__ int call_head(const F32Args& a, int h) {
     return a.hs_inv ? (int)__umulhi((unsigned)h, a.hs_inv) : h;
 }
 
-template <int NN, bool FULL, bool GATED, int HPW>
+template <int NN, bool FULL, bool GATED, int HPW, bool EX>
 struct SmemF32 {
     static constexpr int BP = NN + 4;    // B / C row pitch (floats): b128 rows conflict-free
     static constexpr int MP = QF + 4;    // M^T row pitch
@@ -104,8 +104,7 @@ struct SmemF32 {
     float wj[2][HPW][QF];    // w_t = 2^(acum_end - acum_t) dt'_t
     float ae[2][HPW];        // acum_end
     float sq[GATED ? 2 : 1][HPW][GATED ? 4 : 1][GATED ? QF : 1];   // per-wave sums of u^2 per row
-    // d_state <= 32: the low part of ac
-    alignas(16) float al[NN <= 32 ? 2 : 1][HPW][NN <= 32 ? QF : 1];
+    alignas(16) float al[EX ? 2 : 1][HPW][EX ? QF : 1];   // EX: the low part of ac
 };
 
 using ssm::bload16;
@@ -162,11 +161,12 @@ __device__ __forceinline__ double lane_of(double v, int lane) {
 
 __device__ __forceinline__ float4 as_f4(floatx4 v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
-template <int NN, bool FULL, bool GATED = false, int HPW = 1>
+// EX: running sums of the decay to double precision (scan_dt)
+template <int NN, bool FULL, bool GATED, int HPW, bool EX>
 __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     static_assert(FULL || HPW == 1, "the state-only pass takes one head per workgroup");
-    __shared__ __attribute__((aligned(16))) SmemF32<NN, FULL, GATED, HPW> sm;
-    using SM = SmemF32<NN, FULL, GATED, HPW>;
+    __shared__ __attribute__((aligned(16))) SmemF32<NN, FULL, GATED, HPW, EX> sm;
+    using SM = SmemF32<NN, FULL, GATED, HPW, EX>;
     constexpr int NB = NN / 16;          // n blocks (state tiles per wave, k groups of C B^T)
     constexpr int QB = QF / 16;          // time blocks per chunk
     constexpr int NCB = QB * (QB + 1) / 2;   // causal C B^T tiles per chunk
@@ -361,17 +361,18 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
     float decay_sum = 0.f;
     // dt' of a chunk of qv steps (0 past them), its running sum times A_h and the weights w_t
     // into LDS buffer bf of head k (lane = time step; `put`: this wave writes); returns the
-    // chunk's whole sum. With d_state <= 32 the running sum is kept to double precision, as
-    // hi + lo: decays are differences of it, and a head of fast decay reaches 60 log2 units in a
+    // chunk's whole sum. With EX (d_state <= 32, and heads of more than 64 rows: the shapes that
+    // walked the steps one by one before this kernel took them) the running sum is kept to double
+    // precision, as hi + lo: decays are differences of it, and a head of fast decay reaches 60 log2 units in a
     // chunk, where one fp32 rounding of the sum is 1.3e-6 of the decay (relative error of the
     // final state 1.3e-6 -> 1e-7, against 4e-7 of a product of the steps' decays, which these
     // shapes had before the matrix-core kernel; the scan's time is hidden).
     auto scan_dt = [&](float raw_dt, int qv, int bf, int k, bool put) __attribute__((always_inline)) {
         float dv = raw_dt + dtb;
-        if (a.softplus) dv = NN <= 32 ? ssm::softplus_corr(dv) : ssm::softplus_fast(dv);
+        if (a.softplus) dv = EX ? ssm::softplus_corr(dv) : ssm::softplus_fast(dv);
         dv = lane < qv ? fminf(fmaxf(dv, a.dt_min), a.dt_max) : 0.f;
         float sc, ae, we;
-        if constexpr (NN <= 32) {
+        if constexpr (EX) {
             const double sd = wave_prefix_sum((double)dv * (double)Ah);
             const double ad = lane_of(sd, QF - 1);
             sc = (float)sd;
@@ -509,7 +510,7 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
                     const float acja[4] = {acj.x, acj.y, acj.z, acj.w};
                     const float dvja[4] = {dvj.x, dvj.y, dvj.z, dvj.w};
                     float dl[4] = {aci - acja[0], aci - acja[1], aci - acja[2], aci - acja[3]};
-                    if constexpr (NN <= 32) {
+                    if constexpr (EX) {
                         const float ali = sm.al[buf][k][i];
                         const float4 alj = *reinterpret_cast<const float4*>(&sm.al[buf][k][16 * jb + 4 * q4]);
                         dl[0] += ali - alj.x;
@@ -725,13 +726,13 @@ void plan_f32(int B, int L, int H, int N, int& nchunks, int& nseg, int& per) {
     nseg = (int)ssm::cdiv(nchunks, per);
 }
 
-template <int NN>
+template <int NN, bool EX>
 ssm_status launch(F32Args& a, hipStream_t st) {
     if (a.nseg > 1) {
         F32Args s1 = a;
         const int nwg1 = a.B * a.H * (a.nseg - 1);   // the last segment's local state is unused
         s1.remap = (nwg1 % 8 == 0) ? 1 : 0;
-        ssd_f32_kernel<NN, false><<<nwg1, 256, 0, st>>>(s1);
+        ssd_f32_kernel<NN, false, false, 1, EX><<<nwg1, 256, 0, st>>>(s1);
         ssm_status e = ssm::check_launch("ssd_f32_state_pass");
         if (e != SSM_OK) return e;
         if constexpr (NN > 32) {
@@ -753,11 +754,11 @@ ssm_status launch(F32Args& a, hipStream_t st) {
     const int nwg = a.B * (a.H / hpw) * a.nseg;
     a.remap = (nwg % 8 == 0) ? 1 : 0;
     if (hpw == 2) {
-        if (a.ssq) ssd_f32_kernel<NN, true, true, 2><<<nwg, 512, 0, st>>>(a);
-        else ssd_f32_kernel<NN, true, false, 2><<<nwg, 512, 0, st>>>(a);
+        if (a.ssq) ssd_f32_kernel<NN, true, true, 2, EX><<<nwg, 512, 0, st>>>(a);
+        else ssd_f32_kernel<NN, true, false, 2, EX><<<nwg, 512, 0, st>>>(a);
     } else {
-        if (a.ssq) ssd_f32_kernel<NN, true, true><<<nwg, 256, 0, st>>>(a);
-        else ssd_f32_kernel<NN, true><<<nwg, 256, 0, st>>>(a);
+        if (a.ssq) ssd_f32_kernel<NN, true, true, 1, EX><<<nwg, 256, 0, st>>>(a);
+        else ssd_f32_kernel<NN, true, false, 1, EX><<<nwg, 256, 0, st>>>(a);
     }
     return ssm::check_launch("ssd_f32_chunk_scan");
 }
@@ -833,10 +834,10 @@ ssm_status ssd_f32(const float* x, long ldx, const float* dt, long lddt, const f
         workspace_bytes >= cbo + f32_cb_bytes(B, G, a.nchunks))
         a.cbw = (const float*)((char*)workspace + cbo);
     switch (N) {
-        case 128: return launch<128>(a, st);
-        case 64: return launch<64>(a, st);
-        case 32: return launch<32>(a, st);
-        default: return launch<16>(a, st);
+        case 128: return a.hs > 1 ? launch<128, true>(a, st) : launch<128, false>(a, st);
+        case 64: return a.hs > 1 ? launch<64, true>(a, st) : launch<64, false>(a, st);
+        case 32: return launch<32, true>(a, st);
+        default: return launch<16, true>(a, st);
     }
 }
 

@@ -31,6 +31,8 @@ def close(got, ref, what):
     (1, 700, 4, 2, 16, 128),     # two groups, 128-wide heads, segments
     (1, 2000, 12, 1, 16, 128),   # the large preset
     (1, 4097, 1, 1, 32, 192),    # three 64-row parts of one head, many segments, ragged
+    (1, 300, 4, 2, 64, 128),     # 64 and 128 states: heads of several 64-row parts
+    (2, 130, 3, 1, 128, 128),
 ])
 @pytest.mark.parametrize("state,clamp", [(True, False), (False, True)])
 def test_matches_oracle(B, L, H, G, N, P, state, clamp):
@@ -90,7 +92,8 @@ def test_mixer_matches_oracle(H, N):
     dev.destroy()
 
 
-@pytest.mark.parametrize("B,L,H,N,P", [(1, 64, 8, 16, 64), (2, 333, 12, 16, 128), (1, 90, 4, 32, 64)])
+@pytest.mark.parametrize("B,L,H,N,P", [(1, 64, 8, 16, 64), (2, 333, 12, 16, 128), (1, 90, 4, 32, 64),
+                                       (1, 64, 4, 64, 128), (1, 100, 3, 128, 192)])
 def test_fast_decay_keeps_precision(B, L, H, N, P):
     """Heads whose decay reaches tens of log2 units within a chunk: y and the final state against
     float64 in the 2-norm. A step's decay and weight are a rounded exponent difference d (d 2^-24
