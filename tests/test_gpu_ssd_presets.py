@@ -135,3 +135,27 @@ def test_state_in_place(B, L, H, N, P):
     y2 = kernels.ssd_chunk_scan(*t[:6], h0=state, hT=state)
     torch.cuda.synchronize()
     assert torch.equal(y, y2) and torch.equal(hT, state)
+
+
+@pytest.mark.parametrize("P,N", [(64, 16), (128, 32), (128, 64)])
+@pytest.mark.parametrize("what", [np.inf, -np.inf, np.nan])
+def test_non_finite_x_stays_causal(P, N, what):
+    """x inf or NaN at one step of one channel, at every place of a 16-step tile: the steps before
+    it and the other channels keep the bits that they have without it, and from it on the channel
+    is not finite."""
+    print(f"[case] ssd non-finite x P={P} N={N} {what}", flush=True)
+    from ssmjs_amd import kernels
+    B, L, H = 1, 70, 2
+    t = [torch.from_numpy(a).cuda() for a in inputs(N, B, L, H, P, 1, N)]
+    clean = kernels.ssd_chunk_scan(*t[:6])
+    x = t[0]
+    for step in list(range(16)) + [31, 32, 47, 69]:
+        h, p = step % H, (7 * step) % P
+        keep = x[0, step, h, p].item()
+        x[0, step, h, p] = what
+        y = kernels.ssd_chunk_scan(x, *t[1:6])
+        torch.cuda.synchronize()
+        x[0, step, h, p] = keep
+        assert not torch.isfinite(y[0, step:, h, p]).any()
+        y[0, step:, h, p] = clean[0, step:, h, p]
+        assert torch.equal(y, clean), f"step {step}"
