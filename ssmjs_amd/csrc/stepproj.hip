@@ -32,11 +32,10 @@
 // once per load (launch_pack_step, gemm_h3.hip: a scale per row); X arrives in fp32 and each wave
 // scales and splits its own k range of it in registers, while its W is still on the way from HBM.
 // Range: as there, every output is held against what the split may have lost of elements far
-// below their row's largest (W: the packing's rho; X: 2^-25 for each element of a lane that holds
-// one below 2^-16 of its wave's largest). Its measure is the waves' partial sums taken by
-// magnitude, which are small together only if the operands really are that far apart. Such an
-// output, and one that is not finite (elements that are inf or NaN become NaN), is formed again
-// from the fp32 operands.
+// below their row's largest (W: the packing's rho; X: 2^-25 of each scaled element). Its measure is
+// the waves' partial sums taken by magnitude, which are small together only if the operands really
+// are that far apart. Such an output, and one that is not finite (elements that are inf or NaN
+// become NaN), is formed again from the fp32 operands.
 //
 // Operand order. X is in fragment order (frag_off in glue.hpp): the 1 KB of a (16-row tile,
 // 16-wide k-block) is contiguous, lane-major, lane 16 q + i holding row i, k = 4 q .. + 3, so one
@@ -138,7 +137,7 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     constexpr int RS = (ROWS + 31) / 32, EPT = RS * NC;
     __shared__ float red[MULTI ? 2 : 1][kNW][ROWS][16 * NC + 1];
     __shared__ float sc[64];
-    __shared__ float2 loss[kNW][ROWS];   // (what the split of X may lose, scale) per wave and row
+    __shared__ float scale[kNW][ROWS];   // the groups' scales per wave and row, summed
     __shared__ float us[EPI == EPI_CONVX ? ROWS : 1][16 * NC + 1];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -201,16 +200,15 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     // accumulator's rows 4 q + r of tile i
     u32x4 xh[MT][KW], xl[MT][KW];   // eight fp16 values each
     int ex[NG][MT][4];
-    float2 lost[MT];                // of row l16 of tile i: the passes' losses and scales, summed
+    float scl[MT];                  // of row l16 of tile i: the groups' scales, summed
 #pragma unroll
-    for (int i = 0; i < MT; ++i) lost[i] = make_float2(0.f, 0.f);
+    for (int i = 0; i < MT; ++i) scl[i] = 0.f;
     auto split = [&](const float4 (&x)[MT][KW][2]) __attribute__((always_inline)) {
         // (no branch, and step by step over all groups: their exchanges overlap)
-        unsigned mx[NG * MT], mn[NG * MT];
+        unsigned mx[NG * MT];
 #pragma unroll
         for (int gi = 0; gi < NG * MT; ++gi) {
             mx[gi] = 0;
-            mn[gi] = 0x7fffffffu;
 #pragma unroll
             for (int u = KG * (gi / MT); u < KG * (gi / MT + 1); ++u)
 #pragma unroll
@@ -219,7 +217,6 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
                     const unsigned b0 = __float_as_uint(v.x) & 0x7fffffffu, b1 = __float_as_uint(v.y) & 0x7fffffffu,
                                    b2 = __float_as_uint(v.z) & 0x7fffffffu, b3 = __float_as_uint(v.w) & 0x7fffffffu;
                     mx[gi] = max(max(mx[gi], b0), max(b1, max(b2, b3)));
-                    mn[gi] = min(min(mn[gi], b0), min(b1, min(b2, b3)));
                 }
         }
 #pragma unroll
@@ -233,12 +230,7 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
             const int E = min((int)(mx[gi] >> 23), 254), sh = mx[gi] ? 141 - E : 0;
 #pragma unroll
             for (int r = 0; r < 4; ++r) ex[g][i][r] = -__shfl(sh, 4 * q + r);
-            // lanes whose smallest element (a zero counts) is below 2^-2 scaled: up to 2^-25 lost
-            // of each of the lane's elements
-            const unsigned long long small = __ballot((int)(mn[gi] >> 23) < max(E - 16, 1));
-            const int lanes = __popcll((small >> l16) & 0x0001000100010001ull);
-            lost[i].x += mx[gi] ? __builtin_ldexpf((float)(lanes * 8 * KG), -25 - sh) : 0.f;
-            lost[i].y += mx[gi] ? __builtin_ldexpf(1.f, -sh) : 0.f;
+            scl[i] += mx[gi] ? __builtin_ldexpf(1.f, -sh) : 0.f;
             // (an inf gives hi = inf, lo = NaN, and so NaN in every product of its row)
 #pragma unroll
             for (int u = KG * g; u < KG * (g + 1); ++u)
@@ -336,8 +328,9 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     const auto rg2 = rsrc(a.g2, EPI == EPI_RESID && a.g2 ? (unsigned)a.N * 4u : 0u);
     const auto ryy = rsrc(a.Y, EPI == EPI_RESID ? (unsigned)((long)(a.M - 1) * a.ldy + a.N) * 4u : 0u);
 
-    // the rows' losses over all waves, summed when the first tile's waves have met
-    float2 rl[RS];
+    // 2^37 of the rows' scales over all waves, summed when the first tile's waves have met
+    static_assert(32 * KG == 128, "the factor 2^-18 of the coverage test");
+    float need[RS];
     bool first = true;
     // One column tile: W of its first pass is in wc; the next tile's goes into wnx.
     constexpr int kConvPre = 4;
@@ -436,19 +429,17 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
         if (!MULTI || first) {
 #pragma unroll
             for (int i = 0; i < MT; ++i)
-                if (q == 0) loss[w][16 * ((i + irot) & (MT - 1)) + l16] = lost[i];
+                if (q == 0) scale[w][16 * ((i + irot) & (MT - 1)) + l16] = scl[i];
         }
         __syncthreads();
         if (!MULTI || first) {
 #pragma unroll
             for (int s = 0; s < RS; ++s) {
                 const int ei = min((tid >> 4) + 32 * s, ROWS - 1);
-                rl[s] = loss[0][ei];
+                float t = scale[0][ei];
 #pragma unroll
-                for (int k = 1; k < kNW; ++k) {
-                    rl[s].x += loss[k][ei].x;
-                    rl[s].y += loss[k][ei].y;
-                }
+                for (int k = 1; k < kNW; ++k) t += scale[k][ei];
+                need[s] = t * 0x1p37f;
             }
             first = false;
         }
@@ -467,14 +458,13 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
                 v += t;
                 mag += fabsf(t);
             }
-            v = __builtin_ldexpf(v, (int)(short)wex[j]);
             const bool ok = em < a.M && col_ok[j];
-            // the split's loss, at most 2^15 (loss of X + scale * rho of W), against 2^-22 of the
-            // magnitudes (the factor 2^37 in two parts, within fp32's range)
-            const float2 lo = rl[e % RS];
-            const bool covered = mag * 0x1p-20f >= fmaf(lo.y, __uint_as_float(wex[j] & 0xffff0000u), lo.x) * 0x1p17f;
+            // The split loses at most 2^15 scale (2^-25 (32 KG) + rho) of an output, which has to
+            // be within 2^-22 of its partial sums' magnitudes.
+            const bool covered = mag >= need[e % RS] * (0x1p-18f + __uint_as_float(wex[j] & 0xffff0000u));
+            v = __builtin_ldexpf(v, (int)(short)wex[j]);
             const bool again = ok && !(covered && __builtin_isfinite(v));
-            if (__any(again)) {
+            if (__builtin_expect(__any(again), 0)) {
                 const float t = step_exact(a.X, a.Wf, em, n, a.K, again);
                 v = again ? t : v;
             }
