@@ -74,6 +74,11 @@ __device__ __forceinline__ float softplus_corr(float x) {
     return x < -8.f ? e - 0.5f * e * e : fmaf(e - (w - 1.f), __builtin_amdgcn_rcpf(w), __logf(w));
 }
 
+// Greedy order: v wins over (best, bi) when larger, or equal with a lower index.
+__device__ __forceinline__ void pick(float v, int i, float& best, int& bi) {
+    if (v > best || (v == best && i < bi)) { best = v; bi = i; }
+}
+
 // z * sigmoid(z) with v_exp_f32 and v_rcp_f32 (about 1 ulp each).
 __device__ __forceinline__ float silu_fast(float z) {
     return z * __builtin_amdgcn_rcpf(1.f + __expf(-z));

@@ -22,11 +22,6 @@
 namespace ssm {
 namespace {
 
-// greedy order: v wins over (best, bi) when larger, or equal with a lower index
-__device__ __forceinline__ void pick(float v, int i, float& best, int& bi) {
-    if (v > best || (v == best && i < bi)) { best = v; bi = i; }
-}
-
 // One workgroup per row: the row's pairs merged by a wave-shuffle and LDS tree.
 constexpr int kFin = 256;
 __global__ __launch_bounds__(kFin) void head_argmax_kernel(const float* __restrict__ part,

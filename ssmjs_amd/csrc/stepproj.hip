@@ -80,11 +80,6 @@ __device__ __forceinline__ float sum16(float v) {
     return v;
 }
 
-// greedy order: v wins over (best, bi) when larger, or equal with a lower index
-__device__ __forceinline__ void pick(float v, int i, float& best, int& bi) {
-    if (v > best || (v == best && i < bi)) { best = v; bi = i; }
-}
-
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ halfx8 as_h8(u32x4 v) { return __builtin_bit_cast(halfx8, v); }
 

@@ -32,7 +32,9 @@ def _p(t):
 
 def _stream():
     """Handle of the current device's current stream, without a Stream object around it (1 us of
-    each call)."""
+    each call) where torch has the calls for that."""
+    if _device is None or _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
     return _raw_stream(_device())
 
 

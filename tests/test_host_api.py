@@ -207,3 +207,15 @@ def test_byte_tokenizer_roundtrip():
     t = ByteTokenizer(300)
     assert t.decode(t.encode("héllo")) == "héllo" and t.vocabSize == 300
     assert math.isfinite(len(t.encode("")))
+
+
+def test_stream_handle_without_torchs_private_calls(monkeypatch):
+    # kernels._stream takes the public call where torch has no raw one
+    from types import SimpleNamespace
+
+    import torch
+
+    from ssmjs_amd import kernels
+    monkeypatch.setattr(kernels, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=7))
+    assert kernels._stream() == 7
