@@ -151,14 +151,18 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     // ---- operand loads: a wave's k-blocks go in groups of four, each scaled and summed by itself,
     // and the groups' sums are added in order: the same in every workgroup (equal rows of W give
     // equal results) and whether a pass takes two groups or, with more row tiles in the registers,
-    // one (a row's result does not depend on the rows beside it). Past four k-blocks a wave, two
-    // groups are adjacent. Every workgroup reads the same X; those on one XCD start at row tiles of
-    // their own.
+    // one (a row's result does not depend on the rows beside it). Up to 256 input features a wave
+    // takes one k-block (a.run: the coverage test below wants several partial sums; 128 features
+    // in one wave had a few outputs of every launch formed again), past 1024 two groups are
+    // adjacent. Every workgroup reads the same X; those on one XCD start at row
+    // tiles of their own.
     constexpr int KG = 4, NG = KW / KG;
     static_assert(KW == KG || KW == 2 * KG, "one or two groups");
     const bool halves = KW == KG && a.npass > 1;   // (uniform) a pass takes one of two adjacent groups
     auto block = [&](int p, int u) __attribute__((always_inline)) {
-        return halves ? 2 * KG * (kNW * (p >> 1) + w) + KG * (p & 1) + u : KW * (kNW * p + w) + u;
+        if (KW > KG) return KW * (kNW * p + w) + u;
+        if (halves) return 2 * KG * (kNW * (p >> 1) + w) + KG * (p & 1) + u;
+        return a.run * w + u * a.ustep;   // (a step of KB2: past the operand from u = 1 on)
     };
     const int irot = (r8 / a.rg) & (MT - 1);
     const auto ra = rsrc(a.X, (unsigned)(a.mt * KB) * 1024u);
@@ -762,6 +766,8 @@ ssm_status launch_stepproj(int epi, StepProj a, hipStream_t st) {
     a.we = (const int*)(a.W + step_ex_off(a.N, a.K));
     const StepPlan p = step_plan(a.M, a.N, a.K);
     a.rg = p.rg; a.npass = p.npass;
+    a.run = a.K <= 32 * kNW ? 1 : 4;
+    a.ustep = a.run == 1 ? (int)cdiv(a.K, 32) : 1;
     SSM_REQUIRE(epi != EPI_HEAD || a.nparts == step_head_parts(a.M, a.N, a.K),
                 "stepproj: head pairs");
     if (p.multi) {
