@@ -569,34 +569,44 @@ __global__ __launch_bounds__(256 * HPW, 2) void ssd_f32_kernel(F32Args a) {
 #pragma unroll
                 for (int ib = 0; ib < QB; ++ib) Y[ib] *= ssm::ex2(sm.ac[buf][hw][16 * ib + l16]);
             }
-            // With EX, as in the kernels that took these shapes before, a step that is inf or NaN
-            // must not meet the zeros of M above the diagonal (the steps before it): a chunk with
-            // one multiplies its diagonal tiles without it and adds it to the steps from its own
-            // on. (64-row heads of 64 and 128 states have always let it reach back up to 15
-            // steps; the test costs them 4%: 658 -> 684 us for 8 x 4096 steps of 64 heads.)
-            bool broken = false;
-            if constexpr (EX) {
+            if constexpr (!EX) {
+#pragma unroll
+                for (int ib = 0; ib < QB; ++ib)
+#pragma unroll
+                    for (int jb = 0; jb <= ib; ++jb) {
+                        const float4 mv = *reinterpret_cast<const float4*>(&sm.m[hw][16 * ib + l16][16 * jb + 4 * q4]);
+                        Y[ib] = mfma4(xv[jb][0], mv.x, Y[ib]);
+                        Y[ib] = mfma4(xv[jb][1], mv.y, Y[ib]);
+                        Y[ib] = mfma4(xv[jb][2], mv.z, Y[ib]);
+                        Y[ib] = mfma4(xv[jb][3], mv.w, Y[ib]);
+                    }
+            } else {
+                // As in the kernels that took these shapes before, a step that is inf or NaN must
+                // not meet the zeros of M above the diagonal (the steps before it): a chunk with
+                // one multiplies its diagonal tiles without it and adds it to the steps from its
+                // own on. (64-row heads of 64 and 128 states have always let it reach back up to
+                // 15 steps; the test costs them 4%: 658 -> 684 us for 8 x 4096 steps of 64 heads.)
+                auto y_tile = [&](int ib, int jb, const float (&x)[4]) __attribute__((always_inline)) {
+                    const float4 mv = *reinterpret_cast<const float4*>(&sm.m[hw][16 * ib + l16][16 * jb + 4 * q4]);
+                    Y[ib] = mfma4(x[0], mv.x, Y[ib]);
+                    Y[ib] = mfma4(x[1], mv.y, Y[ib]);
+                    Y[ib] = mfma4(x[2], mv.z, Y[ib]);
+                    Y[ib] = mfma4(x[3], mv.w, Y[ib]);
+                };
                 float xs = 0.f;
 #pragma unroll
                 for (int jb = 0; jb < QB; ++jb)
 #pragma unroll
                     for (int s = 0; s < 4; ++s) xs = fmaf(0.f, xv[jb][s], xs);
-                broken = __any(xs != 0.f);   // (0 x inf and 0 x NaN are NaN)
-            }
-            auto y_tile = [&](int ib, int jb, const float (&x)[4]) __attribute__((always_inline)) {
-                const float4 mv = *reinterpret_cast<const float4*>(&sm.m[hw][16 * ib + l16][16 * jb + 4 * q4]);
-                Y[ib] = mfma4(x[0], mv.x, Y[ib]);
-                Y[ib] = mfma4(x[1], mv.y, Y[ib]);
-                Y[ib] = mfma4(x[2], mv.z, Y[ib]);
-                Y[ib] = mfma4(x[3], mv.w, Y[ib]);
-            };
+                const bool broken = __any(xs != 0.f);   // (0 x inf and 0 x NaN are NaN)
 #pragma unroll
-            for (int ib = 0; ib < QB; ++ib) {
+                for (int ib = 0; ib < QB; ++ib) {
 #pragma unroll
-                for (int jb = 0; jb < ib; ++jb) y_tile(ib, jb, xv[jb]);
-                if (!broken) {
-                    y_tile(ib, ib, xv[ib]);
-                } else {
+                    for (int jb = 0; jb < ib; ++jb) y_tile(ib, jb, xv[jb]);
+                    if (!broken) {
+                        y_tile(ib, ib, xv[ib]);
+                        continue;
+                    }
                     float xf[4];
 #pragma unroll
                     for (int s = 0; s < 4; ++s) xf[s] = __builtin_isfinite(xv[ib][s]) ? xv[ib][s] : 0.f;
