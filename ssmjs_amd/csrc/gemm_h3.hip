@@ -85,7 +85,7 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     const unsigned row_oor = i16 < rows ? 0u : 0x80000000u;
     const unsigned base = (unsigned)((long)i16 * a.ldx * 4);
     floatx4 v[KW][2];
-    unsigned mx = 0;
+    unsigned mx = 0, mn = 0x7fffffffu;
     // k blocks w, w + 8, ...; per pass KW of them (one pass unless K > 256 KW)
     auto fetch = [&](int kb0) {
 #pragma unroll
@@ -111,7 +111,9 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float x = v[u][h][e];   // (a bit_cast of the element itself reads [0])
-                    mx = max(mx, __builtin_bit_cast(unsigned, x) & 0x7fffffffu);
+                    const unsigned m = __builtin_bit_cast(unsigned, x) & 0x7fffffffu;
+                    mx = max(mx, m);
+                    mn = min(mn, m);
                 }
     };
     const bool once = a.KB <= 8 * KW;
@@ -129,7 +131,10 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     const int E = min((int)(mx >> 23), 254);
     const int sh = mx ? 141 - E : 0;
     if (!STEP && w == 0 && q == 0) a.ex[16 * rb + i16] = -sh;
-    float rho = 0.f;
+    // what is left out past 2^-23 of an element is 2^-25 at most, so only elements below 2^-2 scaled
+    // can add to rho: none in most waves of normal data (8192 x 768: 12.5 -> 11.7 us)
+    float rho = 0.f, rho2 = 0.f;
+    const bool small = __any((int)(mn >> 23) < max(E - 16, 1));
     const bool low = __any(sh < 0);   // elements of such a row may scale to zero
     for (int kb0 = w; kb0 < a.KB; kb0 += 8 * KW) {
         if (!once) fetch(kb0);
@@ -144,19 +149,31 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
                 const float s = __builtin_ldexpf(x, sh);
                 const bool fin = (__builtin_bit_cast(unsigned, x) & 0x7f800000u) != 0x7f800000u;
                 const _Float16 hh = (_Float16)s;
-                const float d = s - (float)hh;
-                const _Float16 ll = (_Float16)d;
                 hi[e] = fin ? hh : (_Float16)__builtin_nanf("");
-                lo[e] = fin ? ll : (_Float16)0.f;
+                lo[e] = fin ? (_Float16)(s - (float)hh) : (_Float16)0.f;
+            }
+            if (small) {
                 // (a row with inf or NaN: its outputs are formed from the fp32 operands anyway)
-                rho += fmaxf(fmaf(-0x1p-23f, fabsf(s), fabsf(d - (float)ll)), 0.f);
-                if (low && s == 0.f && x != 0.f) rho += 0x1p-126f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float s = __builtin_ldexpf(v[u][e >> 2][e & 3], sh);
+                    const float left = fabsf((s - (float)hi[e]) - (float)lo[e]);
+                    (e & 1 ? rho2 : rho) += fmaxf(fmaf(-0x1p-23f, fabsf(s), left), 0.f);
+                }
+                if (low) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float x = v[u][e >> 2][e & 3];
+                        if (x != 0.f && __builtin_ldexpf(x, sh) == 0.f) rho += 0x1p-126f;
+                    }
+                }
             }
             halfx8* o = reinterpret_cast<halfx8*>(a.P + ((long)rb * a.KB + kb) * kPairB) + lane;
             o[0] = hi;
             o[64] = lo;
         }
     }
+    rho += rho2;
     rho += __shfl_xor(rho, 16);
     rho += __shfl_xor(rho, 32);
     if (q == 0) rred[w][i16] = rho;
@@ -211,7 +228,7 @@ __device__ __forceinline__ void h3_step() {
 
 // The 16 x 16 outputs of a wave from the fp32 operands, k in [k0, k1), on the fp32 matrix cores:
 // x and w are the lane's rows (row / column lane & 15), k quads 4 (lane >> 4) of each 16.
-__device__ __noinline__ floatx4 h3_exact(const float* x, const float* w, int k0, int k1) {
+__device__ __forceinline__ floatx4 h3_exact(const float* x, const float* w, int k0, int k1) {
     const int q4 = 4 * ((threadIdx.x & 63) >> 4);
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
     constexpr int U = 4;
@@ -235,6 +252,13 @@ __device__ __noinline__ floatx4 h3_exact(const float* x, const float* w, int k0,
     return acc;
 }
 
+// Whether a running sum is large enough for its split: it bounds S = sum |x w| of the scaled
+// operands from below, and 2^15 (rho_x + rho_w) bounds what the split's range leaves out, which is
+// then at most 2^-22 S.
+__device__ __forceinline__ bool h3_large(float s, float rx, float rw) {
+    return fabsf(s) >= 0x1p37f * (rx + rw);
+}
+
 // WM x WN waves, each with TI x TJ 16 x 16 tiles: a workgroup owns (16 TI WM) x (16 TJ WN) of
 // Y and walks its k blocks through NS LDS stages (each its own LDS object, so that reading one
 // does not wait for loads into the others), NS - 1 blocks' fragments in flight while one
@@ -251,6 +275,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
     __shared__ __attribute__((aligned(16))) char s2[NS > 2 ? NF * kFragB : 16];
     __shared__ __attribute__((aligned(16))) char s3[NS > 2 ? NF * kFragB : 16];
     __shared__ float rs[RS ? BM : 1];
+    __shared__ int2 words[BM + BN];
 
     // ---- tile of this workgroup (the order of gemm.hip: consecutive ids per XCD, groups of
     // gm_rows row tiles)
@@ -297,6 +322,21 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
         }
     };
 
+    // the rows' and columns' exponents and losses, for the test halfway and the epilogue: a word a
+    // thread, loaded ahead of the stages (a wait for it does not wait for them)
+    static_assert(BM + BN <= 64 * NW, "a word a thread");
+    int2 word = make_int2(0, __builtin_bit_cast(int, kRhoZero));
+    {
+        const int t = threadIdx.x, k = t < BM ? t : t - BM;
+        if (k < (t < BM ? rows : cols)) {
+            word.x = t < BM ? a.xe[m0 + k] : a.we[n0 + k];
+            word.y = __builtin_bit_cast(int, t < BM ? a.xr[m0 + k] : a.wr[n0 + k]);
+        }
+    }
+    auto rho_of = [](int2 v) { return __builtin_bit_cast(float, v.y); };
+    auto row_word = [&](int i, int r) { return words[16 * (TI * wm + i) + 4 * q + r]; };
+    auto col_word = [&](int j) { return words[BM + 16 * (TJ * wn + j) + i16]; };
+
     floatx4 acc[TI][TJ];
 #pragma unroll
     for (int i = 0; i < TI; ++i)
@@ -340,34 +380,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
         }
     };
 
-    // Whether a running sum is large enough for its split: it bounds S = sum |x w| of the scaled
-    // operands from below, and 2^15 (rho_x + rho_w) bounds what the split's range leaves out, which
-    // is then at most 2^-22 S. Tested halfway (okm: tiles whose sums all are), and at the end for
-    // the others: a row's rho is mostly 0 or a few 2^-26 and its sums 2^27 and more, so an output
-    // fails both only where large elements meet small ones.
-    auto rho_x = [&](int i, float (&v)[4]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 16 * (TI * wm + i) + 4 * q + r;
-            const float rho = a.xr[m0 + min(row, rows - 1)];
-            v[r] = row < rows ? rho : kRhoZero;
-        }
-    };
-    auto rho_w = [&](float (&v)[TJ]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const int c = 16 * (TJ * wn + j) + i16;
-            const float rho = a.wr[n0 + min(c, cols - 1)];
-            v[j] = c < cols ? rho : kRhoZero;
-        }
-    };
-    auto large = [&](float s, float rx, float rw) __attribute__((always_inline)) {
-        return fabsf(s) >= 0x1p37f * (rx + rw);
-    };
+    // The sums are held against the rows' losses halfway (okm: tiles whose sums all are large), and
+    // at the end for the others: a row's rho is mostly 0 or a few 2^-26 and its sums 2^27 and more,
+    // so an output fails both only where large elements meet small ones.
     static_assert(TI * TJ <= 32, "a bit per tile");
     unsigned okm = 0;
-    const int kbm = kb0 + (kb1 - kb0) / (2 * NS) * NS;   // whole turns of the loop below
-    int kb = kb0, end = kbm;
+    // (A slice is only part of a sum: its outputs are held against the losses by the finish.)
+    const int kbm = SPLIT ? kb1 : kb0 + (kb1 - kb0) / (2 * NS) * NS;   // whole turns of the loop below
+    int kb = kb0, end = kbm > kb0 ? kbm : kb1;
     if constexpr (NS == 2) {
         load(s0, kb0);
     } else {
@@ -375,6 +395,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
         load(s1, kb0 + 1);
         load(s2, kb0 + 2);
     }
+    if ((int)threadIdx.x < BM + BN) words[threadIdx.x] = word;
+    // lgkmcnt(0): written before the first turn's barrier, past which the words are read
+    __builtin_amdgcn_s_waitcnt(0xc07f);
     for (;;) {
         if constexpr (NS == 2) {
             for (; kb < end; kb += 2) {
@@ -401,21 +424,25 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
                 compute(s3);
             }
         }
+        asm volatile("" ::: "memory");   // no read of `words` moves above the turns' barriers
         if (end == kb1) break;
         end = kb1;
         float wr[TJ];
-        rho_w(wr);
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) wr[j] = rho_of(col_word(j));
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
             float xr[4];
-            rho_x(i, xr);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) xr[r] = rho_of(row_word(i, r));
 #pragma unroll
             for (int j = 0; j < TJ; ++j) {
                 bool ok = true;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ok = ok && large(acc[i][j][r], xr[r], wr[j]);
+                for (int r = 0; r < 4; ++r) ok = ok && h3_large(acc[i][j][r], xr[r], wr[j]);
                 okm |= ok ? 1u << (i * TJ + j) : 0u;
             }
+            __builtin_amdgcn_sched_barrier(0);   // (few registers beside the sums)
         }
     }
     // the loads past the last block end before the LDS they write is given back
@@ -439,78 +466,82 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_h3_kernel(H3Args a) {
     const long ldo = SPLIT ? a.N : a.ldy;
     float* yo = SPLIT ? a.part + ((long)kz * a.M + m0) * a.N + n0 : a.Y + (long)m0 * a.ldy + n0;
     const auto ry = ssm::rsrc(yo, (unsigned)(((long)(rows - 1) * ldo + cols) * 4));
-    int we[TJ];
+    int2 ww[TJ];
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-        const int c = 16 * (TJ * wn + j) + i16;
-        we[j] = c < cols ? a.we[n0 + c] : 0;
-    }
+    for (int j = 0; j < TJ; ++j) ww[j] = col_word(j);
+    // one output: row scale, beta, gate, store
+    auto put = [&](float v, int row, int c) __attribute__((always_inline)) {
+        const unsigned o = ((unsigned)(row * ldo + c) * 4u) | (c < cols ? 0u : 0x80000000u);
+        if constexpr (!SPLIT) {
+            if constexpr (RS) v *= rs[row];
+            if constexpr (BETA) v += a.beta * ssm::bload4(ry, o);
+            if (n0 + (c & ~15) >= a.gate_c0) v = ssm::silu_fast(v);
+        }
+        ssm::bstore4(v, ry, o);
+    };
+    unsigned redo = 0;   // (uniform) tiles with outputs that are not finite or not covered
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
-        int xe[4];
+        int2 xw[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = 16 * (TI * wm + i) + 4 * q + r;
-            xe[r] = row < rows ? a.xe[m0 + row] : 0;
-        }
+        for (int r = 0; r < 4; ++r) xw[r] = row_word(i, r);
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
             const int c = 16 * (TJ * wn + j) + i16;
-            const unsigned oor = c < cols ? 0u : 0x80000000u;
-            const bool gate = !SPLIT && n0 + 16 * (TJ * wn + j) >= a.gate_c0;
             float vv[4];
-            bool open = !(okm >> (i * TJ + j) & 1);
+            bool fin = true, open = !SPLIT && !(okm >> (i * TJ + j) & 1);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                vv[r] = __builtin_ldexpf(acc[i][j][r], xe[r] + we[j]);
-                open = open || !__builtin_isfinite(vv[r]);
+                vv[r] = __builtin_ldexpf(acc[i][j][r], xw[r].x + ww[j].x);
+                fin = fin && __builtin_isfinite(vv[r]);
             }
-            if (__any(open)) {
-                float xr[4], wr[TJ];
-                rho_x(i, xr);
-                rho_w(wr);
-                bool again[4];
+            if (__any(open || !fin)) {
+                bool large = true;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    again[r] = !__builtin_isfinite(vv[r]) || !large(acc[i][j][r], xr[r], wr[j]);
-                if (__any(again[0] || again[1] || again[2] || again[3])) {
-                    const int row = min(16 * (TI * wm + i) + i16, rows - 1);
-                    const floatx4 ev = h3_exact(a.X + (long)(m0 + row) * a.ldx,
-                                                a.W + (long)(n0 + min(c, cols - 1)) * a.ldw,
-                                                kb0 * kKB, min(kb1 * kKB, a.K));
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) vv[r] = again[r] && open ? ev[r] : vv[r];
-                }
+                    large = large && h3_large(acc[i][j][r], rho_of(xw[r]), rho_of(ww[j]));
+                if (__any(!fin || (open && !large))) redo |= 1u << (i * TJ + j);
             }
+            if (!(redo >> (i * TJ + j) & 1)) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 16 * (TI * wm + i) + 4 * q + r;
-                const unsigned o = ((unsigned)(row * ldo + c) * 4u) | oor;
-                float v = vv[r];
-                if constexpr (!SPLIT) {
-                    if constexpr (RS) v *= rs[row];
-                    if constexpr (BETA) v += a.beta * ssm::bload4(ry, o);
-                    if (gate) v = ssm::silu_fast(v);
-                }
-                ssm::bstore4(v, ry, o);
+                for (int r = 0; r < 4; ++r) put(vv[r], 16 * (TI * wm + i) + 4 * q + r, c);
             }
         }
+    }
+    // the tiles left out, from the fp32 operands (here no accumulator is live)
+    for (; redo; redo &= redo - 1) {
+        const int t = __builtin_ctz(redo), i = t / TJ, j = t % TJ;
+        const int xrow = min(16 * (TI * wm + i) + i16, rows - 1), c = 16 * (TJ * wn + j) + i16;
+        const floatx4 v = h3_exact(a.X + (long)(m0 + xrow) * a.ldx,
+                                   a.W + (long)(n0 + min(c, cols - 1)) * a.ldw, kb0 * kKB,
+                                   min(kb1 * kKB, a.K));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) put(v[r], 16 * (TI * wm + i) + 4 * q + r, c);
     }
 }
 
 // Split-K finish: Y = epilogue(sum over slices z = 0 .. ks-1 of part[z]), added in slice
 // order; the epilogue in the unsplit kernel's order (row scale, beta, gate). Thread
-// (row m = blockIdx.y, columns 4 c4 .. 4 c4 + 3); N % 4 == 0.
+// (row m = blockIdx.y, columns 4 c4 .. 4 c4 + 3); N % 4 == 0. The slices' magnitudes bound S from
+// below, against the losses of the row and the columns; an output that they do not cover is formed
+// again from the fp32 operands by its wave, 4 k a lane.
 __global__ __launch_bounds__(256) void gemm_h3_finish_kernel(H3Args a) {
     const int m = blockIdx.y;
     const int c4 = blockIdx.x * 256 + threadIdx.x;
-    if (4 * c4 >= a.N) return;
+    const bool in = 4 * c4 < a.N;
     const long MN = (long)a.M * a.N;
-    const float4* p = reinterpret_cast<const float4*>(a.part + (long)m * a.N) + c4;
+    const int cc = in ? c4 : 0;   // (whole waves: an idle lane repeats the first columns)
+    const float4* p = reinterpret_cast<const float4*>(a.part + (long)m * a.N) + cc;
+    const int xe = a.xe[m];
+    const float xr = a.xr[m];
+    const int4 we = reinterpret_cast<const int4*>(a.we)[cc];
+    const float4 wr = reinterpret_cast<const float4*>(a.wr)[cc];
     float4 v = p[0];
+    float4 g = make_float4(fabsf(v.x), fabsf(v.y), fabsf(v.z), fabsf(v.w));
     for (int z = 1; z < a.ks; ++z) {
         const float4 u = p[z * (MN / 4)];
         v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
+        g.x += fabsf(u.x); g.y += fabsf(u.y); g.z += fabsf(u.z); g.w += fabsf(u.w);
     }
     float s = 1.f;
     if (a.ssq) {   // same order as the unsplit kernel's row scales
@@ -519,8 +550,37 @@ __global__ __launch_bounds__(256) void gemm_h3_finish_kernel(H3Args a) {
         for (int j = 0; j < a.nssq; ++j) sum += q[j];
         s = rsqrtf(sum * a.inv_div + a.eps);
     }
-    float* y = a.Y + (long)m * a.ldy + 4 * c4;
     float o[4] = {v.x, v.y, v.z, v.w};
+    const float mag[4] = {g.x, g.y, g.z, g.w}, rho[4] = {wr.x, wr.y, wr.z, wr.w};
+    const int ex[4] = {we.x, we.y, we.z, we.w};
+    bool again[4];   // (NaN and inf are the slices' own)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        again[e] = in && mag[e] < __builtin_ldexpf(0x1p37f * (xr + rho[e]), xe + ex[e]);
+    if (__builtin_expect(__any(again[0] || again[1] || again[2] || again[3]), 0)) {
+        const int lane = threadIdx.x & 63;
+        const float* x = a.X + (long)m * a.ldx;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            for (unsigned long long todo = __ballot(again[e]); todo; todo &= todo - 1) {
+                const int src = __builtin_ctzll(todo);
+                const float* w = a.W + (long)(4 * __shfl(c4, src) + e) * a.ldw;
+                float t = 0.f;
+                for (int k = 4 * lane; k < a.K; k += 256) {   // (K % 4 == 0)
+                    const float4 xv = *reinterpret_cast<const float4*>(x + k);
+                    const float4 wv = *reinterpret_cast<const float4*>(w + k);
+                    t = fmaf(xv.x, wv.x, t);
+                    t = fmaf(xv.y, wv.y, t);
+                    t = fmaf(xv.z, wv.z, t);
+                    t = fmaf(xv.w, wv.w, t);
+                }
+#pragma unroll
+                for (int d = 32; d > 0; d >>= 1) t += __shfl_xor(t, d);
+                if (lane == src) o[e] = t;
+            }
+    }
+    if (!in) return;
+    float* y = a.Y + (long)m * a.ldy + 4 * c4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int n = 4 * c4 + e;
