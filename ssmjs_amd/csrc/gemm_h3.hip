@@ -5,7 +5,7 @@
 // magnitude lies in [2^14, 2^15), and each scaled element v is held as two fp16 values,
 // hi = fp16(v) and lo = fp16(v - hi), both rounded to nearest: v - hi is exact in fp32, and
 // hi + lo is v to 2^-23 |v| or 2^-25 (2^-39 of the row's largest magnitude), whichever is
-// larger (the excess over 2^-23 |v|, summed over the row, is kept as rho). The product of a row pair is summed as lo hi + hi lo + hi hi in fp32 accumulators
+// larger (2^-25 for each element that may have the latter is kept as the row's rho). The product of a row pair is summed as lo hi + hi lo + hi hi in fp32 accumulators
 // (v_mfma_f32_16x16x32_f16, whose products are exact in fp32), leaving out lo lo (2^-22 of a
 // product at most); the sum is scaled back exactly in the epilogue. Three MFMAs at 16 times the fp32
 // matrix rate replace one, and 3 K / 32 roundings of the running sum replace K / 4.
@@ -65,7 +65,7 @@ struct PackArgs {
     int R, K, KB;
     char* P;
     int* ex;     // per row: the power of two that undoes the scaling
-    float* rho;  // per row: what hi + lo leave out beyond 2^-23 of an element, summed (scaled)
+    float* rho;  // per row: a bound of what hi + lo leave out beyond 2^-23 of each element (scaled)
 };
 
 // STEP: the order of k of the one-token step's operand (stepproj.hip: lane (q, i) holds k = 4 q ..
@@ -74,7 +74,7 @@ struct PackArgs {
 template <int KW, bool STEP, bool VEC>
 __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     __shared__ unsigned red[8][16];
-    __shared__ float rred[8][16];
+    __shared__ int rred[8][16];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, i16 = lane & 15;
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     const unsigned row_oor = i16 < rows ? 0u : 0x80000000u;
     const unsigned base = (unsigned)((long)i16 * a.ldx * 4);
     floatx4 v[KW][2];
-    unsigned mx = 0, mn = 0x7fffffffu;
+    unsigned mx = 0;
     // k blocks w, w + 8, ...; per pass KW of them (one pass unless K > 256 KW)
     auto fetch = [&](int kb0) {
 #pragma unroll
@@ -113,7 +113,6 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
                     const float x = v[u][h][e];   // (a bit_cast of the element itself reads [0])
                     const unsigned m = __builtin_bit_cast(unsigned, x) & 0x7fffffffu;
                     mx = max(mx, m);
-                    mn = min(mn, m);
                 }
     };
     const bool once = a.KB <= 8 * KW;
@@ -131,11 +130,12 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
     const int E = min((int)(mx >> 23), 254);
     const int sh = mx ? 141 - E : 0;
     if (!STEP && w == 0 && q == 0) a.ex[16 * rb + i16] = -sh;
-    // what is left out past 2^-23 of an element is 2^-25 at most, so only elements below 2^-2 scaled
-    // can add to rho: none in most waves of normal data (8192 x 768: 12.5 -> 11.7 us)
-    float rho = 0.f, rho2 = 0.f;
-    const bool small = __any((int)(mn >> 23) < max(E - 16, 1));
-    const bool low = __any(sh < 0);   // elements of such a row may scale to zero
+    // What is left out past 2^-23 of an element is 2^-25 at most, and nothing from 2^-2 scaled on:
+    // the elements below that are counted, zeros aside (in the doubled bits less one, where a zero
+    // is the largest). Three instructions an element; the sum of what is really left out, a quarter
+    // of this, took nine (1000 x 2048 8.9 -> 10.4 us).
+    const unsigned lim = (unsigned)max(E - 16, 1) << 24;
+    int small = 0;
     for (int kb0 = w; kb0 < a.KB; kb0 += 8 * KW) {
         if (!once) fetch(kb0);
 #pragma unroll
@@ -149,40 +149,24 @@ __global__ __launch_bounds__(512) void pack_h3_kernel(PackArgs a) {
                 const float s = __builtin_ldexpf(x, sh);
                 const bool fin = (__builtin_bit_cast(unsigned, x) & 0x7f800000u) != 0x7f800000u;
                 const _Float16 hh = (_Float16)s;
+                small += 2u * __builtin_bit_cast(unsigned, x) - 1u < lim;
                 hi[e] = fin ? hh : (_Float16)__builtin_nanf("");
                 lo[e] = fin ? (_Float16)(s - (float)hh) : (_Float16)0.f;
-            }
-            if (small) {
-                // (a row with inf or NaN: its outputs are formed from the fp32 operands anyway)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float s = __builtin_ldexpf(v[u][e >> 2][e & 3], sh);
-                    const float left = fabsf((s - (float)hi[e]) - (float)lo[e]);
-                    (e & 1 ? rho2 : rho) += fmaxf(fmaf(-0x1p-23f, fabsf(s), left), 0.f);
-                }
-                if (low) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float x = v[u][e >> 2][e & 3];
-                        if (x != 0.f && __builtin_ldexpf(x, sh) == 0.f) rho += 0x1p-126f;
-                    }
-                }
             }
             halfx8* o = reinterpret_cast<halfx8*>(a.P + ((long)rb * a.KB + kb) * kPairB) + lane;
             o[0] = hi;
             o[64] = lo;
         }
     }
-    rho += rho2;
-    rho += __shfl_xor(rho, 16);
-    rho += __shfl_xor(rho, 32);
-    if (q == 0) rred[w][i16] = rho;
+    small += __shfl_xor(small, 16);
+    small += __shfl_xor(small, 32);
+    if (q == 0) rred[w][i16] = small;
     __syncthreads();
     if (w == 0 && q == 0) {
-        rho = rred[0][i16];
+        small = rred[0][i16];
 #pragma unroll
-        for (int k = 1; k < 8; ++k) rho += rred[k][i16];
-        rho = mx ? rho : kRhoZero;
+        for (int k = 1; k < 8; ++k) small += rred[k][i16];
+        const float rho = mx ? 0x1p-25f * (float)small : kRhoZero;
         if constexpr (STEP) {
             const unsigned up = __builtin_bit_cast(unsigned, rho) + (mx ? 0xffffu : 0u);
             a.ex[16 * rb + i16] = (int)((up & 0xffff0000u) | ((unsigned)-sh & 0xffffu));
