@@ -141,9 +141,10 @@ ssm_status ssm_m1_state_update(const float* x, long ldx, const float* dt, long l
  * lddt; Bm, Cm: (B,L,G,N) of `in_dtype`, row strides ldb/ldc; y: (B,L,H,P) float, ldy;
  * h0/hT: (B,H,P,N) float (may be NULL; hT may alias h0). P = 64 with N in {64, 128} runs the
  * fused MFMA kernel; so do float inputs with P a multiple of 64 and N in {16, 32, 64, 128} when
- * all rows are 16-byte aligned and the workspace is given. Other shapes: with G = 1, N <= 64, float inputs, a dt clamp that cannot bind and
- * the workspace, the Mamba-1 chunked scan over H*P channels; otherwise a sequential kernel
- * (no workspace needed). The chunk length of the reference config (chunkLen) does not change
+ * all rows are 16-byte aligned and the workspace is given. Other shapes: with G = 1, N <= 64,
+ * float inputs, a dt clamp that cannot bind and the workspace, the Mamba-1 chunked scan over H*P
+ * channels; otherwise a sequential kernel (no workspace needed). An x that is inf or NaN changes
+ * no earlier step (P = 64 with N in {64, 128}: up to 15 earlier steps of its channel). The chunk length of the reference config (chunkLen) does not change
  * the result; the kernel uses its own internal chunk. `workspace` holds
  * ssm_ssd_workspace(...) bytes: segment states for long sequences and, for float inputs, the
  * C B^T tiles of every chunk (a workspace with room for the segment states only gives the

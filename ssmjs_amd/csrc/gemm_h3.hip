@@ -14,8 +14,10 @@
 // where the large elements meet zeros or tiny ones, so that the small ones make up the sum.
 // Every output is held against rho (below) and, where its sum is not large enough to
 // cover the loss, formed again from the fp32 operands on the fp32 matrix cores, 16 x 16 outputs
-// at a time: the error is at most (3 K / 32) 2^-24 + 2^-22 3 + 2^-22 of S = sum |x w| for any
-// operands (or the fp32 product's K / 4 roundings of 2^-24). Normal data takes no such path.
+// at a time: the error is at most (3 K / 32) 2^-24 + 2^-20 of S = sum |x w| for any finite
+// operands (or the fp32 product's K / 4 roundings of 2^-24). Normal data takes no such path; the
+// tests of its sums cost nothing measurable at 8192 rows, and the packing's counts 1 us of 9 at
+// 1000 rows of 2048.
 //
 // Non-finite values. An inf or NaN element becomes a NaN in hi, so that every output of its
 // row (column) comes out NaN; an output that is not finite is formed again in the same way, and

@@ -79,9 +79,9 @@ struct StepProj {
     const float* wxt = nullptr; int RN = 0; float* xpart = nullptr;
     // EPI_HEAD: greedy (value, index) pairs, (M, nparts), one per row and workgroup
     float* part = nullptr; int nparts = 0;
-    // set by the launcher: row and column tiles, row groups, passes over K, the k-blocks of a
-    // wave (from run times its number on, ustep apart), W's row words (step_ex_off)
-    int mt = 0, nt = 0, rg = 0, npass = 0, run = 0, ustep = 0;
+    // set by the launcher: row and column tiles, row groups, passes over K, W's row words
+    // (step_ex_off)
+    int mt = 0, nt = 0, rg = 0, npass = 0;
     const int* we = nullptr;
 };
 constexpr int kXpartMaxRN = 128;

@@ -56,7 +56,8 @@
 // Measured (MI355X, weights cold, fp32 MFMA tiles of 16 x 16 -> this): 64 x 4384 x 1024 with the
 // conv update 14.8 -> 13.2 us, 64 x 3072 x 768 10.4 -> 9.0, the head 64 x 32000 x 1024 49 -> 32.8;
 // the narrow ones lose a little, 64 x 1024 x 2048 with the residual 7.5 -> 7.9 and 64 x 768 x 1536
-// 6.5 -> 7.0 (every workgroup splits its rows of X anew).
+// 6.5 -> 7.0 (every workgroup splits its rows of X anew). The coverage test adds 0.2 to 0.3 us to
+// each (decode of 64 sequences, 8 layers: 324 -> 332).
 #include <algorithm>
 
 #include "common.hpp"
@@ -151,10 +152,10 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     // ---- operand loads: a wave's k-blocks go in groups of four, each scaled and summed by itself,
     // and the groups' sums are added in order: the same in every workgroup (equal rows of W give
     // equal results) and whether a pass takes two groups or, with more row tiles in the registers,
-    // one (a row's result does not depend on the rows beside it). Up to 256 input features a wave
-    // takes one k-block (a.run: the coverage test below wants several partial sums; 128 features
-    // in one wave had a few outputs of every launch formed again), past 1024 two groups are
-    // adjacent. Every workgroup reads the same X; those on one XCD start at row
+    // one (a row's result does not depend on the rows beside it). Past 1024 input features two
+    // groups are adjacent. (One k-block a wave for up to 256 features, so that the coverage test
+    // below has several partial sums to go by, saved the 128-wide preset 1.4 us of 72 a step, but its
+    // run-time stride cost every other shape: in_proj of 28 rows 9.5 -> 10.0 us.) Every workgroup reads the same X; those on one XCD start at row
     // tiles of their own.
     constexpr int KG = 4, NG = KW / KG;
     static_assert(KW == KG || KW == 2 * KG, "one or two groups");
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
     auto block = [&](int p, int u) __attribute__((always_inline)) {
         if (KW > KG) return KW * (kNW * p + w) + u;
         if (halves) return 2 * KG * (kNW * (p >> 1) + w) + KG * (p & 1) + u;
-        return a.run * w + u * a.ustep;   // (a step of KB2: past the operand from u = 1 on)
+        return KW * w + u;
     };
     const int irot = (r8 / a.rg) & (MT - 1);
     const auto ra = rsrc(a.X, (unsigned)(a.mt * KB) * 1024u);
@@ -203,33 +204,26 @@ __global__ __launch_bounds__(kNT, 2) void stepproj_kernel(StepProj a) {
 #pragma unroll
     for (int i = 0; i < MT; ++i) scl[i] = 0.f;
     auto split = [&](const float4 (&x)[MT][KW][2]) __attribute__((always_inline)) {
-        // (no branch, and step by step over all groups: their exchanges overlap)
-        unsigned mx[NG * MT];
-#pragma unroll
-        for (int gi = 0; gi < NG * MT; ++gi) {
-            mx[gi] = 0;
-#pragma unroll
-            for (int u = KG * (gi / MT); u < KG * (gi / MT + 1); ++u)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float4 v = x[gi % MT][u][h];
-                    const unsigned b0 = __float_as_uint(v.x) & 0x7fffffffu, b1 = __float_as_uint(v.y) & 0x7fffffffu,
-                                   b2 = __float_as_uint(v.z) & 0x7fffffffu, b3 = __float_as_uint(v.w) & 0x7fffffffu;
-                    mx[gi] = max(max(mx[gi], b0), max(b1, max(b2, b3)));
-                }
-        }
-#pragma unroll
-        for (int o = 16; o <= 32; o *= 2)
-#pragma unroll
-            for (int gi = 0; gi < NG * MT; ++gi)
-                mx[gi] = max(mx[gi], (unsigned)__shfl_xor((int)mx[gi], o));
+        // (tile by tile: the first is split while the next one's loads arrive)
 #pragma unroll
         for (int gi = 0; gi < NG * MT; ++gi) {
             const int g = gi / MT, i = gi % MT;
-            const int E = min((int)(mx[gi] >> 23), 254), sh = mx[gi] ? 141 - E : 0;
+            unsigned mx = 0;
+#pragma unroll
+            for (int u = KG * g; u < KG * (g + 1); ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float4 v = x[i][u][h];
+                    const unsigned m1 = max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu);
+                    const unsigned m2 = max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu);
+                    mx = max(mx, max(m1, m2));
+                }
+            mx = max(mx, (unsigned)__shfl_xor((int)mx, 16));
+            mx = max(mx, (unsigned)__shfl_xor((int)mx, 32));
+            const int sh = mx ? 141 - min((int)(mx >> 23), 254) : 0;
 #pragma unroll
             for (int r = 0; r < 4; ++r) ex[g][i][r] = -__shfl(sh, 4 * q + r);
-            scl[i] += mx[gi] ? __builtin_ldexpf(1.f, -sh) : 0.f;
+            scl[i] += mx ? __builtin_ldexpf(1.f, -sh) : 0.f;
             // (an inf gives hi = inf, lo = NaN, and so NaN in every product of its row)
 #pragma unroll
             for (int u = KG * g; u < KG * (g + 1); ++u)
@@ -766,8 +760,6 @@ ssm_status launch_stepproj(int epi, StepProj a, hipStream_t st) {
     a.we = (const int*)(a.W + step_ex_off(a.N, a.K));
     const StepPlan p = step_plan(a.M, a.N, a.K);
     a.rg = p.rg; a.npass = p.npass;
-    a.run = a.K <= 32 * kNW ? 1 : 4;
-    a.ustep = a.run == 1 ? (int)cdiv(a.K, 32) : 1;
     SSM_REQUIRE(epi != EPI_HEAD || a.nparts == step_head_parts(a.M, a.N, a.K),
                 "stepproj: head pairs");
     if (p.multi) {
